@@ -441,6 +441,7 @@ hipError_t tables_setup(int device, hipStream_t st) {
   // the caller (msh_create) has made `device` current
   hipError_t e = launch_count_tables(st);
   if (e == hipSuccess) e = launch_mt_tables(st);
+  if (e == hipSuccess) e = launch_mc_image(st);
   // complete before any context's stream can launch a kernel that reads them
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e == hipSuccess) done[device] = true;
@@ -472,13 +473,19 @@ int grow(Ctx* c, void** buf, size_t* have, size_t need, const char* what) {
   return MSH_OK;
 }
 
-int setup_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w) {
+// extra: room for the sample bits of the row kernels, at *bits
+int setup_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t extra = 0,
+                    void** bits = nullptr) {
   const size_t need = workspace_layout(units, ncoords, nullptr, nullptr);
-  int rc = grow(c, &c->ws, &c->ws_bytes, need, "workspace allocation");
+  int rc = grow(c, &c->ws, &c->ws_bytes, need + extra, "workspace allocation");
   if (rc) return rc;
   workspace_layout(units, ncoords, c->ws, w);
+  if (bits) *bits = (char*)c->ws + need;
   return MSH_OK;
 }
+
+// The row kernels serve the default family and family 2.
+bool rows_family(const Plan& p) { return p.family < 0 || p.family == 2; }
 
 bool same_call(const Ctx* c, const msh_field* f, const msh_params* p) {
   return c->have && memcmp(&c->field, f, sizeof(*f)) == 0 &&
@@ -608,7 +615,19 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, MSH_ERR_DEVICE, "hipSetDevice");
   Geom g = make_geom(f, pl.method);
   Workspace w{};
-  rc = setup_workspace(c, g.units, (int64_t)g.nx + g.ny + g.nz, &w);
+  const int64_t ncoords = (int64_t)g.nx + g.ny + g.nz;
+  RowsGeom rg{};
+  Geom gr = g;
+  void* bits = nullptr;
+  if (rows_family(pl) && rows_geom(pl, &gr, &rg)) {
+    // with no room for the sample bits the other kernels, which need less,
+    // take the volume
+    if (setup_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg), &bits) == MSH_OK)
+      g = gr;
+    else
+      (void)hipGetLastError();
+  }
+  if (!bits) rc = setup_workspace(c, g.units, ncoords, &w);
   if (rc) return rc;
   int64_t nv = 0, nfc = 0;
   const void* dfield = f->data;
@@ -623,7 +642,8 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
       if (e != hipSuccess) return hip_fail(c, e, "field upload");
       dfield = c->fstage;
     }
-    const VolArgs a = make_vol(pl, g, dfield, w);
+    VolArgs a = make_vol(pl, g, dfield, w);
+    if (bits) rows_vol(rg, bits, &a);
     hipError_t e = launch_count(pl, a, c->stream);
     // the scan also fills the coordinate tables and writes the sizes into
     // the pinned host words itself; a negative word afterwards (not
@@ -640,6 +660,7 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
     if (e != hipSuccess) return hip_fail(c, e, "count/scan");
     nv = c->pinned[1];
     nfc = c->pinned[3];
+    if (bits) rows_emit_tiling(&a, nv);
     c->vol = a;
   }
   c->field = *f;
@@ -1079,14 +1100,18 @@ int msh_autotune(void* ctx, const msh_field* f, const msh_params* p, int32_t* fa
   if (e == hipSuccess) e = hipEventCreate(&e1);
   int best = -1;
   float best_ms = 0.f;
+  const int before = c->family[base.method][base.T][cls];
   for (int fam = 3; fam >= 0 && e == hipSuccess; --fam) {
-    Plan q = base;
-    q.family = fam;
+    // the families count in units of their own
+    c->family[base.method][base.T][cls] = fam;
+    rc = msh_count(ctx, f, p, &nv, &nf);
+    if (rc) break;
+    const Plan q = c->plan;
     VolArgs a = c->vol;
     a.verts = c->ostage;
     a.faces = (int64_t*)((char*)c->ostage + vbytes);
     VolArgs probe = a;
-    if (variant_family(emit_variant(q, &probe)) != fam) continue;  // not for this volume
+    if (!a.bits && variant_family(emit_variant(q, &probe)) != fam) continue;  // not for this volume
     e = launch_emit(q, a, c->stream);  // warm-up
     // the best of at least 3 launches, and of as many as fill about 2 ms
     // (short launches vary more)
@@ -1109,11 +1134,12 @@ int msh_autotune(void* ctx, const msh_field* f, const msh_params* p, int32_t* fa
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
+  if (rc || e != hipSuccess) c->family[base.method][base.T][cls] = before;
+  if (rc) return rc;
   if (e != hipSuccess) return hip_fail(c, e, "autotune");
   c->family[base.method][base.T][cls] = best;
-  c->plan.family = best;
   if (family) *family = best;
-  return MSH_OK;
+  return msh_count(ctx, f, p, &nv, &nf);  // the state of the family chosen
 }
 
 int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_params* params,

@@ -89,6 +89,13 @@ struct VolArgs {
   int32_t czl;             // log2 of the waves that share a count tile's z segment
   int64_t cntiles;         // count tiles (x * y * z segments)
   int64_t cblk0;           // first count block of this volume in a batched launch
+  // the row kernels (rows.h); bits is null for the other kernels
+  uint32_t* bits;          // sample bits, 32 samples along z a word
+  int64_t xs;              // words of an x plane
+  int32_t sw, cw;          // words of a column of samples, of a row of cells
+  int32_t upx;             // units of an x plane
+  int32_t ue;              // units a wave emits one after another
+  uint32_t cwm, cwn;       // 2^32 / cw and 2^16 / cw, rounded down and up (word_pos)
   int32_t nti, ntj;        // emit tiles along x and y
   int64_t ntiles;          // emit tiles
   int64_t eblk0;           // first emit block of this volume in a batched launch
@@ -148,6 +155,21 @@ int variant_family(int variant);
 // the volume alone is too small to fill the device (not in a batch, whose
 // persistent launch is kept full by the other volumes)
 void count_tiling(const Plan& p, VolArgs* a, bool split);
+
+// The row kernels (rows.h): Geom::units in their units, and the layout of
+// the sample bits; false when they do not take the volume.
+struct RowsGeom {
+  int64_t xs;
+  int32_t sw, cw, upx;
+};
+bool rows_geom(const Plan& p, Geom* g, RowsGeom* r);
+// bytes of the sample bits, and VolArgs of a volume with its bits there
+size_t rows_bytes(const Geom& g, const RowsGeom& r);
+void rows_vol(const RowsGeom& r, void* bits, VolArgs* a);
+// emit tiling, once the number of vertices is known
+void rows_emit_tiling(VolArgs* a, int64_t nverts);
+hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st);
+hipError_t launch_rows_mc(const Plan& p, const VolArgs& a, hipStream_t st);
 
 hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream_t st);
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st);
@@ -218,6 +240,7 @@ hipError_t noalloc_setup(int device, void** ptr);
 hipError_t tables_setup(int device, hipStream_t st);
 hipError_t launch_count_tables(hipStream_t st);
 hipError_t launch_mt_tables(hipStream_t st);
+hipError_t launch_mc_image(hipStream_t st);
 // clamp = (0, min(nverts, vcap), 0, min(nfaces, fcap)) from the scan totals,
 // and sizes (when not null) = (nverts, nfaces); null totals count as zero.
 hipError_t launch_noalloc_sizes(const int64_t* totals, int64_t vcap, int64_t fcap, int64_t* clamp,

@@ -948,7 +948,7 @@ VolArgs make_vol(const Plan& p, const Geom& g, const void* field, const Workspac
 }
 
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st) {
-  return launch_count4(p, a, st);
+  return a.bits ? launch_rows_count(p, a, st) : launch_count4(p, a, st);
 }
 
 template <int METHOD, typename T, typename M, typename A, typename Out, int TX, int TY>
@@ -1027,6 +1027,7 @@ static hipError_t emit_any(const Plan& p, int variant, const VolArgs& a, const V
 
 hipError_t launch_emit(const Plan& p, const VolArgs& a0, hipStream_t st) {
   VolArgs a = a0;
+  if (a.bits) return launch_rows_mc(p, a, st);
   const int variant = emit_variant(p, &a);
   return emit_any(p, variant, a, nullptr, nullptr, 0, 0, nullptr, st);
 }

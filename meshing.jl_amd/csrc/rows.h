@@ -1,0 +1,184 @@
+// rows.h -- device helpers of the row kernels (rows.hip: sample bits and
+// counts; rows_mc.hip, rows_sn.hip, rows_mt.hip: the emits).
+//
+// A "column" (x, y) of samples keeps one bit per sample, set below the
+// level, 32 samples along z per word, z fastest in memory: word w of column
+// (x, y) is bits[x * xs + y * sw + w] (sw words a column, xs words an x
+// plane, rounded up to whole 128-byte lines).  Cells along z come 32 to a
+// word too (cw words a cell row), so 32 cells are classified at once from
+// the words of their four columns and those words moved down by one sample.
+//
+// A unit is 64 consecutive words of cells at one x in emission order (y,
+// then z): one lane a word, upx units an x plane, unit u = x * upx + g.  The
+// units' order is the reference's emission order (x outermost, z innermost,
+// src/marching_cubes.jl:40), so a unit's vertices and faces are one run of
+// each output array.
+#pragma once
+#include "device.h"
+
+namespace msh {
+
+// Word w of a column and the same moved down by one sample: bit b of c is
+// the sample at z = 32 w + b, bit b of s the one above it.
+struct Col {
+  uint32_t c, s;
+};
+
+// The cell words of a lane: (y, w) of word q = g * 64 + lane of an x plane,
+// its four columns (x, y), (x+1, y), (x, y+1), (x+1, y+1) and the cells that
+// exist; lanes past the plane's last word have none.
+struct CellWord {
+  uint32_t valid;
+  Col c00, c10, c01, c11;
+};
+// (y, w) of word q0 + i of an x plane, q0 = g * 64 and i < 64 * kMaxUE: q0 is
+// divided in scalar registers (cwm gives the quotient or one less); the
+// lanes' distance t from that row's start is below cw + 512, where a 16-bit
+// reciprocal is exact for short rows and a few compares serve the long ones.
+constexpr int kMaxUE = 8;  // units a wave emits, at most
+constexpr int kShortRow = 120;  // the reciprocal is exact up to 125 words
+struct WordBase {
+  uint32_t y0, w0;
+};
+__device__ __forceinline__ WordBase word_base(const VolArgs& a, int g) {
+  const uint32_t cw = (uint32_t)a.cw, q0 = (uint32_t)g * 64u;
+  uint32_t y0 = __umulhi(q0, a.cwm), w0 = q0 - y0 * cw;
+  if (w0 >= cw) {
+    ++y0;
+    w0 -= cw;
+  }
+  return {y0, w0};
+}
+__device__ __forceinline__ void word_pos(const VolArgs& a, const WordBase& o, uint32_t i, int* y,
+                                         int* w) {
+  const uint32_t cw = (uint32_t)a.cw, t = o.w0 + i;
+  uint32_t dy;
+  if (cw < (uint32_t)kShortRow) {
+    dy = (t * a.cwn) >> 16;
+  } else {  // t < cw + 512 < 6 cw
+    dy = (t >= cw) + (t >= 2 * cw) + (t >= 3 * cw) + (t >= 4 * cw) + (t >= 5 * cw);
+  }
+  *y = (int)(o.y0 + dy);
+  *w = (int)(t - dy * cw);
+}
+
+// A lane's cell words as loaded: the four columns' words and the next ones.
+struct RawWords {
+  uint32_t c[4], n[4];  // (x, y) (x+1, y) (x, y+1) (x+1, y+1)
+  uint32_t valid;
+};
+__device__ __forceinline__ RawWords load_raw(const VolArgs& a, int x, int g, int lane) {
+  RawWords r{};
+  int y, w;
+  word_pos(a, word_base(a, g), (uint32_t)lane, &y, &w);
+  if (y >= a.g.ny - 1) return r;
+  const int left = a.g.nz - 1 - 32 * w;  // cells from this word on
+  r.valid = left >= 32 ? ~0u : (1u << left) - 1u;
+  // a plane's words are counted in 32 bits; the word after a column's last
+  // one is the next column's or the padding behind the plane: its bits
+  // belong to no cell
+  const uint32_t* __restrict__ p0 = a.bits + (int64_t)x * a.xs;
+  const uint32_t* __restrict__ p1 = p0 + a.xs;
+  const uint32_t i = (uint32_t)y * (uint32_t)a.sw + (uint32_t)w, j = i + (uint32_t)a.sw;
+  r.c[0] = p0[i];
+  r.n[0] = p0[i + 1];
+  r.c[1] = p1[i];
+  r.n[1] = p1[i + 1];
+  r.c[2] = p0[j];
+  r.n[2] = p0[j + 1];
+  r.c[3] = p1[j];
+  r.n[3] = p1[j + 1];
+  return r;
+}
+__device__ __forceinline__ CellWord cell_word(const RawWords& r) {
+  CellWord c{};
+  c.valid = r.valid;
+  c.c00 = {r.c[0], __builtin_amdgcn_alignbit(r.n[0], r.c[0], 1)};
+  c.c10 = {r.c[1], __builtin_amdgcn_alignbit(r.n[1], r.c[1], 1)};
+  c.c01 = {r.c[2], __builtin_amdgcn_alignbit(r.n[2], r.c[2], 1)};
+  c.c11 = {r.c[3], __builtin_amdgcn_alignbit(r.n[3], r.c[3], 1)};
+  return c;
+}
+__device__ __forceinline__ CellWord load_cells(const VolArgs& a, int x, int g, int lane) {
+  return cell_word(load_raw(a, x, g, lane));
+}
+// cells with samples on both sides of the level
+__device__ __forceinline__ uint32_t active_cells(const CellWord& r) {
+  const uint32_t any = r.c00.c | r.c10.c | r.c01.c | r.c11.c | r.c00.s | r.c10.s | r.c01.s | r.c11.s;
+  const uint32_t all = r.c00.c & r.c10.c & r.c01.c & r.c11.c & r.c00.s & r.c10.s & r.c01.s & r.c11.s;
+  return any & ~all & r.valid;
+}
+// case of cell b in natural order: (x,y) (x+1,y) (x,y+1) (x+1,y+1), then above
+__device__ __forceinline__ uint32_t cell_case(const CellWord& r, int b) {
+  return ((r.c00.c >> b) & 1u) | (((r.c10.c >> b) & 1u) << 1) | (((r.c01.c >> b) & 1u) << 2) |
+         (((r.c11.c >> b) & 1u) << 3) | (((r.c00.s >> b) & 1u) << 4) |
+         (((r.c10.s >> b) & 1u) << 5) | (((r.c01.s >> b) & 1u) << 6) |
+         (((r.c11.s >> b) & 1u) << 7);
+}
+// the same for cell b of lane L's word
+__device__ __forceinline__ uint32_t cell_case_of(const CellWord& r, int L, int b) {
+  auto from = [&](uint32_t v) {
+    return ((uint32_t)__builtin_amdgcn_ds_bpermute(L << 2, (int)v) >> b) & 1u;
+  };
+  return from(r.c00.c) | (from(r.c10.c) << 1) | (from(r.c01.c) << 2) | (from(r.c11.c) << 3) |
+         (from(r.c00.s) << 4) | (from(r.c10.s) << 5) | (from(r.c01.s) << 6) | (from(r.c11.s) << 7);
+}
+
+// Emit tile t: kWaves x planes (one a wave, so the waves of a block read the
+// same lines) by a.ue units.  Tiles go over 8 blocks along x (32 planes, a
+// 128-byte line of Float32 samples), then along the planes, then to the next
+// 8 blocks, so the tiles in flight on an XCD share their lines in its L2.
+__device__ __forceinline__ void rows_tile(const VolArgs& a, int64_t t, int* x, int* g0) {
+  const uint32_t nxb = (uint32_t)(a.g.nx - 1 + kWaves - 1) / kWaves;
+  const uint32_t gb = (uint32_t)(a.upx + a.ue - 1) / (uint32_t)a.ue;
+  const uint32_t full = nxb / 8, rest = nxb - full * 8;
+  const uint32_t grp = (uint32_t)t / (8 * gb);
+  uint32_t r, n = 8, first = grp;
+  if (grp >= full) {
+    first = full;
+    n = rest;
+  }
+  r = (uint32_t)t - first * 8 * gb;
+  const uint32_t gi = r / n;
+  *x = (int)(first * 8 + (r - gi * n)) * kWaves + wave_id();
+  *g0 = (int)gi * a.ue;
+}
+
+// Two neighbouring values in one load (aligned as one of them).
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) Pair {
+  T a, b;
+};
+
+// 64 records of three values from LDS to the output: records [s0, s1) of the
+// 64 at `out`, the wave's lanes on consecutive values, so that every line is
+// written whole by one store instruction.  Buffer stores: a value outside
+// the records gets an offset past the buffer and is dropped, so there is no
+// branch, and a wait for loads issued before does not wait for the stores.
+// Non-temporal: a line is written once and whole, and kept out of the L2 it
+// leaves room there for the samples that the waves nearby share (301 x 217 x
+// 389 Float32 value noise 250 -> 172 us, 1024^3 Float64 5.39 -> 4.97 ms).
+template <typename V>
+__device__ __forceinline__ void store_records(V* __restrict__ out, const V* stage, int s0, int s1) {
+  const __amdgpu_buffer_rsrc_t r = buffer_rsrc(out, 192 * sizeof(V));
+  const int lane = lane_id();
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int e = lane + 64 * j;
+    const int off = e >= 3 * s0 && e < 3 * s1 ? e * (int)sizeof(V) : 0x7FFFFFFF;
+    const V v = stage[e];
+    if constexpr (sizeof(V) == 4) {
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, off, 0, 2);
+    } else {
+      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, 2);
+    }
+  }
+}
+
+__device__ __forceinline__ int64_t readlane64(int64_t v, int l) {
+  return ((int64_t)__builtin_amdgcn_readlane((int)((uint64_t)v >> 32), l) << 32) |
+         (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+}
+
+}  // namespace msh

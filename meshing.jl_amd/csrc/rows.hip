@@ -1,0 +1,238 @@
+// rows.hip -- the first two passes of the row kernels (see rows.h): the
+// sample bits of the whole field, and the vertex and face counts of every
+// unit from the bits.  Their scan is the one of the other kernels
+// (kernels.hip) over these units.
+#include <algorithm>
+
+#include "rows.h"
+
+#define MSH_LUT static __constant__
+#include "luts.h"
+
+namespace msh {
+namespace {
+
+// ---------------------------------------------------------------------------
+// Sample bits.  A block takes 64 * E columns along x and PW words along a
+// plane's (y, w) order; a wave makes PW / 4 of the words, each lane the words
+// of its E neighbouring columns from loads of E samples (16 at a time, all in
+// flight at once).  The words meet in LDS so that a column's PW words leave
+// together.  Every sample is read once and only once: this pass is bound by
+// HBM reads.
+template <typename T, int E>
+struct __attribute__((packed, aligned(sizeof(T)))) Vec {
+  T v[E];
+};
+
+template <typename T, int PW, int E>
+__device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
+  constexpr int PPW = PW / kWaves, X = kWave * E, ZB = 16;
+  __shared__ uint32_t words[X][PW + 1];
+  const Geom g = a.g;
+  const T thr = (T)a.thr;
+  const int lane = lane_id(), wv = wave_id();
+  const uint32_t nxt = (uint32_t)(g.nx + X - 1) / X;
+  const uint32_t tq = (uint32_t)t / nxt;
+  const int xb = (int)((uint32_t)t - tq * nxt) * X;
+  const uint32_t q0 = tq * PW, nq = (uint32_t)g.ny * (uint32_t)a.sw;
+  const uint64_t pbytes = (uint64_t)g.nx * (uint64_t)g.ny * sizeof(T);
+  // the lane's columns; at the row's end they move back to end with it (two
+  // lanes then make the same words)
+  const int xl = min(xb + lane * E, g.nx - E);
+  const uint32_t xo = (uint32_t)xl * (uint32_t)sizeof(T);
+#pragma unroll 1
+  for (int p = 0; p < PPW; ++p) {
+    const uint32_t q = q0 + (uint32_t)(wv * PPW + p);
+    uint32_t word[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) word[e] = 0;
+    if (q < nq) {
+      const uint32_t y = q / (uint32_t)a.sw, w = q - y * (uint32_t)a.sw;
+      const int n = min(32, g.nz - 32 * (int)w);  // samples of this word
+      const char* col = (const char*)a.f + (uint64_t)(32 * w) * pbytes +
+                        (uint64_t)y * (uint64_t)g.nx * sizeof(T);
+#pragma unroll
+      for (int zb = 0; zb < 32; zb += ZB) {
+        Vec<T, E> v[ZB];
+#pragma unroll
+        for (int z = 0; z < ZB; ++z)
+          v[z] = *(const Vec<T, E>*)(col + (uint64_t)min(zb + z, n - 1) * pbytes + xo);
+#pragma unroll
+        for (int z = 0; z < ZB; ++z)
+#pragma unroll
+          for (int e = 0; e < E; ++e) word[e] |= v[z].v[e] < thr ? 1u << (zb + z) : 0u;
+      }
+      if (n < 32)
+#pragma unroll
+        for (int e = 0; e < E; ++e) word[e] &= (1u << n) - 1u;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (xl + e >= xb) words[xl + e - xb][wv * PPW + p] = word[e];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < X * PW / kBlock; ++k) {
+    const int i = threadIdx.x + k * kBlock;
+    const int x = i / PW, p = i % PW;
+    if (xb + x < g.nx && q0 + p < nq) a.bits[(int64_t)(xb + x) * a.xs + q0 + p] = words[x][p];
+  }
+}
+
+template <typename T, int PW, int E>
+__global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
+  bits_tile<T, PW, E>(a, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// Counts, from the bits alone.  A wave counts kCountUnits units one after
+// another.  Marching Cubes: a cell's vertices are its crossing edges, 12
+// population counts of XORed words for 32 cells at once.  Its faces are its
+// vertices less 2 for each loop its surface makes, and a cell has one loop
+// unless a face of it is ambiguous (its corners alternate around the level)
+// or two opposite corners are cut off by themselves: those few cells, found
+// by ANDs of the same words, take their further loops from the table.
+constexpr int kCountUnits = 2;
+constexpr int kCountTile = kCountUnits * kWaves;
+
+__device__ __forceinline__ uint32_t mc_word_counts(const CellWord& r, const uint8_t* extra) {
+  const uint32_t x0 = r.c00.c ^ r.c10.c, x1 = r.c01.c ^ r.c11.c, x2 = r.c00.s ^ r.c10.s,
+                 x3 = r.c01.s ^ r.c11.s;  // edges along x at y, y+1, above y, above y+1
+  const uint32_t y0 = r.c00.c ^ r.c01.c, y1 = r.c10.c ^ r.c11.c, y2 = r.c00.s ^ r.c01.s,
+                 y3 = r.c10.s ^ r.c11.s;  // along y at x, x+1, above x, above x+1
+  const uint32_t z0 = r.c00.c ^ r.c00.s, z1 = r.c10.c ^ r.c10.s, z2 = r.c01.c ^ r.c01.s,
+                 z3 = r.c11.c ^ r.c11.s;  // along z at (x,y) (x+1,y) (x,y+1) (x+1,y+1)
+  const uint32_t m = r.valid;
+  const uint32_t act = (x0 | x1 | x2 | x3 | y0 | y1 | y2 | y3 | z0 | z1 | z2 | z3) & m;
+  if (__ballot(act != 0) == 0) return 0;
+  const uint32_t v = __popc(x0 & m) + __popc(x1 & m) + __popc(x2 & m) + __popc(x3 & m) +
+                     __popc(y0 & m) + __popc(y1 & m) + __popc(y2 & m) + __popc(y3 & m) +
+                     __popc(z0 & m) + __popc(z1 & m) + __popc(z2 & m) + __popc(z3 & m);
+  uint32_t more = (x0 & y1 & x1) | (x2 & y3 & x3) | (x0 & z1 & x2) | (x1 & z3 & x3) |
+                  (y0 & z2 & y2) | (y1 & z3 & y3);
+  more |= (x0 & y0 & z0) & (x3 & y3 & z3);
+  more |= (x0 & y1 & z1) & (x3 & y2 & z2);
+  more |= (x1 & y0 & z2) & (x2 & y3 & z1);
+  more |= (x1 & y1 & z3) & (x2 & y2 & z0);
+  more &= m;
+  uint32_t f = v - 2u * __popc(act);
+  while (more != 0) {
+    const int b = __builtin_ctz(more);
+    more &= more - 1;
+    f -= extra[cell_case(r, b)];
+  }
+  return v | (f << 16);
+}
+
+template <int METHOD>
+__device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, const uint8_t* extra) {
+  const int lane = lane_id();
+  const uint32_t u0 = (uint32_t)t * kCountTile + (uint32_t)(wave_id() * kCountUnits);
+  uint32_t* __restrict__ cnt = a.cnt + a.ubase;
+#pragma unroll
+  for (int k = 0; k < kCountUnits; ++k) {
+    const uint32_t u = u0 + (uint32_t)k;
+    if (u >= (uint32_t)a.g.units) return;
+    const uint32_t x = u / (uint32_t)a.upx, g = u - x * (uint32_t)a.upx;
+    const CellWord r = load_cells(a, (int)x, (int)g, lane);
+    uint32_t n = 0;  // vertices | faces << 16
+    if constexpr (METHOD == MC) n = mc_word_counts(r, extra);
+    const uint32_t incl = wave_scan_dpp(n);
+    if (lane == kWave - 1) cnt[u] = incl;
+  }
+}
+
+template <int METHOD>
+__global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a) {
+  // Marching Cubes: twice the loops of a case beyond its first
+  __shared__ uint8_t extra[256];
+  if constexpr (METHOD == MC) {
+    const uint32_t m = nat_to_mc(threadIdx.x);
+    const int v = (int)(MC_CASE_VERTS[m] & 0xF), f = (int)(MC_CASE_TRIS[m] & 7);
+    extra[threadIdx.x] = (uint8_t)(v > 0 ? v - f - 2 : 0);
+    __syncthreads();
+  }
+  rows_count_tile<METHOD>(a, blockIdx.x, extra);
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// Host side.
+
+bool rows_geom(const Plan& p, Geom* g, RowsGeom* r) {
+  if (p.method != MC || g->units == 0) return false;
+  r->sw = (g->nz + 31) / 32;
+  r->cw = (g->nz - 1 + 31) / 32;
+  const int64_t words = (int64_t)(g->ny - 1) * r->cw, plane = (int64_t)g->ny * r->sw;
+  if (plane >= (1ll << 30)) return false;  // word numbers of an x plane are 32-bit
+  r->upx = (int32_t)((words + 63) / 64);
+  r->xs = (plane + 31) / 32 * 32;
+  const int64_t units = (int64_t)(g->nx - 1) * r->upx;
+  if (units >= (1ll << 31) || (int64_t)((g->nx + 63) / 64) * ((plane + 7) / 8) >= (1ll << 31))
+    return false;  // block numbers are 32-bit
+  g->units = units;
+  return true;
+}
+
+size_t rows_bytes(const Geom& g, const RowsGeom& r) {
+  return align256((size_t)g.nx * (size_t)r.xs * 4 + 4);
+}
+
+void rows_vol(const RowsGeom& r, void* bits, VolArgs* a) {
+  a->bits = (uint32_t*)bits;
+  a->xs = r.xs;
+  a->sw = r.sw;
+  a->cw = r.cw;
+  a->upx = r.upx;
+  a->cwm = (uint32_t)std::min<uint64_t>((1ull << 32) / (uint64_t)r.cw, 0xFFFFFFFFull);
+  a->cwn = (65536u + (uint32_t)r.cw - 1u) / (uint32_t)r.cw;
+  a->cntiles = (a->g.units + kCountTile - 1) / kCountTile;
+}
+
+// Units a wave emits one after another: one where a unit alone has cells
+// enough to fill the queue's steps, several on sparse fields, whose units
+// would each pay the way to the first sample for a few cells (1024^3 Float32
+// sphere, 12 vertices a unit: 8 units 158 us, 1 unit 349 us; 1024^3 Float64
+// value noise, 520 vertices a unit: 1 unit 5.4 ms, 8 units 6.0 ms), as long
+// as the blocks fill the device.
+void rows_emit_tiling(VolArgs* a, int64_t nverts) {
+  const int64_t nxb = (a->g.nx - 1 + kWaves - 1) / kWaves;
+  a->ue = 1;
+  while (a->ue < kMaxUE && nverts * 2 * a->ue <= 256 * a->g.units &&
+         nxb * ((a->upx + 2 * a->ue - 1) / (2 * a->ue)) >= 8192)
+    a->ue *= 2;
+  a->ntiles = nxb * ((a->upx + a->ue - 1) / a->ue);
+}
+
+template <typename T, int PW, int E>
+static void launch_bits_e(const VolArgs& a, hipStream_t st) {
+  const int64_t nxt = (a.g.nx + kWave * E - 1) / (kWave * E), nq = (int64_t)a.g.ny * a.sw;
+  hipLaunchKernelGGL((k_bits<T, PW, E>), dim3((unsigned)(nxt * ((nq + PW - 1) / PW))), dim3(kBlock),
+                     0, st, a);
+}
+
+// 2 columns a lane: against 1 and 4 the fastest on large volumes (1024^3
+// Float64 1.69 ms, 1.77 with 1; Float32 0.876, 0.90 and 0.888) and as fast
+// on small ones, where shorter tiles (8 words, 256 x 256 x 256 Float32 11.8
+// us) beat the longer ones (32 words, 18 us) until those fill the device.
+template <typename T>
+static void launch_bits_t(const VolArgs& a, hipStream_t st) {
+  const int64_t nxt = (a.g.nx + 2 * kWave - 1) / (2 * kWave), nq = (int64_t)a.g.ny * a.sw;
+  if (nxt * ((nq + 31) / 32) >= 2048)
+    launch_bits_e<T, 32, 2>(a, st);
+  else
+    launch_bits_e<T, 8, 2>(a, st);
+}
+
+hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st) {
+  if (a.cntiles == 0) return hipSuccess;
+  if (p.T == K_F32)
+    launch_bits_t<float>(a, st);
+  else
+    launch_bits_t<double>(a, st);
+  hipLaunchKernelGGL((k_rows_count<MC>), dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a);
+  return hipGetLastError();
+}
+
+}  // namespace msh
