@@ -622,7 +622,8 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
   if (rows_family(pl) && rows_geom(pl, &gr, &rg)) {
     // with no room for the sample bits the other kernels, which need less,
     // take the volume
-    if (setup_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg), &bits) == MSH_OK)
+    if (setup_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr),
+                        &bits) == MSH_OK)
       g = gr;
     else
       (void)hipGetLastError();
@@ -643,7 +644,7 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
       dfield = c->fstage;
     }
     VolArgs a = make_vol(pl, g, dfield, w);
-    if (bits) rows_vol(rg, bits, &a);
+    if (bits) rows_vol(rg, bits, (char*)bits + rows_bytes(gr, rg), &a);
     hipError_t e = launch_count(pl, a, c->stream);
     // the scan also fills the coordinate tables and writes the sizes into
     // the pinned host words itself; a negative word afterwards (not

@@ -91,6 +91,8 @@ struct VolArgs {
   int64_t cblk0;           // first count block of this volume in a batched launch
   // the row kernels (rows.h); bits is null for the other kernels
   uint32_t* bits;          // sample bits, 32 samples along z a word
+  uint16_t* wpre;          // per cell word of a unit: vertices before it in the unit
+                           // (surface nets), from ubase
   int64_t xs;              // words of an x plane
   int32_t sw, cw;          // words of a column of samples, of a row of cells
   int32_t upx;             // units of an x plane
@@ -165,11 +167,13 @@ struct RowsGeom {
 bool rows_geom(const Plan& p, Geom* g, RowsGeom* r);
 // bytes of the sample bits, and VolArgs of a volume with its bits there
 size_t rows_bytes(const Geom& g, const RowsGeom& r);
-void rows_vol(const RowsGeom& r, void* bits, VolArgs* a);
+size_t rows_prefix_bytes(const Plan& p, const Geom& g);  // .. of VolArgs::wpre
+void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a);
 // emit tiling, once the number of vertices is known
 void rows_emit_tiling(VolArgs* a, int64_t nverts);
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st);
 hipError_t launch_rows_mc(const Plan& p, const VolArgs& a, hipStream_t st);
+hipError_t launch_rows_sn(const Plan& p, const VolArgs& a, hipStream_t st);
 
 hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream_t st);
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st);

@@ -29,6 +29,7 @@ struct Col {
 // exist; lanes past the plane's last word have none.
 struct CellWord {
   uint32_t valid;
+  int y, w;
   Col c00, c10, c01, c11;
 };
 // (y, w) of word q0 + i of an x plane, q0 = g * 64 and i < 64 * kMaxUE: q0 is
@@ -66,11 +67,14 @@ __device__ __forceinline__ void word_pos(const VolArgs& a, const WordBase& o, ui
 struct RawWords {
   uint32_t c[4], n[4];  // (x, y) (x+1, y) (x, y+1) (x+1, y+1)
   uint32_t valid;
+  int y, w;
 };
 __device__ __forceinline__ RawWords load_raw(const VolArgs& a, int x, int g, int lane) {
   RawWords r{};
   int y, w;
   word_pos(a, word_base(a, g), (uint32_t)lane, &y, &w);
+  r.y = y;
+  r.w = w;
   if (y >= a.g.ny - 1) return r;
   const int left = a.g.nz - 1 - 32 * w;  // cells from this word on
   r.valid = left >= 32 ? ~0u : (1u << left) - 1u;
@@ -93,6 +97,8 @@ __device__ __forceinline__ RawWords load_raw(const VolArgs& a, int x, int g, int
 __device__ __forceinline__ CellWord cell_word(const RawWords& r) {
   CellWord c{};
   c.valid = r.valid;
+  c.y = r.y;
+  c.w = r.w;
   c.c00 = {r.c[0], __builtin_amdgcn_alignbit(r.n[0], r.c[0], 1)};
   c.c10 = {r.c[1], __builtin_amdgcn_alignbit(r.n[1], r.c[1], 1)};
   c.c01 = {r.c[2], __builtin_amdgcn_alignbit(r.n[2], r.c[2], 1)};
@@ -124,6 +130,45 @@ __device__ __forceinline__ uint32_t cell_case_of(const CellWord& r, int L, int b
          (from(r.c00.s) << 4) | (from(r.c10.s) << 5) | (from(r.c01.s) << 6) | (from(r.c11.s) << 7);
 }
 
+// The five columns around a lane's cell words that hold corners of the cells
+// at -x, -y and both: (x-1, y) (x-1, y+1) (x, y-1) (x+1, y-1) (x-1, y-1).
+// Zero where they do not exist.
+struct BackWords {
+  Col x0, x1, y0, y1, xy;
+};
+__device__ __forceinline__ BackWords load_back(const VolArgs& a, int x, const CellWord& r) {
+  BackWords k{};
+  if (r.valid == 0) return k;
+  const uint32_t* __restrict__ p0 = a.bits + (int64_t)x * a.xs;
+  const uint32_t sw = (uint32_t)a.sw, i = (uint32_t)r.y * sw + (uint32_t)r.w;
+  auto col = [](const uint32_t* __restrict__ p, uint32_t j) -> Col {
+    const uint32_t c = p[j];
+    return {c, __builtin_amdgcn_alignbit(p[j + 1], c, 1)};
+  };
+  if (r.y > 0) {
+    k.y0 = col(p0, i - sw);
+    k.y1 = col(p0 + a.xs, i - sw);
+  }
+  if (x > 0) {
+    const uint32_t* __restrict__ pm = p0 - a.xs;
+    k.x0 = col(pm, i);
+    k.x1 = col(pm, i + sw);
+    if (r.y > 0) k.xy = col(pm, i - sw);
+  }
+  return k;
+}
+// active cells of the word of columns a, b, c, d
+__device__ __forceinline__ uint32_t active_of(const Col& a, const Col& b, const Col& c, const Col& d,
+                                              uint32_t valid) {
+  return ((a.c | b.c | c.c | d.c | a.s | b.s | c.s | d.s) &
+          ~(a.c & b.c & c.c & d.c & a.s & b.s & c.s & d.s)) & valid;
+}
+// First vertex (in the volume's numbering) of cell word q of x plane x.
+__device__ __forceinline__ int64_t word_vertex(const VolArgs& a, int x, uint32_t q) {
+  const int64_t u = (int64_t)x * a.upx + (q >> 6);
+  return a.voff[a.ubase + u] + (int64_t)a.wpre[64 * (a.ubase + u) + (q & 63)];
+}
+
 // Emit tile t: kWaves x planes (one a wave, so the waves of a block read the
 // same lines) by a.ue units.  Tiles go over 8 blocks along x (32 planes, a
 // 128-byte line of Float32 samples), then along the planes, then to the next
@@ -149,6 +194,21 @@ template <typename T>
 struct __attribute__((packed, aligned(sizeof(T)))) Pair {
   T a, b;
 };
+
+// Emit tile of block b.  Blocks are dealt round-robin to the 8 XCDs; a launch
+// of few blocks gives each XCD one run of tiles (xcd_tile), a larger one runs
+// of 32 in turn, so tiles that share lines meet in one L2 and a field whose
+// surface lies in a part of its planes still keeps every XCD busy (1024^3
+// Float32 sphere emit 158 -> 132 us; the 2048 blocks of a 256^3 gyroid are
+// 36 us in one run an XCD and 39 in turns).
+__device__ __forceinline__ int64_t rows_block_tile(int64_t b, int64_t nb) {
+  constexpr int64_t C = 32;
+  if (nb < 8192) return xcd_tile(b, nb);
+  if (b >= nb / (8 * C) * (8 * C)) return b;
+  // (turned by one XCD a round: the y range of a plane is not one XCD's)
+  const int64_t round = (b >> 3) / C, at = (b >> 3) % C;
+  return (round * 8 + (((b & 7) + round) & 7)) * C + at;
+}
 
 // 64 records of three values from LDS to the output: records [s0, s1) of the
 // 64 at `out`, the wave's lanes on consecutive values, so that every line is

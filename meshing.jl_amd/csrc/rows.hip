@@ -124,6 +124,17 @@ __device__ __forceinline__ uint32_t mc_word_counts(const CellWord& r, const uint
   return v | (f << 16);
 }
 
+// Surface nets: a vertex per active cell, and two faces for each of its
+// crossing edges at corner 0 whose four cells exist.
+__device__ __forceinline__ uint32_t sn_word_counts(const CellWord& r, bool xin) {
+  const uint32_t ym = r.y > 0 ? ~0u : 0u, zm = r.w > 0 ? ~0u : ~1u, xm = xin ? ~0u : 0u;
+  const uint32_t m = r.valid;
+  const uint32_t q = __popc((r.c00.c ^ r.c10.c) & m & ym & zm) +
+                     __popc((r.c00.c ^ r.c01.c) & m & zm & xm) +
+                     __popc((r.c00.c ^ r.c00.s) & m & xm & ym);
+  return __popc(active_cells(r)) | (q << 17);
+}
+
 template <int METHOD>
 __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, const uint8_t* extra) {
   const int lane = lane_id();
@@ -137,8 +148,11 @@ __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, con
     const CellWord r = load_cells(a, (int)x, (int)g, lane);
     uint32_t n = 0;  // vertices | faces << 16
     if constexpr (METHOD == MC) n = mc_word_counts(r, extra);
+    if constexpr (METHOD == SN) n = sn_word_counts(r, x > 0);
     const uint32_t incl = wave_scan_dpp(n);
     if (lane == kWave - 1) cnt[u] = incl;
+    if constexpr (METHOD != MC)
+      a.wpre[64 * (a.ubase + u) + lane] = (uint16_t)((incl - n) & 0xFFFF);
   }
 }
 
@@ -161,11 +175,13 @@ __global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a) {
 // Host side.
 
 bool rows_geom(const Plan& p, Geom* g, RowsGeom* r) {
-  if (p.method != MC || g->units == 0) return false;
+  if (p.method == MT || g->units == 0) return false;
   r->sw = (g->nz + 31) / 32;
   r->cw = (g->nz - 1 + 31) / 32;
   const int64_t words = (int64_t)(g->ny - 1) * r->cw, plane = (int64_t)g->ny * r->sw;
   if (plane >= (1ll << 30)) return false;  // word numbers of an x plane are 32-bit
+  // vertices one x plane and one row apart are told apart by 32 bits
+  if (p.method != MC && (int64_t)(g->ny + 1) * g->nz >= (1ll << 31)) return false;
   r->upx = (int32_t)((words + 63) / 64);
   r->xs = (plane + 31) / 32 * 32;
   const int64_t units = (int64_t)(g->nx - 1) * r->upx;
@@ -179,8 +195,13 @@ size_t rows_bytes(const Geom& g, const RowsGeom& r) {
   return align256((size_t)g.nx * (size_t)r.xs * 4 + 4);
 }
 
-void rows_vol(const RowsGeom& r, void* bits, VolArgs* a) {
+size_t rows_prefix_bytes(const Plan& p, const Geom& g) {
+  return p.method == MC ? 0 : align256((size_t)g.units * 64 * sizeof(uint16_t));
+}
+
+void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a) {
   a->bits = (uint32_t*)bits;
+  a->wpre = (uint16_t*)wpre;
   a->xs = r.xs;
   a->sw = r.sw;
   a->cw = r.cw;
@@ -198,8 +219,9 @@ void rows_vol(const RowsGeom& r, void* bits, VolArgs* a) {
 // as the blocks fill the device.
 void rows_emit_tiling(VolArgs* a, int64_t nverts) {
   const int64_t nxb = (a->g.nx - 1 + kWaves - 1) / kWaves;
+  const int64_t full = a->method == MC ? 256 : 64;  // about 64 cells
   a->ue = 1;
-  while (a->ue < kMaxUE && nverts * 2 * a->ue <= 256 * a->g.units &&
+  while (a->ue < kMaxUE && nverts * 2 * a->ue <= full * a->g.units &&
          nxb * ((a->upx + 2 * a->ue - 1) / (2 * a->ue)) >= 8192)
     a->ue *= 2;
   a->ntiles = nxb * ((a->upx + a->ue - 1) / a->ue);
@@ -231,7 +253,8 @@ hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st) {
     launch_bits_t<float>(a, st);
   else
     launch_bits_t<double>(a, st);
-  hipLaunchKernelGGL((k_rows_count<MC>), dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a);
+  const auto k = p.method == MC ? k_rows_count<MC> : k_rows_count<SN>;
+  hipLaunchKernelGGL(k, dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a);
   return hipGetLastError();
 }
 

@@ -249,7 +249,7 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
 
 template <typename T, typename M, typename Out, int CXM>
 __global__ __launch_bounds__(kBlock) void k_rows_mc(VolArgs a) {
-  rows_mc_tile<T, M, Out, CXM>(a, xcd_tile(blockIdx.x, a.ntiles));
+  rows_mc_tile<T, M, Out, CXM>(a, rows_block_tile(blockIdx.x, a.ntiles));
 }
 
 }  // namespace
