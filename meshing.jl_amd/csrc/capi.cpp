@@ -442,6 +442,7 @@ hipError_t tables_setup(int device, hipStream_t st) {
   hipError_t e = launch_count_tables(st);
   if (e == hipSuccess) e = launch_mt_tables(st);
   if (e == hipSuccess) e = launch_mc_image(st);
+  if (e == hipSuccess) e = launch_mt_image(st);
   // complete before any context's stream can launch a kernel that reads them
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e == hipSuccess) done[device] = true;

@@ -92,7 +92,7 @@ struct VolArgs {
   // the row kernels (rows.h); bits is null for the other kernels
   uint32_t* bits;          // sample bits, 32 samples along z a word
   uint16_t* wpre;          // per cell word of a unit: vertices before it in the unit
-                           // (surface nets), from ubase
+                           // (tetrahedra and surface nets), from ubase
   int64_t xs;              // words of an x plane
   int32_t sw, cw;          // words of a column of samples, of a row of cells
   int32_t upx;             // units of an x plane
@@ -174,6 +174,7 @@ void rows_emit_tiling(VolArgs* a, int64_t nverts);
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st);
 hipError_t launch_rows_mc(const Plan& p, const VolArgs& a, hipStream_t st);
 hipError_t launch_rows_sn(const Plan& p, const VolArgs& a, hipStream_t st);
+hipError_t launch_rows_mt(const Plan& p, const VolArgs& a, hipStream_t st);
 
 hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream_t st);
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st);
@@ -245,6 +246,7 @@ hipError_t tables_setup(int device, hipStream_t st);
 hipError_t launch_count_tables(hipStream_t st);
 hipError_t launch_mt_tables(hipStream_t st);
 hipError_t launch_mc_image(hipStream_t st);
+hipError_t launch_mt_image(hipStream_t st);
 // clamp = (0, min(nverts, vcap), 0, min(nfaces, fcap)) from the scan totals,
 // and sizes (when not null) = (nverts, nfaces); null totals count as zero.
 hipError_t launch_noalloc_sizes(const int64_t* totals, int64_t vcap, int64_t fcap, int64_t* clamp,

@@ -1027,7 +1027,10 @@ static hipError_t emit_any(const Plan& p, int variant, const VolArgs& a, const V
 
 hipError_t launch_emit(const Plan& p, const VolArgs& a0, hipStream_t st) {
   VolArgs a = a0;
-  if (a.bits) return p.method == MC ? launch_rows_mc(p, a, st) : launch_rows_sn(p, a, st);
+  if (a.bits)
+    return p.method == MC   ? launch_rows_mc(p, a, st)
+           : p.method == MT ? launch_rows_mt(p, a, st)
+                            : launch_rows_sn(p, a, st);
   const int variant = emit_variant(p, &a);
   return emit_any(p, variant, a, nullptr, nullptr, 0, 0, nullptr, st);
 }

@@ -210,24 +210,29 @@ __device__ __forceinline__ int64_t rows_block_tile(int64_t b, int64_t nb) {
   return (round * 8 + (((b & 7) + round) & 7)) * C + at;
 }
 
-// 64 records of three values from LDS to the output: records [s0, s1) of the
-// 64 at `out`, the wave's lanes on consecutive values, so that every line is
+// 64 records of three values from LDS to the output, each through `value`:
+// records [s0, s1) of the 64 at `out`, the wave's lanes on consecutive values, so that every line is
 // written whole by one store instruction.  Buffer stores: a value outside
 // the records gets an offset past the buffer and is dropped, so there is no
 // branch, and a wait for loads issued before does not wait for the stores.
 // Non-temporal: a line is written once and whole, and kept out of the L2 it
 // leaves room there for the samples that the waves nearby share (301 x 217 x
 // 389 Float32 value noise 250 -> 172 us, 1024^3 Float64 5.39 -> 4.97 ms).
-template <typename V>
-__device__ __forceinline__ void store_records(V* __restrict__ out, const V* stage, int s0, int s1) {
-  const __amdgpu_buffer_rsrc_t r = buffer_rsrc(out, 192 * sizeof(V));
+struct Same {
+  template <typename V>
+  __device__ V operator()(V v) const { return v; }
+};
+template <typename O, typename V, class F = Same>
+__device__ __forceinline__ void store_records(O* __restrict__ out, const V* stage, int s0, int s1,
+                                              F value = F{}) {
+  const __amdgpu_buffer_rsrc_t r = buffer_rsrc(out, 192 * sizeof(O));
   const int lane = lane_id();
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int e = lane + 64 * j;
-    const int off = e >= 3 * s0 && e < 3 * s1 ? e * (int)sizeof(V) : 0x7FFFFFFF;
-    const V v = stage[e];
-    if constexpr (sizeof(V) == 4) {
+    const int off = e >= 3 * s0 && e < 3 * s1 ? e * (int)sizeof(O) : 0x7FFFFFFF;
+    const O v = value(stage[e]);
+    if constexpr (sizeof(O) == 4) {
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, off, 0, 2);
     } else {
       typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));

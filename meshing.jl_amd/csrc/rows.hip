@@ -135,6 +135,55 @@ __device__ __forceinline__ uint32_t sn_word_counts(const CellWord& r, bool xin) 
   return __popc(active_cells(r)) | (q << 17);
 }
 
+// Marching Tetrahedra.  Faces: a tetrahedron whose corners differ has one
+// where an odd number of them is below the level and two where two are.
+// Vertices: crossing edges that the cell owns, the seven that end at its far
+// corner and, on the volume's first layers, those whose end corner lies on
+// the layer (src/marching_tetrahedra.jl:67-84: the first voxel to request an
+// edge owns its vertex).
+constexpr int kMtA[19] = {0, 1, 3, 0, 4, 5, 7, 4, 0, 1, 2, 3, 0, 0, 0, 4, 1, 3, 0};
+constexpr int kMtB[19] = {1, 2, 2, 3, 5, 6, 6, 7, 4, 5, 6, 7, 2, 7, 5, 6, 6, 6, 6};
+constexpr int kMtXyz[8] = {0, 2, 3, 1, 4, 6, 7, 5};  // dx | dy << 1 | dz << 2
+constexpr int kMtTets[6][2] = {{2, 1}, {7, 3}, {3, 2}, {1, 5}, {4, 7}, {5, 4}};  // beside 0 and 6
+
+__device__ __forceinline__ uint32_t mt_word_counts(const CellWord& r, bool x0) {
+  const uint32_t w[8] = {r.c00.c, r.c01.c, r.c11.c, r.c10.c, r.c00.s, r.c01.s, r.c11.s, r.c10.s};
+  const uint32_t m = r.valid;
+  if (__ballot(active_cells(r) != 0) == 0) return 0;
+  uint32_t f = 0;
+  const uint32_t odd06 = w[0] ^ w[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const uint32_t p = w[kMtTets[k][0]], q = w[kMtTets[k][1]];
+    const uint32_t odd = (odd06 ^ p ^ q) & m;
+    const uint32_t differ = ((w[0] | w[6] | p | q) & ~(w[0] & w[6] & p & q)) & m;
+    f += __popc(odd) + 2u * __popc(differ & ~odd);
+  }
+  const bool y0 = r.y == 0, z0 = r.w == 0;
+  uint32_t v = 0;
+#pragma unroll
+  for (int e = 0; e < 19; ++e) {
+    const int back = 7 & ~kMtXyz[kMtB[e]];  // axes on which the edge's end corner is at 0
+    if (back == 0) {
+      v += __popc((w[kMtA[e]] ^ w[kMtB[e]]) & m);
+    } else if (back == 4) {
+      v += z0 ? (w[kMtA[e]] ^ w[kMtB[e]]) & m & 1u : 0u;
+    }
+  }
+  if (__ballot(x0 || y0) != 0) {
+#pragma unroll
+    for (int e = 0; e < 19; ++e) {
+      const int back = 7 & ~kMtXyz[kMtB[e]];
+      if (!(back & 3)) continue;
+      uint32_t own = (back & 4) ? (z0 ? 1u : 0u) : ~0u;
+      if ((back & 1) && !x0) own = 0;
+      if ((back & 2) && !y0) own = 0;
+      v += __popc((w[kMtA[e]] ^ w[kMtB[e]]) & m & own);
+    }
+  }
+  return v | (f << 16);
+}
+
 template <int METHOD>
 __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, const uint8_t* extra) {
   const int lane = lane_id();
@@ -148,6 +197,7 @@ __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, con
     const CellWord r = load_cells(a, (int)x, (int)g, lane);
     uint32_t n = 0;  // vertices | faces << 16
     if constexpr (METHOD == MC) n = mc_word_counts(r, extra);
+    if constexpr (METHOD == MT) n = mt_word_counts(r, x == 0);
     if constexpr (METHOD == SN) n = sn_word_counts(r, x > 0);
     const uint32_t incl = wave_scan_dpp(n);
     if (lane == kWave - 1) cnt[u] = incl;
@@ -175,13 +225,15 @@ __global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a) {
 // Host side.
 
 bool rows_geom(const Plan& p, Geom* g, RowsGeom* r) {
-  if (p.method == MT || g->units == 0) return false;
+  if (g->units == 0) return false;
   r->sw = (g->nz + 31) / 32;
   r->cw = (g->nz - 1 + 31) / 32;
   const int64_t words = (int64_t)(g->ny - 1) * r->cw, plane = (int64_t)g->ny * r->sw;
   if (plane >= (1ll << 30)) return false;  // word numbers of an x plane are 32-bit
   // vertices one x plane and one row apart are told apart by 32 bits
-  if (p.method != MC && (int64_t)(g->ny + 1) * g->nz >= (1ll << 31)) return false;
+  // (a cell owns at most 13)
+  if (p.method != MC && (int64_t)(g->ny + 1) * g->nz * (p.method == MT ? 13 : 1) >= (1ll << 31))
+    return false;
   r->upx = (int32_t)((words + 63) / 64);
   r->xs = (plane + 31) / 32 * 32;
   const int64_t units = (int64_t)(g->nx - 1) * r->upx;
@@ -253,7 +305,7 @@ hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st) {
     launch_bits_t<float>(a, st);
   else
     launch_bits_t<double>(a, st);
-  const auto k = p.method == MC ? k_rows_count<MC> : k_rows_count<SN>;
+  const auto k = p.method == MC ? k_rows_count<MC> : p.method == MT ? k_rows_count<MT> : k_rows_count<SN>;
   hipLaunchKernelGGL(k, dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a);
   return hipGetLastError();
 }
