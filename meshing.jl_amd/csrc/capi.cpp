@@ -41,9 +41,10 @@ struct Launch {
 // tetrahedra 3: the 256^3 gyroid emits take 0.056, 0.12 and 0.17 ms);
 // counting costs the same per cell for every method.
 double cell_cost(const VolArgs& v, const Plan& p, bool emit) {
+  const double w = p.method == MT ? 3.0 : p.method == SN ? 2.0 : 1.0;
+  if (v.bits) return (double)v.g.units * (emit ? w : 1.0);
   const double zc = (double)(v.g.zseg > 0 ? v.g.zseg : 0);
-  return emit ? (double)v.ntiles * zc * (p.method == MT ? 3.0 : p.method == SN ? 2.0 : 1.0)
-              : (double)v.cntiles * zc;
+  return emit ? (double)v.ntiles * zc * w : (double)v.cntiles * zc;
 }
 
 // Launch order for spreading: most work first (each goes to the stream with
@@ -73,9 +74,10 @@ struct BatchState {
   std::vector<msh_params> params;
   std::vector<Plan> plans;
   std::vector<VolArgs> vols;       // host copy of the device descriptors
-  std::vector<Launch> counts, emits;
+  std::vector<Launch> bits, counts, emits;  // bits: sample-bit launches of the row kernels
+  bool rows = false;               // every volume goes through the row kernels
   std::vector<int64_t> sizes;      // 4 per volume: first vertex, nverts, first face, nfaces
-  int64_t units = 0, ncoords = 0, cblocks = 0, eblocks = 0;
+  int64_t units = 0, ncoords = 0, cblocks = 0, eblocks = 0, bblocks = 0;
   size_t ctr_off = 0;              // work-queue counters in the batch workspace: 8 per
                                    // count launch, then 8 per emit launch
 };
@@ -778,6 +780,11 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   if (rc) return rc;
   b.plans.assign((size_t)n, Plan{});
   std::vector<Geom> geoms((size_t)n);
+  // the row kernels take the batch when they take every volume of it (its
+  // units are scanned together)
+  std::vector<Geom> rgeoms((size_t)n);
+  std::vector<RowsGeom> rows((size_t)n);
+  b.rows = true;
   for (int v = 0; v < n; ++v) {
     rc = make_plan(c, &fields[v], &params[v], &b.plans[v]);
     if (rc) {
@@ -788,6 +795,9 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     geoms[v] = make_geom(&fields[v], b.plans[v].method, true);
     if (geoms[v].units > 0 && !fields[v].data)
       return fail(c, MSH_ERR_ARGUMENT, "volume " + std::to_string(v) + ": null field data");
+    rgeoms[v] = geoms[v];
+    if (geoms[v].units > 0)
+      b.rows = b.rows && rows_family(b.plans[v]) && rows_geom(b.plans[v], &rgeoms[v], &rows[v]);
   }
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, MSH_ERR_DEVICE, "hipSetDevice");
 
@@ -805,7 +815,26 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     }
   }
   Workspace w{};
-  rc = setup_workspace(c, units, ncoords, &w);
+  void* bits = nullptr;
+  if (b.rows && units > 0) {
+    int64_t runits = 0;
+    size_t extra = 0;
+    for (int v = 0; v < n; ++v) {
+      if (geoms[v].units == 0) continue;
+      runits += rgeoms[v].units;
+      extra += rows_bytes(rgeoms[v], rows[v]);
+    }
+    // (with no room for the sample bits the other kernels take the batch)
+    extra += align256((size_t)runits * 64 * sizeof(uint16_t));
+    if (setup_workspace(c, runits, ncoords, &w, extra, &bits) == MSH_OK) {
+      units = runits;
+      geoms = rgeoms;
+    } else {
+      (void)hipGetLastError();
+    }
+  }
+  b.rows = bits != nullptr;
+  if (!bits) rc = setup_workspace(c, units, ncoords, &w);
   if (rc) return rc;
   if (hbytes) {
     rc = grow(c, &c->fstage, &c->fstage_bytes, hbytes, "field staging allocation");
@@ -817,6 +846,8 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   b.vols.assign((size_t)n, VolArgs{});
   std::vector<int> emit_var((size_t)n, 0);
   int64_t ubase = 0, cbase = 0;
+  uint16_t* wpre = (uint16_t*)bits;
+  char* vbits = (char*)bits + align256((size_t)units * 64 * sizeof(uint16_t));
   for (int v = 0; v < n; ++v) {
     const void* df = fields[v].data;
     if (fields[v].memory == MSH_HOST && geoms[v].units > 0) df = (char*)c->fstage + hoff[v];
@@ -826,14 +857,22 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     a.ubase = ubase;
     a.sz = nullptr;  // set below, once the sizes array is placed
     emit_var[v] = emit_variant(b.plans[v], &a);
+    if (bits && geoms[v].units > 0) {
+      rows_vol(rows[v], vbits, wpre, &a);
+      rows_emit_tiling(&a, -1);
+      vbits += rows_bytes(geoms[v], rows[v]);
+      emit_var[v] = kRowsVariant + cx_class(a);
+    }
     if (geoms[v].units == 0) {
       a.cntiles = 0;
       a.ntiles = 0;
+      a.bntiles = 0;
     }
     b.vols[v] = a;
     ubase += geoms[v].units;
     cbase += (int64_t)geoms[v].nx + geoms[v].ny + geoms[v].nz;
   }
+  b.bits.clear();
   b.counts.clear();
   b.emits.clear();
   // Within a launch, the volumes' tiles are queued longest first (a tile
@@ -844,6 +883,21 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   std::stable_sort(ord.begin(), ord.end(),
                    [&](int x, int y) { return geoms[x].nz > geoms[y].nz; });
   std::vector<char> done((size_t)n, 0);
+  int64_t bblocks = 0;
+  if (b.rows)
+    for (int T : {(int)K_F32, (int)K_F64}) {
+      Launch L;
+      L.plan.T = T;
+      L.gbase = bblocks;
+      for (int u : ord) {
+        if (b.plans[u].T != T) continue;
+        b.vols[u].bblk0 = bblocks;
+        bblocks += b.vols[u].bntiles;
+      }
+      L.nblocks = bblocks - L.gbase;
+      L.cost = (double)L.nblocks * (T == K_F64 ? 2.0 : 1.0);
+      if (L.nblocks) b.bits.push_back(L);
+    }
   int64_t cblocks = 0;
   for (int v : ord) {
     if (done[v]) continue;
@@ -851,7 +905,9 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     L.plan = b.plans[v];
     L.gbase = cblocks;
     for (int u : ord) {
-      if (done[u] || b.plans[u].T != L.plan.T || b.plans[u].method != L.plan.method) continue;
+      // (the row kernels count from the bits, whatever the element type)
+      if (done[u] || (!b.rows && b.plans[u].T != L.plan.T) || b.plans[u].method != L.plan.method)
+        continue;
       done[u] = 1;
       b.vols[u].cblk0 = cblocks;
       cblocks += b.vols[u].cntiles;
@@ -878,17 +934,18 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     L.nblocks = eblocks - L.gbase;
     if (L.nblocks) b.emits.push_back(L);
   }
-  if (cblocks > INT32_MAX || eblocks > INT32_MAX)
+  if (cblocks > INT32_MAX || eblocks > INT32_MAX || bblocks > INT32_MAX)
     return fail(c, MSH_ERR_ARGUMENT, "batch too large for one launch");
 
   // device side: descriptors | cmap | emap | sizes
   const size_t b_vols = align256(sizeof(VolArgs) * (size_t)(n > 0 ? n : 1));
   const size_t b_cmap = align256(4 * (size_t)(cblocks + 1));
   const size_t b_emap = align256(4 * (size_t)(eblocks + 1));
+  const size_t b_bmap = b.rows ? align256(4 * (size_t)(bblocks + 1)) : 0;
   const size_t b_sizes = align256(32 * (size_t)(n > 0 ? n : 1));
   const size_t nctr = 8 * (b.counts.size() + b.emits.size());
   const size_t b_ctr = align256(4 * (nctr + 1));
-  rc = grow(c, &c->bws, &c->bws_bytes, b_vols + b_cmap + b_emap + b_sizes + b_ctr,
+  rc = grow(c, &c->bws, &c->bws_bytes, b_vols + b_cmap + b_emap + b_sizes + b_ctr + b_bmap,
             "batch workspace");
   if (rc) return rc;
   VolArgs* dvols = (VolArgs*)c->bws;
@@ -897,6 +954,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   int64_t* dsizes = (int64_t*)((char*)emap + b_emap);
   b.ctr_off = b_vols + b_cmap + b_emap + b_sizes;
   uint32_t* ctrs = (uint32_t*)((char*)c->bws + b.ctr_off);
+  int32_t* bmap = b.rows ? (int32_t*)((char*)ctrs + b_ctr) : nullptr;
   for (int v = 0; v < n; ++v) b.vols[v].sz = dsizes + 4 * v;
   // pinned host side: descriptors | sizes
   if (c->hbatch_bytes < b_vols + b_sizes) {
@@ -923,14 +981,23 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess && n > 0)
       e = hipMemcpyAsync(dvols, c->hbatch, sizeof(VolArgs) * (size_t)n, hipMemcpyHostToDevice,
                          c->stream);
-    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, c->stream);
+    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, c->stream);
     if (e == hipSuccess) e = launch_coords_batch(dvols, n, c->stream);
-    if (e == hipSuccess) e = launch_zero_u32(ctrs, (int64_t)(8 * b.counts.size()), c->stream);
+    if (e == hipSuccess && !b.rows)
+      e = launch_zero_u32(ctrs, (int64_t)(8 * b.counts.size()), c->stream);
+    for (const Launch& L : b.bits)
+      if (e == hipSuccess)
+        e = launch_rows_bits_batch(L.plan.T, RowsBatch{dvols, bmap, L.gbase, L.nblocks}, c->stream);
     Spread sp{c};
     if (e == hipSuccess) e = sp.start((int)b.counts.size());
     for (size_t k : by_cost(b.counts)) {
       if (e != hipSuccess) break;
-      e = launch_count_batch(b.counts[k].plan, dvols, cmap, b.counts[k].gbase,
+      if (b.rows)
+        e = launch_rows_count_batch(b.counts[k].plan.method,
+                                    RowsBatch{dvols, cmap, b.counts[k].gbase, b.counts[k].nblocks},
+                                    sp.next(b.counts[k].cost));
+      else
+        e = launch_count_batch(b.counts[k].plan, dvols, cmap, b.counts[k].gbase,
                              b.counts[k].nblocks, ctrs + 8 * k, sp.next(b.counts[k].cost));
     }
     const hipError_t ej = sp.finish();
@@ -969,6 +1036,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   b.ncoords = ncoords;
   b.cblocks = cblocks;
   b.eblocks = eblocks;
+  b.bblocks = bblocks;
   b.have = true;
   return MSH_OK;
 }
@@ -1028,7 +1096,8 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
     hipError_t e = hipMemcpyAsync(dvols, c->hbatch, sizeof(VolArgs) * (size_t)n,
                                   hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipEventRecord(c->upload, c->stream);
-    if (e == hipSuccess) e = launch_zero_u32(ectr, (int64_t)(8 * b.emits.size()), c->stream);
+    if (e == hipSuccess && !b.rows)
+      e = launch_zero_u32(ectr, (int64_t)(8 * b.emits.size()), c->stream);
     Spread sp{c};
     if (e == hipSuccess) e = sp.start((int)b.emits.size());
     for (size_t k : by_cost(b.emits)) {
@@ -1195,7 +1264,7 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
       for (size_t i = 0; i < m && takes; ++i) {
         Plan q = c->batch.plans[i];
         VolArgs probe = c->batch.vols[i];
-        takes = variant_family(emit_variant(q, &probe)) == fam;
+        takes = probe.bits ? fam == 2 : variant_family(emit_variant(q, &probe)) == fam;
       }
       if (!takes) continue;
       size_t total = 256;
@@ -1249,7 +1318,7 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
     if (g >= 0)
       for (int v : members[(size_t)g]) {
         VolArgs probe = c->batch.vols[v];
-        *took = *took && variant_family(emit_variant(c->batch.plans[v], &probe)) == fam;
+        *took = *took && (probe.bits ? fam == 2 : variant_family(emit_variant(c->batch.plans[v], &probe)) == fam);
       }
     if (!*took) return MSH_OK;
     size_t total = 256;
@@ -1291,6 +1360,23 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
     float cur = 0.f;
     bool took = true;
     rc = time_all(-1, 0, &cur, &took);
+    // the row kernels take a batch only as a whole: every group on them
+    if (rc == MSH_OK && !no_room && std::any_of(best.begin(), best.end(), [](int f) { return f != 2; })) {
+      auto set_all = [&](bool rows) {
+        for (size_t g = 0; g < gkey.size(); ++g)
+          c->family[gkey[g] / (3 * kSizeClasses)][(gkey[g] / kSizeClasses) % 3][gkey[g] % kSizeClasses] =
+              rows ? 2 : best[g];
+      };
+      set_all(true);
+      float ms = 0.f;
+      rc = time_all(-1, 2, &ms, &took);
+      if (rc == MSH_OK && !no_room && ms < cur) {
+        std::fill(best.begin(), best.end(), 2);
+        cur = ms;
+      } else {
+        set_all(false);
+      }
+    }
     // (with no room for the whole batch there is nothing to compare against)
     std::vector<size_t> gord(rc == MSH_OK && !no_room ? gkey.size() : 0);
     for (size_t g = 0; g < gord.size(); ++g) gord[g] = g;

@@ -97,6 +97,7 @@ struct VolArgs {
   int32_t sw, cw;          // words of a column of samples, of a row of cells
   int32_t upx;             // units of an x plane
   int32_t ue;              // units a wave emits one after another
+  int64_t bntiles, bblk0;  // sample-bit tiles in a batched launch, its first block there
   uint32_t cwm, cwn;       // 2^32 / cw and 2^16 / cw, rounded down and up (word_pos)
   int32_t nti, ntj;        // emit tiles along x and y
   int64_t ntiles;          // emit tiles
@@ -169,12 +170,30 @@ bool rows_geom(const Plan& p, Geom* g, RowsGeom* r);
 size_t rows_bytes(const Geom& g, const RowsGeom& r);
 size_t rows_prefix_bytes(const Plan& p, const Geom& g);  // .. of VolArgs::wpre
 void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a);
-// emit tiling, once the number of vertices is known
+// emit tiling, from the number of vertices (negative: not known yet)
 void rows_emit_tiling(VolArgs* a, int64_t nverts);
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st);
-hipError_t launch_rows_mc(const Plan& p, const VolArgs& a, hipStream_t st);
-hipError_t launch_rows_sn(const Plan& p, const VolArgs& a, hipStream_t st);
-hipError_t launch_rows_mt(const Plan& p, const VolArgs& a, hipStream_t st);
+// A batched launch: tiles gbase .. gbase + nblocks of the batch, whose volumes
+// the map names.
+struct RowsBatch {
+  const VolArgs* vols;
+  const int32_t* map;
+  int64_t gbase, nblocks;
+};
+// axis types: 1 all Float64, 2 all Float32, 0 mixed
+inline int cx_class(const VolArgs& a) { return a.cxmask == 0 ? 1 : a.cxmask == 7 ? 2 : 0; }
+hipError_t launch_rows_mc(const Plan& p, int cxclass, const VolArgs& a, const RowsBatch* b,
+                          hipStream_t st);
+hipError_t launch_rows_sn(const Plan& p, int cxclass, const VolArgs& a, const RowsBatch* b,
+                          hipStream_t st);
+hipError_t launch_rows_mt(const Plan& p, int cxclass, const VolArgs& a, const RowsBatch* b,
+                          hipStream_t st);
+hipError_t launch_rows_emit(const Plan& p, int cxclass, const VolArgs& a, const RowsBatch* b,
+                            hipStream_t st);
+hipError_t launch_rows_bits_batch(int T, const RowsBatch& b, hipStream_t st);
+hipError_t launch_rows_count_batch(int method, const RowsBatch& b, hipStream_t st);
+// variant (emit_variant) of a volume of the row kernels in a batch
+constexpr int kRowsVariant = 256;  // + cx_class
 
 hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream_t st);
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st);
@@ -199,7 +218,8 @@ hipError_t launch_emit(const Plan& p, const VolArgs& a, hipStream_t st);
 // Plan types and emit variant); gbase is the launch's first block in the
 // block->volume maps.
 hipError_t launch_coords_batch(const VolArgs* vols, int n, hipStream_t st);
-hipError_t launch_fill_maps(const VolArgs* vols, int n, int32_t* cmap, int32_t* emap,
+// (bmap: sample-bit tiles of the row kernels, or null)
+hipError_t launch_fill_maps(const VolArgs* vols, int n, int32_t* cmap, int32_t* emap, int32_t* bmap,
                             hipStream_t st);
 // Persistent count and emit launches (families 2 and 3) take their tiles
 // from 8 work-queue counters at ctr, which must be zero at launch.

@@ -76,11 +76,13 @@ __global__ void k_coords_b(const VolArgs* __restrict__ vols) {
 
 // Block -> volume maps of a batch: one block per volume fills its ranges.
 __global__ void k_fill_maps(const VolArgs* __restrict__ vols, int32_t* __restrict__ cmap,
-                            int32_t* __restrict__ emap) {
+                            int32_t* __restrict__ emap, int32_t* __restrict__ bmap) {
   const int v = blockIdx.x;
   const VolArgs& a = vols[v];
   for (int64_t i = threadIdx.x; i < a.cntiles; i += blockDim.x) cmap[a.cblk0 + i] = v;
   for (int64_t i = threadIdx.x; i < a.ntiles; i += blockDim.x) emap[a.eblk0 + i] = v;
+  if (bmap)
+    for (int64_t i = threadIdx.x; i < a.bntiles; i += blockDim.x) bmap[a.bblk0 + i] = v;
 }
 
 // Per-volume sizes of a batch from the scan over all volumes' units (volume
@@ -1027,10 +1029,7 @@ static hipError_t emit_any(const Plan& p, int variant, const VolArgs& a, const V
 
 hipError_t launch_emit(const Plan& p, const VolArgs& a0, hipStream_t st) {
   VolArgs a = a0;
-  if (a.bits)
-    return p.method == MC   ? launch_rows_mc(p, a, st)
-           : p.method == MT ? launch_rows_mt(p, a, st)
-                            : launch_rows_sn(p, a, st);
+  if (a.bits) return launch_rows_emit(p, cx_class(a), a, nullptr, st);
   const int variant = emit_variant(p, &a);
   return emit_any(p, variant, a, nullptr, nullptr, 0, 0, nullptr, st);
 }
@@ -1041,10 +1040,10 @@ hipError_t launch_coords_batch(const VolArgs* vols, int n, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_fill_maps(const VolArgs* vols, int n, int32_t* cmap, int32_t* emap,
+hipError_t launch_fill_maps(const VolArgs* vols, int n, int32_t* cmap, int32_t* emap, int32_t* bmap,
                             hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_maps, dim3((unsigned)n), dim3(256), 0, st, vols, cmap, emap);
+  hipLaunchKernelGGL(k_fill_maps, dim3((unsigned)n), dim3(256), 0, st, vols, cmap, emap, bmap);
   return hipGetLastError();
 }
 
@@ -1094,6 +1093,10 @@ hipError_t launch_sizes_batch(const VolArgs* vols, int n, const Workspace& w, in
 hipError_t launch_emit_batch(const Plan& p, int variant, const VolArgs* vols,
                              const int32_t* emap, int64_t gbase, int64_t nblocks, uint32_t* ctr,
                              hipStream_t st) {
+  if (variant >= kRowsVariant) {
+    const RowsBatch b{vols, emap, gbase, nblocks};
+    return launch_rows_emit(p, variant - kRowsVariant, VolArgs{}, &b, st);
+  }
   return emit_any(p, variant, VolArgs{}, vols, emap, gbase, nblocks, ctr, st);
 }
 

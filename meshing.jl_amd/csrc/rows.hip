@@ -84,6 +84,15 @@ __global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
   bits_tile<T, PW, E>(a, blockIdx.x);
 }
 
+// Batched: a block per tile of the launch; the map names its volume.
+template <typename T, int PW, int E>
+__global__ __launch_bounds__(kBlock) void k_bits_b(const VolArgs* __restrict__ vols,
+                                                   const int32_t* __restrict__ bmap, int64_t gbase) {
+  const int64_t b = gbase + blockIdx.x;
+  const VolArgs a = vols[__builtin_amdgcn_readfirstlane(bmap[b])];
+  bits_tile<T, PW, E>(a, b - a.bblk0);
+}
+
 // ---------------------------------------------------------------------------
 // Counts, from the bits alone.  A wave counts kCountUnits units one after
 // another.  Marching Cubes: a cell's vertices are its crossing edges, 12
@@ -92,6 +101,7 @@ __global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
 // unless a face of it is ambiguous (its corners alternate around the level)
 // or two opposite corners are cut off by themselves: those few cells, found
 // by ANDs of the same words, take their further loops from the table.
+constexpr int kBatchPW = 8;
 constexpr int kCountUnits = 2;
 constexpr int kCountTile = kCountUnits * kWaves;
 
@@ -206,17 +216,33 @@ __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, con
   }
 }
 
+// Marching Cubes: twice the loops of a case beyond its first
 template <int METHOD>
-__global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a) {
-  // Marching Cubes: twice the loops of a case beyond its first
-  __shared__ uint8_t extra[256];
+__device__ __forceinline__ void count_table(uint8_t* extra) {
   if constexpr (METHOD == MC) {
     const uint32_t m = nat_to_mc(threadIdx.x);
     const int v = (int)(MC_CASE_VERTS[m] & 0xF), f = (int)(MC_CASE_TRIS[m] & 7);
     extra[threadIdx.x] = (uint8_t)(v > 0 ? v - f - 2 : 0);
     __syncthreads();
   }
+}
+
+template <int METHOD>
+__global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a) {
+  __shared__ uint8_t extra[256];
+  count_table<METHOD>(extra);
   rows_count_tile<METHOD>(a, blockIdx.x, extra);
+}
+
+template <int METHOD>
+__global__ __launch_bounds__(kBlock) void k_rows_count_b(const VolArgs* __restrict__ vols,
+                                                         const int32_t* __restrict__ cmap,
+                                                         int64_t gbase) {
+  __shared__ uint8_t extra[256];
+  count_table<METHOD>(extra);
+  const int64_t b = gbase + blockIdx.x;
+  const VolArgs a = vols[__builtin_amdgcn_readfirstlane(cmap[b])];
+  rows_count_tile<METHOD>(a, b - a.cblk0, extra);
 }
 
 }  // namespace
@@ -261,6 +287,9 @@ void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a) {
   a->cwm = (uint32_t)std::min<uint64_t>((1ull << 32) / (uint64_t)r.cw, 0xFFFFFFFFull);
   a->cwn = (65536u + (uint32_t)r.cw - 1u) / (uint32_t)r.cw;
   a->cntiles = (a->g.units + kCountTile - 1) / kCountTile;
+  // (a batch's tiles are those of a small volume: its volumes fill the device)
+  a->bntiles = (int64_t)((a->g.nx + 2 * kWave - 1) / (2 * kWave)) *
+               (((int64_t)a->g.ny * a->sw + kBatchPW - 1) / kBatchPW);
 }
 
 // Units a wave emits one after another: one where a unit alone has cells
@@ -268,12 +297,13 @@ void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a) {
 // would each pay the way to the first sample for a few cells (1024^3 Float32
 // sphere, 12 vertices a unit: 8 units 158 us, 1 unit 349 us; 1024^3 Float64
 // value noise, 520 vertices a unit: 1 unit 5.4 ms, 8 units 6.0 ms), as long
-// as the blocks fill the device.
+// as the blocks fill the device.  One where the vertices are not known yet
+// (a batch lays its tiles out before it counts): nverts < 0.
 void rows_emit_tiling(VolArgs* a, int64_t nverts) {
   const int64_t nxb = (a->g.nx - 1 + kWaves - 1) / kWaves;
   const int64_t full = a->method == MC ? 256 : 64;  // about 64 cells
   a->ue = 1;
-  while (a->ue < kMaxUE && nverts * 2 * a->ue <= full * a->g.units &&
+  while (nverts >= 0 && a->ue < kMaxUE && nverts * 2 * a->ue <= full * a->g.units &&
          nxb * ((a->upx + 2 * a->ue - 1) / (2 * a->ue)) >= 8192)
     a->ue *= 2;
   a->ntiles = nxb * ((a->upx + a->ue - 1) / a->ue);
@@ -308,6 +338,28 @@ hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st) {
   const auto k = p.method == MC ? k_rows_count<MC> : p.method == MT ? k_rows_count<MT> : k_rows_count<SN>;
   hipLaunchKernelGGL(k, dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a);
   return hipGetLastError();
+}
+
+hipError_t launch_rows_bits_batch(int T, const RowsBatch& b, hipStream_t st) {
+  const dim3 grid((unsigned)b.nblocks);
+  if (T == K_F32)
+    hipLaunchKernelGGL((k_bits_b<float, kBatchPW, 2>), grid, dim3(kBlock), 0, st, b.vols, b.map, b.gbase);
+  else
+    hipLaunchKernelGGL((k_bits_b<double, kBatchPW, 2>), grid, dim3(kBlock), 0, st, b.vols, b.map, b.gbase);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_count_batch(int method, const RowsBatch& b, hipStream_t st) {
+  const auto k = method == MC ? k_rows_count_b<MC> : method == MT ? k_rows_count_b<MT> : k_rows_count_b<SN>;
+  hipLaunchKernelGGL(k, dim3((unsigned)b.nblocks), dim3(kBlock), 0, st, b.vols, b.map, b.gbase);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_emit(const Plan& p, int cxclass, const VolArgs& a, const RowsBatch* b,
+                            hipStream_t st) {
+  if (p.method == MC) return launch_rows_mc(p, cxclass, a, b, st);
+  if (p.method == MT) return launch_rows_mt(p, cxclass, a, b, st);
+  return launch_rows_sn(p, cxclass, a, b, st);
 }
 
 }  // namespace msh

@@ -286,29 +286,46 @@ __global__ __launch_bounds__(kBlock) void k_rows_sn(VolArgs a) {
   rows_sn_tile<T, M, Out, CXM>(a, rows_block_tile(blockIdx.x, a.ntiles));
 }
 
+// Batched: a block per tile of the launch; the map names its volume.
+template <typename T, typename M, typename Out, int CXM>
+__global__ __launch_bounds__(kBlock) void k_rows_sn_b(const VolArgs* __restrict__ vols,
+                                                  const int32_t* __restrict__ emap, int64_t gbase) {
+  const int64_t b = gbase + rows_block_tile(blockIdx.x, gridDim.x);
+  const VolArgs a = vols[__builtin_amdgcn_readfirstlane(emap[b])];
+  rows_sn_tile<T, M, Out, CXM>(a, b - a.eblk0);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
 // Host side.
 
-template <typename T, typename M, typename Out>
-static hipError_t rows_sn_t(const VolArgs& a, hipStream_t st) {
-  const dim3 grid((unsigned)a.ntiles);
-  if (a.cxmask == 0)
-    hipLaunchKernelGGL((k_rows_sn<T, M, Out, 0>), grid, dim3(kBlock), 0, st, a);
-  else if (a.cxmask == 7)
-    hipLaunchKernelGGL((k_rows_sn<T, M, Out, 7>), grid, dim3(kBlock), 0, st, a);
+template <typename T, typename M, typename Out, int CXM>
+static hipError_t rows_sn_cx(const VolArgs& a, const RowsBatch* b, hipStream_t st) {
+  if (b)
+    hipLaunchKernelGGL((k_rows_sn_b<T, M, Out, CXM>), dim3((unsigned)b->nblocks), dim3(kBlock), 0, st, b->vols,
+                       b->map, b->gbase);
   else
-    hipLaunchKernelGGL((k_rows_sn<T, M, Out, -1>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_rows_sn<T, M, Out, CXM>), dim3((unsigned)a.ntiles), dim3(kBlock), 0, st, a);
   return hipGetLastError();
 }
 
-hipError_t launch_rows_sn(const Plan& p, const VolArgs& a, hipStream_t st) {
-  if (a.ntiles == 0) return hipSuccess;
-  if (p.T == K_F32 && p.M == K_F32 && p.Out == K_F32) return rows_sn_t<float, float, float>(a, st);
-  if (p.T == K_F32 && p.M == K_F32) return rows_sn_t<float, float, double>(a, st);
-  if (p.T == K_F32) return rows_sn_t<float, double, double>(a, st);
-  return rows_sn_t<double, double, double>(a, st);
+template <typename T, typename M, typename Out>
+static hipError_t rows_sn_t(int cxclass, const VolArgs& a, const RowsBatch* b, hipStream_t st) {
+  switch (cxclass) {
+    case 1: return rows_sn_cx<T, M, Out, 0>(a, b, st);
+    case 2: return rows_sn_cx<T, M, Out, 7>(a, b, st);
+    default: return rows_sn_cx<T, M, Out, -1>(a, b, st);
+  }
+}
+
+hipError_t launch_rows_sn(const Plan& p, int cxclass, const VolArgs& a, const RowsBatch* b,
+                          hipStream_t st) {
+  if ((b ? b->nblocks : a.ntiles) == 0) return hipSuccess;
+  if (p.T == K_F32 && p.M == K_F32 && p.Out == K_F32) return rows_sn_t<float, float, float>(cxclass, a, b, st);
+  if (p.T == K_F32 && p.M == K_F32) return rows_sn_t<float, float, double>(cxclass, a, b, st);
+  if (p.T == K_F32) return rows_sn_t<float, double, double>(cxclass, a, b, st);
+  return rows_sn_t<double, double, double>(cxclass, a, b, st);
 }
 
 }  // namespace msh

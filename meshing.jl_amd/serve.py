@@ -103,6 +103,19 @@ class FieldSpec:
         return nx * ny * nz * (4 if self.dtype == "float32" else 8)
 
 
+def _workspace_units(nx, ny, nz):
+    """Workspace of a volume's count in units of 24 bytes: one per cell row
+    for the kernels that count by rows, or the sample bits (a bit per sample,
+    rows of planes padded to 128 bytes) and 156 bytes per 64 words of cells
+    for the kernels that go by words, whichever is more."""
+    if min(nx, ny, nz) < 2:
+        return 0
+    words = -(-nz // 32)
+    plane = -(-ny * words // 32) * 32
+    groups = (nx - 1) * -(-(ny - 1) * -(-(nz - 1) // 32) // 64)
+    return max((nx - 1) * (ny - 1), -(-(4 * nx * plane + 156 * groups) // 24))
+
+
 @dataclass
 class _Req:
     field: object
@@ -189,7 +202,7 @@ class Server:
             # stream has queued so far
             ready = self.torch.cuda.Event()
             ready.record(self.torch.cuda.current_stream(field.device))
-        units = max(nx - 1, 0) * max(ny - 1, 0)
+        units = _workspace_units(nx, ny, nz)
         fut = Future()
         r = _Req(field, method, axes or ((-1, 1),) * 3, fut, time.perf_counter(), nbytes, units)
         r.extra["on_done"] = on_done
