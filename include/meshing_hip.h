@@ -174,6 +174,11 @@ int msh_set_kernel_family(void* ctx, int32_t method, int32_t dtype, int32_t fami
  * and leaves merging them to the caller; it has no welding function. */
 int msh_weld(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t nfaces,
              int64_t* faces, void* verts_out, int64_t* nunique);
+/* msh_weld with the renumbered faces written to faces_out instead (room for
+ * nfaces x 3; faces itself, or apart from it); faces outside 1..nverts are
+ * copied as they are. */
+int msh_weld_to(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t nfaces,
+                const int64_t* faces, int64_t* faces_out, void* verts_out, int64_t* nunique);
 
 /* Synthetic fields, generated on the device into a column-major buffer of
  * nx*ny*nz elements of `dtype`.  kind: 0 sphere sqrt(x^2+y^2+z^2)-p0 on

@@ -450,28 +450,30 @@ def weld(vertices, faces, device=0):
         if not (_is_device_tensor(vertices) and _is_device_tensor(faces)):
             raise TypeError("weld takes CUDA tensors or numpy arrays")
         V = vertices.contiguous()
-        F = faces.to(torch.int64).contiguous().clone()  # renumbered in place
+        F = faces.to(torch.int64).contiguous()
     if V.ndim != 2 or V.shape[1] != 3 or F.ndim != 2 or F.shape[1] != 3:
         raise ValueError("vertices and faces must be (n, 3) arrays")
     if V.dtype not in (torch.float32, torch.float64):
         raise TypeError("vertex coordinates must be Float32 or Float64")
     kind = MSH_FLOAT32 if V.dtype == torch.float32 else MSH_FLOAT64
     out = torch.empty_like(V)
+    G = torch.empty_like(F)
     n = ctypes.c_int64()
     ctx = context(V.device.index)
     L = _capi.lib()
     with ctx.lock:
         ctx.check(L.msh_set_stream(
             ctx.handle, ctypes.c_void_p(torch.cuda.current_stream(V.device).cuda_stream)))
-        ctx.check(L.msh_weld(ctx.handle, kind, V.shape[0],
-                             ctypes.c_void_p(V.data_ptr() if V.numel() else None), F.shape[0],
-                             ctypes.c_void_p(F.data_ptr() if F.numel() else None),
-                             ctypes.c_void_p(out.data_ptr() if out.numel() else None),
-                             ctypes.byref(n)))
+        ctx.check(L.msh_weld_to(ctx.handle, kind, V.shape[0],
+                                ctypes.c_void_p(V.data_ptr() if V.numel() else None), F.shape[0],
+                                ctypes.c_void_p(F.data_ptr() if F.numel() else None),
+                                ctypes.c_void_p(G.data_ptr() if G.numel() else None),
+                                ctypes.c_void_p(out.data_ptr() if out.numel() else None),
+                                ctypes.byref(n)))
     out = out[:n.value].clone()
     if host:
-        return out.cpu().numpy(), F.cpu().numpy()
-    return out, F
+        return out.cpu().numpy(), G.cpu().numpy()
+    return out, G
 
 
 from .io import NrrdInfo, read_nrrd, read_ply, write_nrrd, write_ply  # noqa: E402

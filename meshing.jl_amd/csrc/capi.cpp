@@ -1412,13 +1412,18 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
 
 int msh_weld(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t nfaces,
              int64_t* faces, void* verts_out, int64_t* nunique) {
+  return msh_weld_to(ctx, kind, nverts, verts, nfaces, faces, faces, verts_out, nunique);
+}
+
+int msh_weld_to(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t nfaces,
+                const int64_t* faces, int64_t* faces_out, void* verts_out, int64_t* nunique) {
   Ctx* c = (Ctx*)ctx;
   if (!c) return MSH_ERR_ARGUMENT;
   if (kind != K_F32 && kind != K_F64)
     return fail(c, MSH_ERR_UNSUPPORTED, "vertex coordinates must be Float32 or Float64");
   if (nverts < 0 || nfaces < 0) return fail(c, MSH_ERR_ARGUMENT, "negative size");
   if (!nunique) return fail(c, MSH_ERR_ARGUMENT, "null nunique");
-  if ((nverts > 0 && (!verts || !verts_out)) || (nfaces > 0 && !faces))
+  if ((nverts > 0 && (!verts || !verts_out)) || (nfaces > 0 && (!faces || !faces_out)))
     return fail(c, MSH_ERR_ARGUMENT, "null buffer");
   const size_t vbytes = (size_t)nverts * 3 * (kind == K_F32 ? 4 : 8);
   if (nverts > 0 && (const char*)verts_out < (const char*)verts + vbytes &&
@@ -1428,25 +1433,30 @@ int msh_weld(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t
   if (nverts > ((int64_t)3 << 30) || nfaces > (int64_t)1 << 40)
     return fail(c, MSH_ERR_ARGUMENT, "mesh too large (at most 3 * 2^30 vertices)");
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, MSH_ERR_DEVICE, "hipSetDevice");
-  // workspace: flags | prefixes | first appearances | tiles | sizes | region bounds | hash table
+  // workspace: new indices | first appearances | slots | local first
+  // appearances | tiles | sizes | region bounds | hash table
   int64_t nslots = 1;
   while (nslots < nverts + nverts / 4 + 1) nslots <<= 1;
   const int64_t U = nverts > 0 ? nverts : 1;
   const int64_t T = (U + 4095) / 4096;
-  const size_t b_flag = align256((size_t)U * 4), b_i64 = align256((size_t)U * 8);
+  const size_t isz = weld_index_bytes(nverts);
+  const size_t b_idx = align256((size_t)U * isz), b_slot = align256((size_t)U * 4);
+  const size_t b_lrep = align256((size_t)U * 2);
   const size_t b_tcnt = align256((size_t)(T + 1) * 4), b_toff = align256((size_t)T * 8);
-  const size_t b_tot = 256, b_bnd = 512, b_table = align256((size_t)nslots * 8);
-  const size_t need = b_flag + 2 * b_i64 + b_tcnt + b_toff + b_tot + b_bnd + b_table;
+  const size_t b_tot = 256, b_bnd = 512, b_table = align256((size_t)nslots * isz);
+  const size_t need = 2 * b_idx + b_slot + b_lrep + b_tcnt + b_toff + b_tot + b_bnd + b_table;
   int rc = grow(c, &c->wws, &c->wws_bytes, need, "weld workspace allocation");
   if (rc) return rc;
   WeldArgs a{};
   char* q = (char*)c->wws;
-  a.flag = (uint32_t*)q;
-  q += b_flag;
-  a.pos = (int64_t*)q;
-  q += b_i64;
-  a.rep = (int64_t*)q;
-  q += b_i64;
+  a.pos = q;
+  q += b_idx;
+  a.rep = q;
+  q += b_idx;
+  a.slot = (uint32_t*)q;
+  q += b_slot;
+  a.lrep = (uint16_t*)q;
+  q += b_lrep;
   a.tilecnt = (uint32_t*)q;
   q += b_tcnt;
   a.tileoff = (int64_t*)q;
@@ -1464,6 +1474,7 @@ int msh_weld(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t
   a.verts = verts;
   a.verts_out = verts_out;
   a.faces = faces;
+  a.faces_out = faces_out;
   a.nslots = nslots;
   hipError_t e = launch_weld(a, c->stream);
   if (e == hipSuccess)

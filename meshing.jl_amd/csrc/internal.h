@@ -238,18 +238,22 @@ struct WeldArgs {
   int64_t nverts, nfaces;
   const void* verts;     // nverts x 3
   void* verts_out;       // welded vertices, room for nverts x 3
-  int64_t* faces;        // nfaces x 3, 1-based, renumbered in place
-  int64_t* table;        // hash slots: a power of two >= 1.25 nverts
+  const int64_t* faces;  // nfaces x 3, 1-based
+  int64_t* faces_out;    // renumbered (may be faces itself)
+  int64_t* table;        // hash slots: a power of two >= 1.25 nverts, weld_index_bytes each
   int64_t nslots;
   uint64_t* bounds;      // room for 63 x-region bounds of a large table
-  int64_t* rep;          // nverts: index of the vertex's first appearance
-  uint32_t* flag;        // nverts: 1 at first appearances
-  int64_t* pos;          // nverts: exclusive prefix of flag
-  uint32_t* tilecnt;     // per 4096 vertices: flags (room rounded up to 8 bytes)
+  void* rep;             // nverts indices: the vertex's first appearance
+  void* pos;             // nverts indices: new index, at first appearances
+  uint32_t* slot;        // nverts: table slot, at local first appearances
+  uint16_t* lrep;        // nverts: local first appearance
+  uint32_t* tilecnt;     // per 4096 vertices: first appearances (room rounded up to 8 bytes)
   int64_t* tileoff;      // per 4096 vertices: exclusive prefix of tilecnt
   int64_t* total;        // welded count
   int64_t* bad;          // count of face indices outside 1..nverts
 };
+// bytes of a vertex index in the weld's workspace
+size_t weld_index_bytes(int64_t nverts);
 hipError_t launch_weld(const WeldArgs& a, hipStream_t st);
 
 hipError_t launch_generate(int kind, int dtype, int64_t nx, int64_t ny, int64_t nz,

@@ -19,16 +19,21 @@
 //                   showed), so every slot ends holding the first appearance
 //                   of its key; each vertex notes its slot
 //   k_weld_rep      per vertex: its key's first appearance (one table load
-//                   per local key); flag = first itself; per tile of 4096
-//                   vertices: its count of flags
+//                   per local key); per tile of 4096 vertices: its count of
+//                   first appearances
 //   k_weld_tiles    one block: exclusive prefix of the tile counts, total =
 //                   welded count
-//   k_weld_pos      exclusive prefix of the flags = new index of each first
-//                   appearance (reduce-then-scan: no block waits on another)
-//   k_weld_compact  first appearances to their new slots
-//   k_weld_faces    face indices renumbered in place to the new index of
-//                   their vertex's first appearance (out-of-range indices
-//                   are counted and left as they are)
+//   k_weld_pos      exclusive prefix of the first appearances = their new
+//                   index (reduce-then-scan: no block waits on another), and
+//                   the first appearances themselves to their new slots
+//   k_weld_faces    face indices renumbered to the new index of their
+//                   vertex's first appearance (out-of-range indices are
+//                   counted and left as they are)
+//
+// The vertex indices in the table, the first appearances and the new indices
+// are 32-bit (I = uint32_t) for meshes of up to 2^31 vertices: every pass
+// moves half the bytes of these, and a line of the table holds twice the slots.
+// @@MEASURED@@
 //
 // A key's home slot in a large table is its x region's block of slots plus
 // the hash's low bits inside it.  Vertices of a mesh are emitted cell by
@@ -72,6 +77,18 @@ __device__ __forceinline__ uint64_t key_hash(W x, W y, W z) {
 __global__ void k_fill_i64(int64_t* __restrict__ p, int64_t n, int64_t v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
+}
+
+// Atomics on table slots (an empty slot holds all ones).
+__device__ __forceinline__ uint32_t slot_cas(uint32_t* p, uint32_t want, uint32_t v) {
+  return atomicCAS(p, want, v);
+}
+__device__ __forceinline__ uint64_t slot_cas(uint64_t* p, uint64_t want, uint64_t v) {
+  return atomicCAS((unsigned long long*)p, (unsigned long long)want, (unsigned long long)v);
+}
+__device__ __forceinline__ void slot_min(uint32_t* p, uint32_t v) { atomicMin(p, v); }
+__device__ __forceinline__ void slot_min(uint64_t* p, uint64_t v) {
+  atomicMin((unsigned long long*)p, (unsigned long long)v);
 }
 
 // An IEEE bit pattern as an unsigned integer whose order is the numeric
@@ -143,23 +160,23 @@ __device__ __forceinline__ uint64_t home_slot(W x, uint64_t h, const uint64_t* b
 
 // Global insert of vertex i with key (x, y, z), probing from slot h:
 // returns its slot.
-template <typename W>
-__device__ __forceinline__ uint32_t global_insert(const W* __restrict__ v, int64_t i, W x, W y,
-                                                  W z, uint64_t h, unsigned long long* table,
-                                                  uint64_t mask) {
+template <typename W, typename I>
+__device__ __forceinline__ uint32_t global_insert(const W* __restrict__ v, I i, W x, W y, W z,
+                                                  uint64_t h, I* table, uint64_t mask) {
+  constexpr I kFree = (I)~(I)0;
   while (true) {
     // a plain load first: a CAS on a taken slot measured slower
-    unsigned long long cur = __hip_atomic_load(&table[h], __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-    if (cur == ~0ull) {
-      cur = atomicCAS(&table[h], ~0ull, (unsigned long long)i);
-      if (cur == ~0ull) break;  // claimed
+    I cur = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (cur == kFree) {
+      cur = slot_cas(&table[h], kFree, i);
+      if (cur == kFree) break;  // claimed
     }
     // every index a slot ever holds has the slot's key, so this compare
     // does not depend on which of them it reads
-    if (v[3 * cur] == x && v[3 * cur + 1] == y && v[3 * cur + 2] == z) {
+    const W* k = v + 3 * (int64_t)cur;
+    if (k[0] == x && k[1] == y && k[2] == z) {
       // a slot only ever decreases: above what it showed, i cannot lower it
-      if ((unsigned long long)i < cur) atomicMin(&table[h], (unsigned long long)i);
+      if (i < cur) slot_min(&table[h], i);
       break;
     }
     h = (h + 1) & mask;
@@ -176,10 +193,9 @@ constexpr int kWeldLS = 2 * kWeldLT;   // local hash slots
 // the first appearance of each local key to the global table; each vertex
 // notes that local first appearance, whose slot k_weld_rep reads once for
 // all of them.
-template <typename W>
+template <typename W, typename I>
 __global__ __launch_bounds__(kBlock) void k_weld_insert(const W* __restrict__ v, int64_t nv,
-                                                        unsigned long long* table,
-                                                        uint64_t mask,
+                                                        I* table, uint64_t mask,
                                                         const uint64_t* __restrict__ bounds,
                                                         int nreg, int rbits,
                                                         uint32_t* __restrict__ slot,
@@ -227,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_weld_insert(const W* __restrict__ v,
     if (l == (uint32_t)j) {
       const W x = key[3 * j], y = key[3 * j + 1], z = key[3 * j + 2];
       const uint64_t h = home_slot(x, key_hash(x, y, z), bnd, nreg, rbits);
-      slot[base + j] = global_insert(v, base + j, x, y, z, h, table, mask);
+      slot[base + j] = global_insert<W, I>(v, (I)(base + j), x, y, z, h, table, mask);
     }
   }
 }
@@ -239,21 +255,25 @@ static_assert(kWeldLT % kBlock == 0 && kWeldTile % kWeldLT == 0 && kWeldLT <= 65
 
 // Same windows as k_weld_insert: the local first appearances read their
 // key's smallest index from the table, the others take it from them.
-__global__ __launch_bounds__(kBlock) void k_weld_rep(int64_t nv,
-                                                     const int64_t* __restrict__ table,
+template <typename I>
+__global__ __launch_bounds__(kBlock) void k_weld_rep(int64_t nv, const I* __restrict__ table,
                                                      const uint32_t* __restrict__ slot,
                                                      const uint16_t* __restrict__ lrep,
-                                                     int64_t* __restrict__ rep,
-                                                     uint32_t* __restrict__ flag,
+                                                     I* __restrict__ rep,
                                                      uint32_t* __restrict__ tilecnt) {
-  __shared__ int64_t res[kWeldLT];
+  __shared__ I res[kWeldLT];
   constexpr int PER = kWeldLT / kBlock;
   const int64_t base = (int64_t)blockIdx.x * kWeldLT;
   const int n = nv - base < kWeldLT ? (int)(nv - base) : kWeldLT;
+  uint16_t l[PER];
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
     const int j = threadIdx.x + q * kBlock;
-    if (j < n && lrep[base + j] == j) res[j] = table[slot[base + j]];
+    l[q] = 0;
+    if (j < n) {
+      l[q] = lrep[base + j];
+      if (l[q] == j) res[j] = table[slot[base + j]];
+    }
   }
   __syncthreads();
 #pragma unroll
@@ -262,10 +282,9 @@ __global__ __launch_bounds__(kBlock) void k_weld_rep(int64_t nv,
     const int64_t i = base + j;
     bool first = false;
     if (j < n) {
-      const int64_t r = res[lrep[i]];  // the smallest index of i's key
+      const I r = res[l[q]];  // the smallest index of i's key
       rep[i] = r;
-      first = r == i;
-      flag[i] = first ? 1u : 0u;
+      first = r == (I)i;
     }
     // a wave's 64 vertices here are consecutive and lie in one tile
     const uint64_t b = __ballot(first);
@@ -273,7 +292,7 @@ __global__ __launch_bounds__(kBlock) void k_weld_rep(int64_t nv,
   }
 }
 
-// Exclusive prefix of the flags in three steps: the tile counts (above),
+// Exclusive prefix of the first appearances in three steps: the tile counts (above),
 // their prefix in one block (here), then each tile's own (k_weld_pos).
 __global__ __launch_bounds__(1024) void k_weld_tiles(const uint32_t* __restrict__ tilecnt,
                                                      int64_t ntiles, int64_t* __restrict__ tileoff,
@@ -298,21 +317,26 @@ __global__ __launch_bounds__(1024) void k_weld_tiles(const uint32_t* __restrict_
 }
 
 // One tile per block in kWeldPer rounds of 256 consecutive vertices, so
-// every load and store of a round is one coalesced stretch.
-__global__ __launch_bounds__(kBlock) void k_weld_pos(const uint32_t* __restrict__ flag,
-                                                     int64_t nv,
+// every load and store of a round is one coalesced stretch.  A first
+// appearance goes to its new slot as soon as that is known: a pass of its own
+// would read the vertices' new indices again.
+template <typename W, typename I>
+__global__ __launch_bounds__(kBlock) void k_weld_pos(const W* __restrict__ v,
+                                                     const I* __restrict__ rep, int64_t nv,
                                                      const int64_t* __restrict__ tileoff,
-                                                     int64_t* __restrict__ pos) {
+                                                     I* __restrict__ pos, W* __restrict__ out) {
   __shared__ uint32_t s_w[kWeldPer][kWaves];
   const int lane = lane_id(), wv = threadIdx.x / kWave;
   const int64_t base = (int64_t)blockIdx.x * kWeldTile + threadIdx.x;
-  uint32_t f[kWeldPer], incl[kWeldPer];
+  bool f[kWeldPer];
+  uint32_t below[kWeldPer];
 #pragma unroll
   for (int q = 0; q < kWeldPer; ++q) {
     const int64_t i = base + q * kBlock;
-    f[q] = i < nv ? flag[i] : 0u;
-    incl[q] = wave_scan_dpp(f[q]);
-    if (lane == kWave - 1) s_w[q][wv] = incl[q];
+    f[q] = i < nv && rep[i] == (I)i;
+    const uint64_t b = __ballot(f[q]);
+    below[q] = lanes_below(b);
+    if (lane == 0) s_w[q][wv] = (uint32_t)__popcll(b);
   }
   __syncthreads();
   int64_t run = tileoff[blockIdx.x];
@@ -325,51 +349,47 @@ __global__ __launch_bounds__(kBlock) void k_weld_pos(const uint32_t* __restrict_
       all += s_w[q][w];
     }
     const int64_t i = base + q * kBlock;
-    if (i < nv) pos[i] = run + before + incl[q] - f[q];
+    if (f[q]) {  // (only first appearances are asked for their new index)
+      const int64_t o = run + before + below[q];
+      pos[i] = (I)o;
+      out[3 * o] = v[3 * i];
+      out[3 * o + 1] = v[3 * i + 1];
+      out[3 * o + 2] = v[3 * i + 2];
+    }
     run += all;
   }
 }
 
-template <typename W>
-__global__ void k_weld_compact(const W* __restrict__ v, int64_t nv,
-                               const int64_t* __restrict__ pos,
-                               const uint32_t* __restrict__ flag, W* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nv || !flag[i]) return;
-  const int64_t o = pos[i];  // a first appearance's new index
-  out[3 * o] = v[3 * i];
-  out[3 * o + 1] = v[3 * i + 1];
-  out[3 * o + 2] = v[3 * i + 2];
-}
-
-__global__ void k_weld_faces(int64_t* __restrict__ f, int64_t n,
-                             const int64_t* __restrict__ rep, const int64_t* __restrict__ pos,
-                             int64_t nv, unsigned long long* __restrict__ bad) {
+template <typename I>
+__global__ void k_weld_faces(const int64_t* f, int64_t* out, int64_t n,  // (may be the same)
+                             const I* __restrict__ rep, const I* __restrict__ pos, int64_t nv,
+                             unsigned long long* __restrict__ bad) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  const int64_t j = f[k];
+  int64_t j = f[k];
   if (j >= 1 && j <= nv)
-    f[k] = pos[rep[j - 1]] + 1;  // the new index of the vertex's first appearance
+    j = (int64_t)pos[rep[j - 1]] + 1;  // the new index of the vertex's first appearance
   else
     atomicAdd(bad, 1ull);
+  out[k] = j;
 }
 
 unsigned grid_of(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
-template <typename W>
+template <typename W, typename I>
 hipError_t weld_t(const WeldArgs& a, hipStream_t st) {
   const W* v = (const W*)a.verts;
+  I* table = (I*)a.table;
+  I* rep = (I*)a.rep;
+  I* pos = (I*)a.pos;
   hipLaunchKernelGGL(k_fill_i64, dim3(1), dim3(kBlock), 0, st, a.bad, (int64_t)1, (int64_t)0);
   if (a.nverts > 0) {
-    hipLaunchKernelGGL(k_fill_i64, dim3(grid_of(a.nslots)), dim3(kBlock), 0, st, a.table,
-                       a.nslots, (int64_t)-1);
-    // slots (4 bytes per vertex) and local first appearances (2 bytes) live
-    // in pos until k_weld_pos overwrites it
-    uint32_t* slot = (uint32_t*)a.pos;
-    uint16_t* lrep = (uint16_t*)(slot + a.nverts);
+    // (room is whole 256 bytes: the last word may reach past the slots)
+    const int64_t words = (a.nslots * (int64_t)sizeof(I) + 7) / 8;
+    hipLaunchKernelGGL(k_fill_i64, dim3(grid_of(words)), dim3(kBlock), 0, st, a.table, words,
+                       (int64_t)-1);
     const unsigned nwin = (unsigned)((a.nverts + kWeldLT - 1) / kWeldLT);
-    // x regions only where the table outgrows the caches (2^23 slots,
-    // 64 MiB, and up)
+    // x regions only where the table outgrows the caches (2^23 slots and up)
     int lg = 0;
     while (((int64_t)1 << lg) < a.nslots) ++lg;
     const int nreg = lg >= 23 ? kWeldRegions : 1;
@@ -378,34 +398,36 @@ hipError_t weld_t(const WeldArgs& a, hipStream_t st) {
     if (nreg > 1)
       hipLaunchKernelGGL((k_weld_bounds<W>), dim3(1), dim3(kWeldSortBlock), 0, st, v, a.nverts,
                          nreg, a.bounds);
-    hipLaunchKernelGGL((k_weld_insert<W>), dim3(nwin), dim3(kBlock), 0, st, v, a.nverts,
-                       (unsigned long long*)a.table, (uint64_t)(a.nslots - 1),
-                       (const uint64_t*)a.bounds, nreg, rbits, slot, lrep);
+    hipLaunchKernelGGL((k_weld_insert<W, I>), dim3(nwin), dim3(kBlock), 0, st, v, a.nverts, table,
+                       (uint64_t)(a.nslots - 1), (const uint64_t*)a.bounds, nreg, rbits, a.slot,
+                       a.lrep);
     const int64_t ntiles = (a.nverts + kWeldTile - 1) / kWeldTile;
     hipLaunchKernelGGL(k_fill_i64, dim3(grid_of((ntiles + 1) / 2)), dim3(kBlock), 0, st,
                        (int64_t*)a.tilecnt, (ntiles + 1) / 2, (int64_t)0);
-    hipLaunchKernelGGL(k_weld_rep, dim3(nwin), dim3(kBlock), 0, st, a.nverts,
-                       (const int64_t*)a.table, (const uint32_t*)slot, (const uint16_t*)lrep,
-                       a.rep, a.flag, a.tilecnt);
+    hipLaunchKernelGGL((k_weld_rep<I>), dim3(nwin), dim3(kBlock), 0, st, a.nverts,
+                       (const I*)table, (const uint32_t*)a.slot, (const uint16_t*)a.lrep, rep,
+                       a.tilecnt);
     hipLaunchKernelGGL(k_weld_tiles, dim3(1), dim3(1024), 0, st, (const uint32_t*)a.tilecnt,
                        ntiles, a.tileoff, a.total);
-    hipLaunchKernelGGL(k_weld_pos, dim3((unsigned)ntiles), dim3(kBlock), 0, st,
-                       (const uint32_t*)a.flag, a.nverts, (const int64_t*)a.tileoff, a.pos);
-    hipLaunchKernelGGL((k_weld_compact<W>), dim3(grid_of(a.nverts)), dim3(kBlock), 0, st, v,
-                       a.nverts, (const int64_t*)a.pos, (const uint32_t*)a.flag,
-                       (W*)a.verts_out);
+    hipLaunchKernelGGL((k_weld_pos<W, I>), dim3((unsigned)ntiles), dim3(kBlock), 0, st, v,
+                       (const I*)rep, a.nverts, (const int64_t*)a.tileoff, pos, (W*)a.verts_out);
   }
   if (a.nfaces > 0)
-    hipLaunchKernelGGL(k_weld_faces, dim3(grid_of(3 * a.nfaces)), dim3(kBlock), 0, st, a.faces,
-                       3 * a.nfaces, (const int64_t*)a.rep, (const int64_t*)a.pos, a.nverts,
+    hipLaunchKernelGGL((k_weld_faces<I>), dim3(grid_of(3 * a.nfaces)), dim3(kBlock), 0, st, a.faces,
+                       a.faces_out, 3 * a.nfaces, (const I*)rep, (const I*)pos, a.nverts,
                        (unsigned long long*)a.bad);
   return hipGetLastError();
 }
 
 }  // namespace
 
+size_t weld_index_bytes(int64_t nverts) { return nverts <= ((int64_t)1 << 31) ? 4 : 8; }
+
 hipError_t launch_weld(const WeldArgs& a, hipStream_t st) {
-  return a.out_kind == K_F32 ? weld_t<uint32_t>(a, st) : weld_t<uint64_t>(a, st);
+  const bool narrow = weld_index_bytes(a.nverts) == 4;
+  if (a.out_kind == K_F32)
+    return narrow ? weld_t<uint32_t, uint32_t>(a, st) : weld_t<uint32_t, uint64_t>(a, st);
+  return narrow ? weld_t<uint64_t, uint32_t>(a, st) : weld_t<uint64_t, uint64_t>(a, st);
 }
 
 }  // namespace msh
