@@ -107,6 +107,7 @@ struct Ctx {
   hipStream_t aux[kSpreadWays - 1] = {};
   hipEvent_t fork = nullptr, join[kSpreadWays - 1] = {};
   int64_t* pinned = nullptr;  // 4 x int64 for the totals
+  uint32_t* done = nullptr;   // device word, zero between calls (ScanTail)
   void* scratch = nullptr;    // this device's static scratch (msh_isosurface_noalloc)
   void* wws = nullptr;        // weld: hash table, scan workspace, indices
   size_t wws_bytes = 0;
@@ -529,13 +530,17 @@ int msh_create(int device, void** out) {
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->pinned, 4 * sizeof(int64_t), hipHostMallocDefault);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->upload, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipMalloc((void**)&c->done, 256);
+  if (e == hipSuccess) e = launch_zero_u32(c->done, 64, c->own);
   // once per device, with the device current: the address of its copy of
   // the static scratch array
   if (e == hipSuccess) e = noalloc_setup(device, &c->scratch);
   if (e == hipSuccess) e = tables_setup(device, c->own);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->own);
   if (e != hipSuccess) {
     if (c->upload) (void)hipEventDestroy(c->upload);
     if (c->pinned) (void)hipHostFree(c->pinned);
+    if (c->done) (void)hipFree(c->done);
     if (c->own) (void)hipStreamDestroy(c->own);
     delete c;
     return e == hipErrorOutOfMemory ? MSH_ERR_OUT_OF_MEMORY : MSH_ERR_DEVICE;
@@ -567,6 +572,7 @@ int msh_destroy(void* ctx) {
   if (c->fork) (void)hipEventDestroy(c->fork);
   if (c->upload) (void)hipEventDestroy(c->upload);
   if (c->pinned) (void)hipHostFree(c->pinned);
+  if (c->done) (void)hipFree(c->done);
   if (c->own) (void)hipStreamDestroy(c->own);
   delete c;
   return MSH_OK;
@@ -648,13 +654,17 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
     }
     VolArgs a = make_vol(pl, g, dfield, w);
     if (bits) rows_vol(rg, bits, (char*)bits + rows_bytes(gr, rg), &a);
-    hipError_t e = launch_count(pl, a, c->stream);
+    c->pinned[1] = c->pinned[3] = -1;
+    const CoordArgs ca = coord_args(pl, g, w.coords);
+    // a volume of one scan tile is scanned by the count's last block
+    const bool tail = bits && g.units <= kScanTile;
+    hipError_t e = launch_count(
+        pl, a, c->stream,
+        tail ? ScanTail{c->done, w.voff, w.foff, w.totals, c->pinned, ca} : ScanTail{});
     // the scan also fills the coordinate tables and writes the sizes into
     // the pinned host words itself; a negative word afterwards (not
     // written) is read back by a copy
-    c->pinned[1] = c->pinned[3] = -1;
-    const CoordArgs ca = coord_args(pl, g, w.coords);
-    if (e == hipSuccess) e = launch_scan(g, w, c->stream, c->pinned, &ca);
+    if (e == hipSuccess && !tail) e = launch_scan(g, w, c->stream, c->pinned, &ca);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess && (c->pinned[1] < 0 || c->pinned[3] < 0)) {
       e = hipMemcpyAsync(c->pinned, w.totals, 4 * sizeof(int64_t), hipMemcpyDeviceToHost,

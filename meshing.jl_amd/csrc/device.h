@@ -253,6 +253,26 @@ __device__ __forceinline__ uint32_t seg_scan_dpp(uint32_t v) {
   return v;
 }
 
+// LinRange coordinates: xp[i] = CX((1-t)*a + t*b), t = (i-1)/max(1, n-1)
+// (Julia Base lerpi; used at src/marching_cubes.jl:36-38).
+__device__ __forceinline__ double lerpi(int j, int n, double a, double b, bool f32) {
+  const int d = n - 1 > 1 ? n - 1 : 1;
+  const double t = (double)j / (double)d;
+  const double v = (1.0 - t) * a + t * b;
+  return f32 ? (double)(float)v : v;
+}
+
+// coordinate i of the three axes laid end to end (x, then y, then z)
+__device__ __forceinline__ double coord_at(const CoordArgs& c, int i) {
+  int axis = 0, n = c.nx, j = i;
+  if (i >= c.nx + c.ny) {
+    axis = 2; n = c.nz; j = i - c.nx - c.ny;
+  } else if (i >= c.nx) {
+    axis = 1; n = c.ny; j = i - c.nx;
+  }
+  return lerpi(j, n, c.a[axis], c.b[axis], (c.mask >> axis) & 1);
+}
+
 // Raw buffer resource over `bytes` bytes at p (32-bit data format, so
 // loads past `bytes` return 0 instead of touching memory).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* p, uint32_t bytes) {

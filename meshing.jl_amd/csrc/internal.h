@@ -159,6 +159,15 @@ int variant_family(int variant);
 // persistent launch is kept full by the other volumes)
 void count_tiling(const Plan& p, VolArgs* a, bool split);
 
+// The LinRange coordinates of a volume's three axes, end to end, into out.
+struct CoordArgs {
+  double* out;
+  int nx, ny, nz;
+  double a[3], b[3];
+  int mask;  // bit k: axis k in Float32
+};
+CoordArgs coord_args(const Plan& p, const Geom& g, double* coords);
+
 // The row kernels (rows.h): Geom::units in their units, and the layout of
 // the sample bits; false when they do not take the volume.
 struct RowsGeom {
@@ -172,7 +181,14 @@ size_t rows_prefix_bytes(const Plan& p, const Geom& g);  // .. of VolArgs::wpre
 void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a);
 // emit tiling, from the number of vertices (negative: not known yet)
 void rows_emit_tiling(VolArgs* a, int64_t nverts);
-hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st);
+// The count's last block to finish also scans the units (one scan tile of
+// them at most) and does what launch_scan does; done null: no scan.
+struct ScanTail {
+  uint32_t* done;  // blocks that are through: zero at launch, left zero
+  int64_t *voff, *foff, *totals, *host;
+  CoordArgs coords;
+};
+hipError_t launch_rows_count(const Plan& p, const VolArgs& a, const ScanTail& tail, hipStream_t st);
 // A batched launch: tiles gbase .. gbase + nblocks of the batch, whose volumes
 // the map names.
 struct RowsBatch {
@@ -196,15 +212,9 @@ hipError_t launch_rows_count_batch(int method, const RowsBatch& b, hipStream_t s
 constexpr int kRowsVariant = 256;  // + cx_class
 
 hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream_t st);
-hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st);
-// The LinRange coordinates of a volume's three axes, end to end, into out.
-struct CoordArgs {
-  double* out;
-  int nx, ny, nz;
-  double a[3], b[3];
-  int mask;  // bit k: axis k in Float32
-};
-CoordArgs coord_args(const Plan& p, const Geom& g, double* coords);
+// (row kernels: tail as launch_rows_count; others ignore it)
+hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st,
+                        const ScanTail& tail = ScanTail{});
 // host: pinned host words that also receive the vertex and face totals
 // (at [1] and [3]), or null; coords: coordinate tables the scan also fills
 // (in its one-block tile scan, or block 0 of the fused apply) instead of a

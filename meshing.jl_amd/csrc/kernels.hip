@@ -33,27 +33,6 @@
 namespace msh {
 namespace {
 
-// ---------------------------------------------------------------------------
-// LinRange coordinates: xp[i] = CX((1-t)*a + t*b), t = (i-1)/max(1, n-1)
-// (Julia Base lerpi; used at src/marching_cubes.jl:36-38).
-__device__ __forceinline__ double lerpi(int j, int n, double a, double b, bool f32) {
-  const int d = n - 1 > 1 ? n - 1 : 1;
-  const double t = (double)j / (double)d;
-  const double v = (1.0 - t) * a + t * b;
-  return f32 ? (double)(float)v : v;
-}
-
-// coordinate i of the three axes laid end to end (x, then y, then z)
-__device__ __forceinline__ double coord_at(const CoordArgs& c, int i) {
-  int axis = 0, n = c.nx, j = i;
-  if (i >= c.nx + c.ny) {
-    axis = 2; n = c.nz; j = i - c.nx - c.ny;
-  } else if (i >= c.nx) {
-    axis = 1; n = c.ny; j = i - c.nx;
-  }
-  return lerpi(j, n, c.a[axis], c.b[axis], (c.mask >> axis) & 1);
-}
-
 __global__ void k_coords(CoordArgs c) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < c.nx + c.ny + c.nz) c.out[i] = coord_at(c, i);
@@ -949,8 +928,8 @@ VolArgs make_vol(const Plan& p, const Geom& g, const void* field, const Workspac
   return a;
 }
 
-hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st) {
-  return a.bits ? launch_rows_count(p, a, st) : launch_count4(p, a, st);
+hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st, const ScanTail& tail) {
+  return a.bits ? launch_rows_count(p, a, tail, st) : launch_count4(p, a, st);
 }
 
 template <int METHOD, typename T, typename M, typename A, typename Out, int TX, int TY>

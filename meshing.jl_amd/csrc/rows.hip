@@ -227,11 +227,74 @@ __device__ __forceinline__ void count_table(uint8_t* extra) {
   }
 }
 
+// The scan of a volume of one scan tile, by the last block to finish its
+// counts (the others' counts are visible to it: each block makes its own
+// visible to the device before it adds itself to `done`).  Small volumes are
+// launches and little else: two launches fewer, 32^3 Float32 sphere call
+// 40.5 -> 36.9 us.
+__device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
+  __shared__ bool last;
+  __shared__ uint64_t s_w[kWaves];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = atomicAdd(t.done, 1u) == gridDim.x - 1;
+    __threadfence();
+  }
+  __syncthreads();
+  if (!last) return;
+  const int units = (int)a.g.units, base = (int)threadIdx.x * kScanItems;
+  uint32_t c[kScanItems];
+  uint64_t sum = 0;  // vertices | faces << 32
+#pragma unroll
+  for (int q = 0; q < kScanItems; ++q) {
+    c[q] = base + q < units
+               ? __hip_atomic_load(&a.cnt[base + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+               : 0u;
+    sum += (uint64_t)(c[q] & 0xFFFF) | ((uint64_t)(c[q] >> 16) << 32);
+  }
+  const uint64_t incl = wave_incl_scan64(sum);
+  if (lane_id() == kWave - 1) s_w[wave_id()] = incl;
+  __syncthreads();
+  uint64_t before = 0, all = 0;
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q) {
+    before += q < wave_id() ? s_w[q] : 0ull;
+    all += s_w[q];
+  }
+  const uint64_t excl = before + incl - sum;
+  int64_t rv = (int64_t)(excl & 0xFFFFFFFFu), rf = (int64_t)(excl >> 32);
+#pragma unroll
+  for (int q = 0; q < kScanItems; ++q) {
+    if (base + q < units) {
+      t.voff[base + q] = rv;
+      t.foff[base + q] = rf;
+    }
+    rv += c[q] & 0xFFFF;
+    rf += c[q] >> 16;
+  }
+  if (threadIdx.x == 0) {
+    const int64_t nv = (int64_t)(all & 0xFFFFFFFFu), nf = (int64_t)(all >> 32);
+    t.totals[0] = 0;
+    t.totals[1] = nv;
+    t.totals[2] = 0;
+    t.totals[3] = nf;
+    *t.done = 0;
+    t.host[1] = nv;
+    t.host[3] = nf;
+    __threadfence_system();
+  }
+}
+
 template <int METHOD>
-__global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a) {
+__global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a, ScanTail tail) {
   __shared__ uint8_t extra[256];
+  if (tail.done && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < tail.coords.nx + tail.coords.ny + tail.coords.nz; i += kBlock)
+      tail.coords.out[i] = coord_at(tail.coords, i);
   count_table<METHOD>(extra);
   rows_count_tile<METHOD>(a, blockIdx.x, extra);
+  if (tail.done) scan_tail(a, tail);
 }
 
 template <int METHOD>
@@ -329,14 +392,14 @@ static void launch_bits_t(const VolArgs& a, hipStream_t st) {
     launch_bits_e<T, 8, 2>(a, st);
 }
 
-hipError_t launch_rows_count(const Plan& p, const VolArgs& a, hipStream_t st) {
+hipError_t launch_rows_count(const Plan& p, const VolArgs& a, const ScanTail& tail, hipStream_t st) {
   if (a.cntiles == 0) return hipSuccess;
   if (p.T == K_F32)
     launch_bits_t<float>(a, st);
   else
     launch_bits_t<double>(a, st);
   const auto k = p.method == MC ? k_rows_count<MC> : p.method == MT ? k_rows_count<MT> : k_rows_count<SN>;
-  hipLaunchKernelGGL(k, dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a);
+  hipLaunchKernelGGL(k, dim3((unsigned)a.cntiles), dim3(kBlock), 0, st, a, tail);
   return hipGetLastError();
 }
 

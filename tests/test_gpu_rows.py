@@ -70,3 +70,10 @@ def test_sparse_units(pkg, oracle, name):
     z = np.linspace(0, 1, 2)[None, None, :]
     f = np.asfortranarray((np.sqrt(x * x + y * y) - 0.5 + 0.001 * z).astype(np.float32))
     assert check(pkg, oracle, f, name) > 1000
+
+
+@pytest.mark.parametrize("name", ["mc", "mt", "sn"])
+@pytest.mark.parametrize("nx", [2049, 2050])  # 2048 units, scanned by the count's last block, and one more
+def test_scan_in_the_count(pkg, oracle, nx, name):
+    for seed in (1, 2):
+        assert check(pkg, oracle, noise((nx, 65, 5), seed, np.float32), name) > 1000
