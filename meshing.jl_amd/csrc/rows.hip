@@ -13,24 +13,40 @@ namespace msh {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Sample bits.  A block takes 64 * E columns along x and PW words along a
-// plane's (y, w) order; a wave makes PW / 4 of the words, each lane the words
-// of its E neighbouring columns from loads of E samples (16 at a time, all in
-// flight at once).  The words meet in LDS so that a column's PW words leave
-// together.  Every sample is read once and only once: this pass is bound by
-// HBM reads.
+// Sample bits.  A block takes 64 * E * WX columns along x and PW words along
+// a plane's (y, w) order; WX of its waves lie side by side along x, the
+// others share the words, each lane making the words of its E neighbouring
+// columns from loads of E samples (16 at a time, all in flight at once).  The
+// words meet in LDS so that a column's PW words leave together.  Every sample
+// is read once and only once: this pass is bound by HBM reads, which reach
+// 5.4 to 5.7 TB/s of the 6.8 that a linear read gets here (each load takes 256
+// or 512 bytes of a plane).  NT: non-temporal loads.
 template <typename T, int E>
 struct __attribute__((packed, aligned(sizeof(T)))) Vec {
   T v[E];
 };
 
-template <typename T, int PW, int E>
+template <typename T, int E, bool NT>
+__device__ __forceinline__ Vec<T, E> load_vec(const char* p) {
+  if constexpr (!NT) {
+    return *(const Vec<T, E>*)p;
+  } else if constexpr (E == 1) {
+    return {{__builtin_nontemporal_load((const T*)p)}};
+  } else {
+    static_assert(E == 2, "one or two samples");
+    typedef T T2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    const T2 v = __builtin_nontemporal_load((const T2*)p);
+    return {{v.x, v.y}};
+  }
+}
+
+template <typename T, int PW, int E, int WX, bool NT>
 __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
-  constexpr int PPW = PW / kWaves, X = kWave * E, ZB = 16;
+  constexpr int PPW = PW * WX / kWaves, X = kWave * E * WX, ZB = 16;
   __shared__ uint32_t words[X][PW + 1];
   const Geom g = a.g;
   const T thr = (T)a.thr;
-  const int lane = lane_id(), wv = wave_id();
+  const int lane = lane_id(), wv = wave_id() / WX, wx = wave_id() % WX;
   const uint32_t nxt = (uint32_t)(g.nx + X - 1) / X;
   const uint32_t tq = (uint32_t)t / nxt;
   const int xb = (int)((uint32_t)t - tq * nxt) * X;
@@ -38,7 +54,7 @@ __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
   const uint64_t pbytes = (uint64_t)g.nx * (uint64_t)g.ny * sizeof(T);
   // the lane's columns; at the row's end they move back to end with it (two
   // lanes then make the same words)
-  const int xl = min(xb + lane * E, g.nx - E);
+  const int xl = min(xb + (wx * kWave + lane) * E, g.nx - E);
   const uint32_t xo = (uint32_t)xl * (uint32_t)sizeof(T);
 #pragma unroll 1
   for (int p = 0; p < PPW; ++p) {
@@ -56,7 +72,7 @@ __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
         Vec<T, E> v[ZB];
 #pragma unroll
         for (int z = 0; z < ZB; ++z)
-          v[z] = *(const Vec<T, E>*)(col + (uint64_t)min(zb + z, n - 1) * pbytes + xo);
+          v[z] = load_vec<T, E, NT>(col + (uint64_t)min(zb + z, n - 1) * pbytes + xo);
 #pragma unroll
         for (int z = 0; z < ZB; ++z)
 #pragma unroll
@@ -79,9 +95,9 @@ __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
   }
 }
 
-template <typename T, int PW, int E>
+template <typename T, int PW, int E, int WX, bool NT>
 __global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
-  bits_tile<T, PW, E>(a, blockIdx.x);
+  bits_tile<T, PW, E, WX, NT>(a, blockIdx.x);
 }
 
 // Batched: a block per tile of the launch; the map names its volume.
@@ -90,7 +106,7 @@ __global__ __launch_bounds__(kBlock) void k_bits_b(const VolArgs* __restrict__ v
                                                    const int32_t* __restrict__ bmap, int64_t gbase) {
   const int64_t b = gbase + blockIdx.x;
   const VolArgs a = vols[__builtin_amdgcn_readfirstlane(bmap[b])];
-  bits_tile<T, PW, E>(a, b - a.bblk0);
+  bits_tile<T, PW, E, 1, false>(a, b - a.bblk0);
 }
 
 // ---------------------------------------------------------------------------
@@ -102,7 +118,7 @@ __global__ __launch_bounds__(kBlock) void k_bits_b(const VolArgs* __restrict__ v
 // or two opposite corners are cut off by themselves: those few cells, found
 // by ANDs of the same words, take their further loops from the table.
 constexpr int kBatchPW = 8;
-constexpr int kCountUnits = 2;
+constexpr int kCountUnits = 2;  // (1: 32^3 0.6 us faster, 1024^3 30 us slower)
 constexpr int kCountTile = kCountUnits * kWaves;
 
 __device__ __forceinline__ uint32_t mc_word_counts(const CellWord& r, const uint8_t* extra) {
@@ -372,24 +388,36 @@ void rows_emit_tiling(VolArgs* a, int64_t nverts) {
   a->ntiles = nxb * ((a->upx + a->ue - 1) / a->ue);
 }
 
-template <typename T, int PW, int E>
+template <typename T, int PW, int E, int WX, bool NT>
 static void launch_bits_e(const VolArgs& a, hipStream_t st) {
-  const int64_t nxt = (a.g.nx + kWave * E - 1) / (kWave * E), nq = (int64_t)a.g.ny * a.sw;
-  hipLaunchKernelGGL((k_bits<T, PW, E>), dim3((unsigned)(nxt * ((nq + PW - 1) / PW))), dim3(kBlock),
-                     0, st, a);
+  constexpr int X = kWave * E * WX;
+  const int64_t nxt = (a.g.nx + X - 1) / X, nq = (int64_t)a.g.ny * a.sw;
+  hipLaunchKernelGGL((k_bits<T, PW, E, WX, NT>), dim3((unsigned)(nxt * ((nq + PW - 1) / PW))),
+                     dim3(kBlock), 0, st, a);
 }
 
-// 2 columns a lane: against 1 and 4 the fastest on large volumes (1024^3
-// Float64 1.69 ms, 1.77 with 1; Float32 0.876, 0.90 and 0.888) and as fast
-// on small ones, where shorter tiles (8 words, 256 x 256 x 256 Float32 11.8
-// us) beat the longer ones (32 words, 18 us) until those fill the device.
+// A field of up to twice the last-level cache (256 MB) is read through it, so
+// that the emit finds samples there: with non-temporal loads the 256^3 Float32
+// gyroid's emit takes 50 us instead of 35, and surface nets of 384 x 320 x 448
+// Float64 noise (440 MB) 596 us a call instead of 570, although their bits
+// take 67 instead of 77; at 512^3 Float32 both are level.  Its tiles have 32
+// words of a column, whose 128 bytes leave as a line; 8 where those are too
+// few to fill the device (256^3 Float32 11.8 us, 18 with 32), or 4 (32^3 4.2
+// us, 5.3 with 8).  A larger field is read past the cache, by waves side by
+// side along x where that pads no more than the narrower tile does: 1024^3
+// Float32 0.91 -> 0.79 ms (0.82 with the narrower tile), Float64 1.68 -> 1.51
+// ms (1.51).
 template <typename T>
 static void launch_bits_t(const VolArgs& a, hipStream_t st) {
-  const int64_t nxt = (a.g.nx + 2 * kWave - 1) / (2 * kWave), nq = (int64_t)a.g.ny * a.sw;
-  if (nxt * ((nq + 31) / 32) >= 2048)
-    launch_bits_e<T, 32, 2>(a, st);
+  const int64_t nq = (int64_t)a.g.ny * a.sw, x128 = (a.g.nx + 127) / 128, x256 = (a.g.nx + 255) / 256;
+  if ((int64_t)a.g.nx * a.g.ny * a.g.nz * (int64_t)sizeof(T) > (512ll << 20))
+    2 * x256 == x128 ? launch_bits_e<T, 32, 1, 4, true>(a, st)
+                     : launch_bits_e<T, 32, 2, 1, true>(a, st);
+  else if (x128 * ((nq + 31) / 32) >= 2048)
+    launch_bits_e<T, 32, 2, 1, false>(a, st);
   else
-    launch_bits_e<T, 8, 2>(a, st);
+    x128 * ((nq + 7) / 8) >= 256 ? launch_bits_e<T, 8, 2, 1, false>(a, st)
+                                 : launch_bits_e<T, 4, 2, 1, false>(a, st);
 }
 
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, const ScanTail& tail, hipStream_t st) {

@@ -77,3 +77,15 @@ def test_sparse_units(pkg, oracle, name):
 def test_scan_in_the_count(pkg, oracle, nx, name):
     for seed in (1, 2):
         assert check(pkg, oracle, noise((nx, 65, 5), seed, np.float32), name) > 1000
+
+
+@pytest.mark.parametrize("dtype,shape", [
+    (np.float32, (200, 20000, 36)), (np.float64, (250, 800, 347)),  # tiles of 256 columns
+    (np.float32, (301, 910, 500)), (np.float64, (40, 53000, 33)),  # tiles of 128
+])
+def test_field_beyond_the_cache(pkg, oracle, dtype, shape):
+    # over 512 MiB, with ends of tiles along x and of words along z
+    x, y, z = (np.linspace(-1, 1, n, dtype=dtype) for n in shape)
+    f = np.empty(shape, dtype, order="F")
+    f[:] = np.sin(400 * y)[None, :, None] * x[:, None, None] + dtype(0.3) * z - dtype(0.9)
+    assert check(pkg, oracle, f, "mc") > 1000
