@@ -11,7 +11,7 @@
 //                   sampled evenly over the vertices and keeps their
 //                   quantiles as the bounds of the table's 64 x regions
 //   k_weld_insert   open-addressing hash table over the coordinate bits,
-//                   first within each block's 512 vertices in LDS, then
+//                   first within each block's 1024 vertices in LDS, then
 //                   over the whole mesh for the block's first appearances:
 //                   the first vertex of a key claims a slot (CAS from -1),
 //                   equal keys then lower it to their smallest index
@@ -33,7 +33,8 @@
 // The vertex indices in the table, the first appearances and the new indices
 // are 32-bit (I = uint32_t) for meshes of up to 2^31 vertices: every pass
 // moves half the bytes of these, and a line of the table holds twice the slots.
-// @@MEASURED@@
+// 384^3 Float32 value noise mesh against 64-bit indices: k_weld_rep 455 -> 349
+// us, prefix and compaction 295 -> 193, the call 2553 -> 2151.
 //
 // A key's home slot in a large table is its x region's block of slots plus
 // the hash's low bits inside it.  Vertices of a mesh are emitted cell by
@@ -102,10 +103,13 @@ __device__ __forceinline__ uint64_t ordered(uint64_t b) {
 
 constexpr int kWeldSample = 4096;     // x coordinates sorted for the region bounds
 constexpr int kWeldRegions = 64;      // regions of a large table (measured: 64 beat 512 and none)
-constexpr int kWeldSortBlock = 1024;
+constexpr int kWeldSortBlock = kWeldSample / 4;  // a wave sorts 256 of them by itself
 
 // One block: bounds[r - 1] = the (r / nreg) quantile of the sampled x
 // coordinates (as ordered integers), r = 1 .. nreg - 1 (bitonic sort in LDS).
+// One block's chain of steps, alone on the device: a step of stride 128 or
+// less stays within the 256 values of a wave and needs no barrier of the
+// block, which leaves 15 of the 78 (37 us; 60 with a barrier each).
 template <typename W>
 __global__ __launch_bounds__(kWeldSortBlock) void k_weld_bounds(const W* __restrict__ v,
                                                                int64_t nv, int nreg,
@@ -116,17 +120,20 @@ __global__ __launch_bounds__(kWeldSortBlock) void k_weld_bounds(const W* __restr
   __syncthreads();
   for (int size = 2; size <= kWeldSample; size <<= 1)
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int k = threadIdx.x; k < kWeldSample; k += kWeldSortBlock) {
-        const int p = k ^ stride;
-        if (p > k) {
-          const uint64_t a = s[k], b = s[p];
-          if ((a > b) == ((k & size) == 0)) {  // ascending runs where k & size is 0
-            s[k] = b;
-            s[p] = a;
-          }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {  // the wave's 128 pairs
+        const int i = wave_id() * 2 * kWave + q * kWave + lane_id();
+        const int k = 2 * i - (i & (stride - 1)), p = k + stride;
+        const uint64_t a = s[k], b = s[p];
+        if ((a > b) == ((k & size) == 0)) {  // ascending runs where k & size is 0
+          s[k] = b;
+          s[p] = a;
         }
       }
-      __syncthreads();
+      if (stride > 2 * kWave || (stride == 1 && size >= 4 * kWave))
+        __syncthreads();
+      else
+        wave_sync();
     }
   for (int r = threadIdx.x + 1; r < nreg; r += kWeldSortBlock)
     bounds[r - 1] = s[(int64_t)r * kWeldSample / nreg];
@@ -184,17 +191,22 @@ __device__ __forceinline__ uint32_t global_insert(const W* __restrict__ v, I i, 
   return (uint32_t)h;
 }
 
-constexpr int kWeldLT = 512;           // vertices per block: the local pass's window
+constexpr int kWeldLT = 1024;          // vertices per block: the local pass's window
 constexpr int kWeldLS = 2 * kWeldLT;   // local hash slots
+constexpr int kWeldBlock = 512;        // its threads
 
 // Copies of a vertex sit close together in extraction order (the cubes
 // around an edge are neighbours in the same or the next cell row), so each
-// block first welds its 512 consecutive vertices in LDS and sends only
+// block first welds its 1024 consecutive vertices in LDS and sends only
 // the first appearance of each local key to the global table; each vertex
 // notes that local first appearance, whose slot k_weld_rep reads once for
-// all of them.
+// all of them.  Bound by the latency of the table's loads and atomics, which
+// go past the L2s: a longer window sends fewer, a shorter one leaves more
+// blocks to overlap theirs.  384^3 Float32 value noise mesh: 512 vertices and
+// 256 threads 1149 us, 1024 and 512 1074, 2048 and 512 1144, 2048 and 1024
+// 1073 (and k_weld_rep 384 us instead of 357), 4096 and 1024 1354.
 template <typename W, typename I>
-__global__ __launch_bounds__(kBlock) void k_weld_insert(const W* __restrict__ v, int64_t nv,
+__global__ __launch_bounds__(kWeldBlock) void k_weld_insert(const W* __restrict__ v, int64_t nv,
                                                         I* table, uint64_t mask,
                                                         const uint64_t* __restrict__ bounds,
                                                         int nreg, int rbits,
@@ -204,17 +216,17 @@ __global__ __launch_bounds__(kBlock) void k_weld_insert(const W* __restrict__ v,
   __shared__ uint32_t lt[kWeldLS];  // local slot -> smallest local index of its key
   __shared__ uint64_t bnd[kWeldRegions - 1];
   constexpr uint32_t kEmpty = 0xFFFFFFFFu;
-  constexpr int PER = kWeldLT / kBlock;
+  constexpr int PER = kWeldLT / kWeldBlock;
   const int64_t base = (int64_t)blockIdx.x * kWeldLT;
   const int n = nv - base < kWeldLT ? (int)(nv - base) : kWeldLT;
-  for (int k = threadIdx.x; k < kWeldLS; k += kBlock) lt[k] = kEmpty;
-  for (int k = threadIdx.x; k < nreg - 1; k += kBlock) bnd[k] = bounds[k];
-  for (int k = threadIdx.x; k < 3 * n; k += kBlock) key[k] = v[3 * base + k];
+  for (int k = threadIdx.x; k < kWeldLS; k += kWeldBlock) lt[k] = kEmpty;
+  for (int k = threadIdx.x; k < nreg - 1; k += kWeldBlock) bnd[k] = bounds[k];
+  for (int k = threadIdx.x; k < 3 * n; k += kWeldBlock) key[k] = v[3 * base + k];
   __syncthreads();
   uint32_t ls[PER];
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
-    const int j = threadIdx.x + q * kBlock;
+    const int j = threadIdx.x + q * kWeldBlock;
     ls[q] = 0;
     if (j >= n) continue;
     const W x = key[3 * j], y = key[3 * j + 1], z = key[3 * j + 2];
@@ -236,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void k_weld_insert(const W* __restrict__ v,
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
-    const int j = threadIdx.x + q * kBlock;
+    const int j = threadIdx.x + q * kWeldBlock;
     if (j >= n) continue;
     const uint32_t l = lt[ls[q]];
     lrep[base + j] = (uint16_t)l;
@@ -250,25 +262,25 @@ __global__ __launch_bounds__(kBlock) void k_weld_insert(const W* __restrict__ v,
 
 constexpr int kWeldTile = 4096;                 // vertices per prefix tile
 constexpr int kWeldPer = kWeldTile / kBlock;     // per thread in k_weld_pos
-static_assert(kWeldLT % kBlock == 0 && kWeldTile % kWeldLT == 0 && kWeldLT <= 65536,
+static_assert(kWeldLT % kWeldBlock == 0 && kWeldTile % kWeldLT == 0 && kWeldLT <= 65536,
               "windows of whole waves inside one prefix tile, 16-bit local indices");
 
 // Same windows as k_weld_insert: the local first appearances read their
 // key's smallest index from the table, the others take it from them.
 template <typename I>
-__global__ __launch_bounds__(kBlock) void k_weld_rep(int64_t nv, const I* __restrict__ table,
+__global__ __launch_bounds__(kWeldBlock) void k_weld_rep(int64_t nv, const I* __restrict__ table,
                                                      const uint32_t* __restrict__ slot,
                                                      const uint16_t* __restrict__ lrep,
                                                      I* __restrict__ rep,
                                                      uint32_t* __restrict__ tilecnt) {
   __shared__ I res[kWeldLT];
-  constexpr int PER = kWeldLT / kBlock;
+  constexpr int PER = kWeldLT / kWeldBlock;
   const int64_t base = (int64_t)blockIdx.x * kWeldLT;
   const int n = nv - base < kWeldLT ? (int)(nv - base) : kWeldLT;
   uint16_t l[PER];
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
-    const int j = threadIdx.x + q * kBlock;
+    const int j = threadIdx.x + q * kWeldBlock;
     l[q] = 0;
     if (j < n) {
       l[q] = lrep[base + j];
@@ -278,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_weld_rep(int64_t nv, const I* __rest
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
-    const int j = threadIdx.x + q * kBlock;
+    const int j = threadIdx.x + q * kWeldBlock;
     const int64_t i = base + j;
     bool first = false;
     if (j < n) {
@@ -398,13 +410,13 @@ hipError_t weld_t(const WeldArgs& a, hipStream_t st) {
     if (nreg > 1)
       hipLaunchKernelGGL((k_weld_bounds<W>), dim3(1), dim3(kWeldSortBlock), 0, st, v, a.nverts,
                          nreg, a.bounds);
-    hipLaunchKernelGGL((k_weld_insert<W, I>), dim3(nwin), dim3(kBlock), 0, st, v, a.nverts, table,
+    hipLaunchKernelGGL((k_weld_insert<W, I>), dim3(nwin), dim3(kWeldBlock), 0, st, v, a.nverts, table,
                        (uint64_t)(a.nslots - 1), (const uint64_t*)a.bounds, nreg, rbits, a.slot,
                        a.lrep);
     const int64_t ntiles = (a.nverts + kWeldTile - 1) / kWeldTile;
     hipLaunchKernelGGL(k_fill_i64, dim3(grid_of((ntiles + 1) / 2)), dim3(kBlock), 0, st,
                        (int64_t*)a.tilecnt, (ntiles + 1) / 2, (int64_t)0);
-    hipLaunchKernelGGL((k_weld_rep<I>), dim3(nwin), dim3(kBlock), 0, st, a.nverts,
+    hipLaunchKernelGGL((k_weld_rep<I>), dim3(nwin), dim3(kWeldBlock), 0, st, a.nverts,
                        (const I*)table, (const uint32_t*)a.slot, (const uint16_t*)a.lrep, rep,
                        a.tilecnt);
     hipLaunchKernelGGL(k_weld_tiles, dim3(1), dim3(1024), 0, st, (const uint32_t*)a.tilecnt,

@@ -1,4 +1,4 @@
-"""Vertex welding at the ends of its windows (512 vertices), prefix tiles (4096)
+"""Vertex welding at the ends of its windows (1024 vertices), prefix tiles (4096)
 and table sizes, through both entry points (faces renumbered in place, and
 into another buffer), against the definition: exact."""
 import ctypes
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("nv", [1, 2, 511, 512, 513, 4095, 4096, 4097, 13107, 70001])
+@pytest.mark.parametrize("nv", [1, 2, 511, 512, 513, 1023, 1024, 1025, 4095, 4096, 4097, 13107, 70001])
 def test_window_and_tile_ends(pkg, oracle, nv, dtype):
     import torch
     from importlib import import_module
