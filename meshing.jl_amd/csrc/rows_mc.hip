@@ -209,28 +209,22 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
     const uint64_t rest = (todo >> (gi - g0)) & ~1ull;
     const int gn = rest ? gi + __builtin_ctzll(rest) : g1;
     if (gn < g1) raw = load_raw(a, x, gn, lane);  // the next unit's words, meanwhile
-    uint32_t act = active_cells(r);
+    const uint32_t act = active_cells(r);
     const uint32_t incl = wave_scan_dpp(__popc(act));
     const int total = __builtin_amdgcn_readlane((int)incl, kWave - 1);
-    int k = (int)incl - (int)__popc(act);
     for (int lo = 0; lo < total;) {
       // the next cells of the unit that fit the queue, at most 64
       const int take = min(min(kCells - nc, kWave), total - lo);
-      while (act != 0 && k < lo + take) {
-        wm.list[nc + k - lo] = (uint32_t)lane | ((uint32_t)__builtin_ctz(act) << 9);
-        act &= act - 1;
-        ++k;
-      }
-      wave_sync();
       const int c = nc + lane;
       const bool in = lane < take;
-      const uint32_t e = in ? wm.list[c] : 0u;
-      const uint32_t cs = cell_case_of(r, (int)(e & 63), (int)(e >> 9));
+      int L, b;
+      listed_cell(act, incl, lo, take, wm.list + nc, &L, &b);
+      const uint32_t cs = cell_case_of(r, L, b);
       const uint32_t pk = in ? sm.tab.cnt[cs] : 0u;
       const uint32_t inc = wave_scan_dpp(pk);
       const uint32_t sv = V + ((inc - pk) & 0xFFFF), sf = F + ((inc - pk) >> 16);
       if (in) {
-        wm.list[c] = (e + 64u * (uint32_t)(gi - g0)) | (cs << 14);
+        wm.list[c] = ((uint32_t)L + 64u * (uint32_t)(gi - g0)) | ((uint32_t)b << 9) | (cs << 14);
         wm.lpv[c] = (uint16_t)sv;
         wm.lpf[c] = (uint16_t)sf;
         atomicOr((unsigned long long*)&wm.vbits[sv >> 6], 1ull << (sv & 63));

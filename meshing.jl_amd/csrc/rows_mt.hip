@@ -447,7 +447,6 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
       for (int i = 0; i < 9; ++i) above |= k[i].hi << (2 * i);
       const uint32_t incl = wave_scan_dpp(__popc(act));
       const int total = __builtin_amdgcn_readlane((int)incl, kWave - 1);
-      int at = (int)incl - (int)__popc(act);
       // the words at -x, -y and both: how far back their first vertices are
       // from this word's, and their cells' vertices
       uint32_t w10 = 0, w01 = 0, w11 = 0, pre = 0;
@@ -485,21 +484,11 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
                (three(m0, m3, m1, c00) << 16);
         }
       }
-      while (done > 0 && act != 0 && at < done) {  // the cells that are through
-        act &= act - 1;
-        ++at;
-      }
       while (done < total && nc < kCells) {
         const int take = min(min(kCells - nc, kWave), total - done);
-        while (act != 0 && at < done + take) {
-          wm.list[nc + at - done] = (uint32_t)lane | ((uint32_t)__builtin_ctz(act) << 9);
-          act &= act - 1;
-          ++at;
-        }
-        wave_sync();
         const bool in = lane < take;
-        const uint32_t e = in ? wm.list[nc + lane] : 0u;
-        const int L = (int)(e & 63), b = (int)(e >> 9);
+        int L, b;
+        listed_cell(act, incl, done, take, wm.list + nc, &L, &b);
         auto from = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(L << 2, (int)v); };
         const uint32_t hi = from(above), lowm = (1u << b) - 1u;
         uint32_t n27 = 0;
@@ -535,7 +524,8 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
           const uint32_t nb = (x > 0 ? 1u : 0u) | (cy > 0 ? 2u : 0u) | (cz > 0 ? 4u : 0u);
           const uint32_t near = (x < 2 || cy < 2 || cz < 2) ? 1u : 0u;
           const int c = nc + lane;
-          wm.list[c] = (e + 64u * (uint32_t)(gi - g0)) | (zc << 14) | (nb << 22) | (near << 25);
+          wm.list[c] = ((uint32_t)L + 64u * (uint32_t)(gi - g0)) | ((uint32_t)b << 9) | (zc << 14) | (nb << 22) |
+                       (near << 25);
           wm.around[c] = n27;
           wm.d10[c] = d10;
           wm.d01[c] = d01;

@@ -204,13 +204,12 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
       const CellWord r = load_cells(a, x, gi, lane);
       const BackWords k = load_back(a, x, r);
       uint32_t act = active_cells(r);
-      const uint32_t here = act;
       const uint32_t a10 = active_of(k.x0, r.c00, k.x1, r.c01, r.valid);
       const uint32_t a01 = active_of(k.y0, k.y1, r.c00, r.c10, r.valid);
       const uint32_t a11 = active_of(k.xy, k.y0, k.x0, r.c00, r.valid);
       const uint32_t incl = wave_scan_dpp(__popc(act));
       const int total = __builtin_amdgcn_readlane((int)incl, kWave - 1);
-      int at = (int)incl - (int)__popc(act);
+      const int at = (int)incl - (int)__popc(act);
       // how far back the first vertices of the words at -x, -y and both are
       // from this word's (only a quad's cells are asked for, and they exist)
       uint32_t w10 = 0, w01 = 0, w11 = 0;
@@ -225,25 +224,15 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
       // quads only where the cells at -1 exist: the axes of corner 0's edges
       // that a cell of the word may have faces on (bit 0 of the column: z > 0)
       const uint32_t has = (r.y > 0 ? 1u : 0u) | (x > 0 ? 2u : 0u) | (r.w > 0 ? 4u : 0u);
-      while (done > 0 && act != 0 && at < done) {  // the cells that are through
-        act &= act - 1;
-        ++at;
-      }
       while (done < total && nc < kCells) {
         const int take = min(min(kCells - nc, kWave), total - done);
-        while (act != 0 && at < done + take) {
-          wm.list[nc + at - done] = (uint32_t)lane | ((uint32_t)__builtin_ctz(act) << 9);
-          act &= act - 1;
-          ++at;
-        }
-        wave_sync();
         const bool in = lane < take;
-        const uint32_t e = in ? wm.list[nc + lane] : 0u;
-        const int L = (int)(e & 63), b = (int)(e >> 9);
+        int L, b;
+        listed_cell(act, incl, done, take, wm.list + nc, &L, &b);
         auto from = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(L << 2, (int)v); };
         const uint32_t c = cell_case_of(r, L, b);
         const uint32_t lowm = (1u << b) - 1u;
-        const uint32_t mine = __popc(from(here) & lowm);
+        const uint32_t mine = __popc(from(act) & lowm);
         const uint32_t d10 = from(w10) + mine - __popc(from(a10) & lowm);
         const uint32_t d01 = from(w01) + mine - __popc(from(a01) & lowm);
         const uint32_t d11 = from(w11) + mine - __popc(from(a11) & lowm);
@@ -257,7 +246,7 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
         const uint32_t inc = wave_scan_dpp(n), sf = F + inc - n;
         const uint64_t with = __ballot(n != 0);
         if (in) {
-          wm.list[nc + lane] = (e + 64u * (uint32_t)(gi - g0)) | (c << 14);
+          wm.list[nc + lane] = ((uint32_t)L + 64u * (uint32_t)(gi - g0)) | ((uint32_t)b << 9) | (c << 14);
           wm.d10[nc + lane] = d10;
           wm.d01[nc + lane] = d01;
           wm.d11[nc + lane] = d11;
