@@ -492,32 +492,50 @@ def traffic_of(workload, family_id):
     return e["bytes_per_launch"]
 
 
-# the emit kernel an autotuned family launches, per method: (name, template
-# prefix after the method parameter); MC's brick depth per element type and
-# family (family 3 halves it)
-_EMIT_NAMES = {"mc": {3: "k_emit_mc5", 2: "k_emit_mc5", 1: "k_emit_mc4", 0: "k_emit"},
-               "mt": {2: "k_emit_h5", 1: "k_emit_halo", 0: "k_emit"},
-               "sn": {3: "k_emit_h5", 2: "k_emit_h5", 1: "k_emit_halo", 0: "k_emit"}}
+# the emit kernel an autotuned family launches, per method.  Family 2 is the
+# row kernels; a volume they do not take (or have no memory for) goes to the
+# lanes-along-x kernel of the second table, in counter runs of such volumes.
+_EMIT_NAMES = {"mc": {3: "k_emit_mc5", 2: "k_rows_mc", 1: "k_emit_mc4", 0: "k_emit"},
+               "mt": {2: "k_rows_mt", 1: "k_emit_halo", 0: "k_emit"},
+               "sn": {3: "k_emit_h5", 2: "k_rows_sn", 1: "k_emit_halo", 0: "k_emit"}}
+_FALLBACK_NAMES = {"mc": "k_emit_mc5", "mt": "k_emit_h5", "sn": "k_emit_h5"}
+# brick depth of the lanes-along-x emits per element type or method, and family
 _MC5_ZC = {("float32", 2): 16, ("float32", 3): 8, ("float64", 2): 8, ("float64", 3): 4}
-# brick depth of the tetrahedra / surface-nets emit per family
 _H5_ZC = {("mt", 2): 4, ("sn", 2): 8, ("sn", 3): 4}
 
 
-def _emit_pattern(method, dtype, family_id):
-    """A regular expression matching the demangled name of the emit kernel
-    that `family_id` launches for this (method, field type)."""
-    import re
-    name = _EMIT_NAMES[method][family_id]
+def _emit_patterns(method, dtype, family_id):
+    """Regular expressions matching the demangled names of the emit kernels
+    that `family_id` launches for this (method, field type), the preferred
+    one first."""
     t = "float" if dtype == "float32" else "double"
-    if name == "k_emit_mc5":
-        return re.compile(rf"k_emit_mc5<{t}, [a-z]+, [a-z]+, {_MC5_ZC[(dtype, family_id)]},")
     mid = {"mc": 0, "mt": 1, "sn": 2}[method]
-    if name == "k_emit":
-        return re.compile(rf"k_emit<{mid}, {t},")
-    if name == "k_emit_h5":
-        return re.compile(rf"k_emit_h5<{mid}, {t}, [a-z]+, [a-z]+, [a-z]+, "
-                          rf"{_H5_ZC[(method, family_id)]},")
-    return re.compile(rf"{name}<{mid}, {t},")
+    names = [_EMIT_NAMES[method][family_id]]
+    if family_id == 2:
+        names.append(_FALLBACK_NAMES[method])
+    out = []
+    for name in names:
+        if name.startswith("k_rows_"):
+            out.append(rf"{name}<{t},")
+        elif name == "k_emit_mc5":
+            out.append(rf"k_emit_mc5<{t}, [a-z]+, [a-z]+, {_MC5_ZC[(dtype, family_id)]},")
+        elif name == "k_emit_h5":
+            out.append(rf"k_emit_h5<{mid}, {t}, [a-z]+, [a-z]+, [a-z]+, "
+                       rf"{_H5_ZC[(method, family_id)]},")
+        else:
+            out.append(rf"{name}<{mid}, {t},")
+    return [re.compile(x) for x in out]
+
+
+def _count_patterns(method, dtype, family_id):
+    """The same for the count: of the row kernels the pass that reads the
+    field, k_bits."""
+    t = "float" if dtype == "float32" else "double"
+    mid = {"mc": 0, "mt": 1, "sn": 2}[method]
+    out = [rf"k_count4<{t}, {mid},"]
+    if family_id == 2:
+        out.insert(0, rf"k_bits<{t},")
+    return [re.compile(x) for x in out]
 
 
 def summarize_counters(fetch_dir, write_dir, line_file, out_file=TRAFFIC_FILE, copy_bytes=1 << 30):
@@ -564,15 +582,16 @@ def summarize_counters(fetch_dir, write_dir, line_file, out_file=TRAFFIC_FILE, c
         for i, (key, meth, dtype, r, pick) in enumerate(loads):
             lo = gens[i] if i < len(gens) else 0
             hi = gens[i + 1] if i + 1 < len(gens) else float("inf")
-            t = "float" if dtype == "float32" else "double"
-            mid = {"mc": 0, "mt": 1, "sn": 2}[meth]
-            for part, pat in (("emit", _emit_pattern(meth, dtype, r["family_id"])),
-                              ("count", re.compile(rf"k_count4<{t}, {mid},"))):
-                grids = {}
-                for x in rs:
-                    if lo <= int(x["Dispatch_Id"]) < hi and pat.search(x["Kernel_Name"]):
-                        grids.setdefault((x["Kernel_Name"], int(x["Grid_Size"])), []).append(
-                            float(x["Counter_Value"]))
+            for part, pats in (("emit", _emit_patterns(meth, dtype, r["family_id"])),
+                               ("count", _count_patterns(meth, dtype, r["family_id"]))):
+                for pat in pats:
+                    grids = {}
+                    for x in rs:
+                        if lo <= int(x["Dispatch_Id"]) < hi and pat.search(x["Kernel_Name"]):
+                            grids.setdefault((x["Kernel_Name"], int(x["Grid_Size"])), []).append(
+                                float(x["Counter_Value"]))
+                    if grids:
+                        break
                 if not grids:
                     continue
                 # the 1024^3 launches have the largest grid of their
@@ -654,7 +673,8 @@ def main():
             # a sparse field: the emit fetches only the z chunks with active
             # cells, and the count pass, which reads every sample once,
             # dominates (its time includes the scan and the size read-back)
-            b, t, kernel = r["field_bytes"], r["count_s"], "k_count4"
+            b, t = r["field_bytes"], r["count_s"]
+            kernel = "k_bits" if r["family_id"] == 2 else "k_count4"
             traffic = traffic_of(workload + "_count", r["family_id"])
         else:
             b, t = r["field_bytes"] + r["out_bytes"], r["emit_s"]

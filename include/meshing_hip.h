@@ -120,18 +120,21 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
  * stream other than the null stream) runs each phase from a hipGraph: the
  * second such call captures the phase's copies and launches, later calls
  * replay it (new output pointers travel through the descriptor copy, so
- * they may change).  The count and emit kernels of the batch are persistent:
- * as many blocks as fit on the device take the batch's tiles from a work
- * queue.  msh_batch_graph_launches reports how many times each phase has run
+ * they may change).  A batch whose volumes all take the row kernels runs them
+ * with a block per tile; in any other, the count and emit kernels are
+ * persistent: as many blocks as fit on the device take the batch's tiles
+ * from a work queue.  msh_batch_graph_launches reports how many times each phase has run
  * from a graph on this context.  No counterpart in the reference. */
 int msh_batch_graph_launches(void* ctx, int64_t* count_phase, int64_t* emit_phase);
 
-/* Kernel choice.  The emit pass has kernel families per method: 2 lanes
- * along x (the default), 1 lanes along z, 0 a generic kernel, and 3 the
- * lanes-along-x kernel with half-depth bricks (a tile shape, for Naive
- * Surface Nets and for Marching Cubes with one element type throughout and
- * Float64 axes; otherwise the same as 2); each family falls back to the
- * next one down for volumes it cannot take.
+/* Kernel choice.  There are kernel families per method: 2 the row kernels
+ * (the default: one bit per sample, counts and emits by words of 32 samples
+ * along z; lanes along x with full-depth bricks for a volume they do not
+ * take or have no memory for), 3 lanes along x with half-depth bricks (a
+ * tile shape, for Naive Surface Nets and for Marching Cubes with one element
+ * type throughout and Float64 axes; otherwise lanes along x with full-depth
+ * bricks), 1 lanes along z and 0 a generic kernel; each family falls back to
+ * the next one down for volumes it cannot take.
  * msh_autotune counts the given field, times the emit of every family that
  * takes it (the best of 3 to 50 launches each, about 2 ms, on the
  * context's stream, into a scratch buffer) and records the fastest for the
@@ -152,9 +155,9 @@ int msh_autotune(void* ctx, const msh_field* field, const msh_params* params, in
  * run side by side, one pass over the groups (most volumes first) times the
  * whole batch with each other family that takes the group and keeps a
  * change that makes it 1% faster.  chosen[v] (n entries, may be null)
- * returns volume v's.  A batch runs the persistent batched kernels,
- * whose best shape differs from a lone small volume's (which cannot fill
- * the device by itself).  Leaves no batch state behind: call
+ * returns volume v's.  A batch runs batched kernels, whose best
+ * shape differs from a lone small volume's (which cannot fill the device by
+ * itself).  Leaves no batch state behind: call
  * msh_batch_count next. */
 int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_params* params,
                        int32_t* chosen);

@@ -38,7 +38,7 @@ __all__ = ["isosurface", "isosurface_batch", "AbstractMeshingAlgorithm", "Marchi
            "read_nrrd", "write_nrrd", "NrrdInfo", "read_ply", "write_ply"]
 
 # emit kernel families, best first (see msh_autotune in include/meshing_hip.h)
-KERNEL_FAMILIES = {3: "lanes along x, half-depth bricks", 2: "lanes along x",
+KERNEL_FAMILIES = {3: "lanes along x, half-depth bricks", 2: "rows of sample bits",
                    1: "lanes along z", 0: "generic", -1: "default"}
 
 
@@ -343,8 +343,8 @@ def autotune(sdf, method=None, *args, X=(-1, 1), Y=(-1, 1), Z=(-1, 1), device=0)
     context (size classes by cell count: below 2^20, below 2^23, larger);
     later calls of isosurface, isosurface_batch and the server on that
     device use it for volumes of that class.  Returns the chosen family (3
-    lanes along x with half-depth bricks, 2 lanes along x, 1 lanes along z,
-    0 generic; see KERNEL_FAMILIES)."""
+    lanes along x with half-depth bricks, 2 rows of sample bits, 1 lanes
+    along z, 0 generic; see KERNEL_FAMILIES)."""
     method, X, Y, Z = _split_args(method, args, X, Y, Z)
     f, keep, on_dev = _field(sdf)
     p = _params(method, X, Y, Z)

@@ -147,8 +147,9 @@ __device__ __forceinline__ uint32_t nth_bit(uint32_t x, uint32_t r) {
 // incl = their inclusive count: its word's lane and its bit (0 from `take`
 // on).  Each word with cells marks its first one's place in mark[0, take);
 // the word of a place is the last one marked at or before it.  (A loop over
-// the bits of each lane's word waits for the fullest word: it took a fifth
-// of the emits' vector and half of their scalar instructions.)
+// the bits of each lane's word waits for the fullest word: 301 x 217 x 389
+// Float32 Marching Cubes emit 174 us so, 160 us this way; 512^3 tetrahedra
+// 1584 and 1553.)
 __device__ __forceinline__ void listed_cell(uint32_t act, uint32_t incl, int lo, int take,
                                             uint32_t* mark, int* word, int* bit) {
   const int lane = lane_id();
@@ -251,10 +252,11 @@ __device__ __forceinline__ int64_t rows_block_tile(int64_t b, int64_t nb) {
 }
 
 // 64 records of three values from LDS to the output, each through `value`:
-// records [s0, s1) of the 64 at `out`, the wave's lanes on consecutive values, so that every line is
-// written whole by one store instruction.  Buffer stores: a value outside
-// the records gets an offset past the buffer and is dropped, so there is no
-// branch, and a wait for loads issued before does not wait for the stores.
+// records [s0, s1) of the 64 at `out`, the wave's lanes on consecutive
+// values, so that every line is written whole by one store instruction.
+// Buffer stores: a value outside the records gets an offset past the buffer
+// and is dropped, so there is no branch, and a wait for loads issued before
+// does not wait for the stores.
 // Non-temporal: a line is written once and whole, and kept out of the L2 it
 // leaves room there for the samples that the waves nearby share (301 x 217 x
 // 389 Float32 value noise 250 -> 172 us, 1024^3 Float64 5.39 -> 4.97 ms).

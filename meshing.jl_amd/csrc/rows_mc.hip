@@ -15,11 +15,13 @@
 // bytes per z chunk, about two writes a line, and classifies every cell twice
 // over; here a unit's run is kilobytes long and the empty cells cost one AND
 // of words for 32 of them.  Emit, before -> now: 256^3 Float32 gyroid 80 ->
-// 36 us, 301 x 217 x 389 Float32 value noise (rows not 16-byte aligned) 449
-// -> 172 us, 1024^3 Float64 value noise 7.0 -> 4.97 ms.  The writes alone
-// take 2.6 ms of the last (3.8 TB/s), the samples' lines the rest: the 64
-// vertices of a step lie on dozens of planes, and a 128-byte line is fetched
-// about three times before the 16 planes x that share it are done with it.
+// 35 us, 301 x 217 x 389 Float32 value noise (rows not 16-byte aligned) 449
+// -> 160 us, 1024^3 Float64 value noise 7.0 -> 4.8 ms.  The last reads 5.1 GB
+// and writes 9.8 GB, 2.9 ms at the rate of a copy; the rest is the wait of
+// the gathers (the two samples and two pairs of coordinates of 64 vertices
+// that lie on dozens of lines) for their turn in the address unit, at 4
+// waves a SIMD.  Blocks of 8 and 16 waves, whose planes share the lines, were
+// slower (5.1 and 5.2 ms): a block then lasts as long as its slowest wave.
 #include <type_traits>
 
 #include "rows.h"

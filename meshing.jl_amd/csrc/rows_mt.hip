@@ -19,7 +19,7 @@
 // take these from the constant tables.
 //
 // Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 158 -> 90 us, 512^3
-// Float32 value noise 2.05 -> 1.58 ms.
+// Float32 value noise 2.05 -> 1.55 ms.
 // Bound by vector issue (55% of the cycles on the noise) and the
 // latency of each step at 2.8 waves a SIMD (128 registers, 40 KB of LDS a
 // block).  A queue of 64 cells with all 19 edge numbers in LDS, which saves

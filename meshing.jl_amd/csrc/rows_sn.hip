@@ -13,8 +13,8 @@
 // as in rows_mc.hip.  A unit that does not fit the queue is read again after
 // the emit, which so needs no registers for it.
 //
-// Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 114 -> 39 us,
-// 384 x 320 x 448 Float64 value noise 774 -> 459 us.  Bound by vector issue
+// Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 114 -> 37 us,
+// 384 x 320 x 448 Float64 value noise 774 -> 482 us.  Bound by vector issue
 // (58% of the cycles there, most of it the divisions and interpolations of
 // the edges) and by the latency of each step's look-ups at 3 to 4 waves a
 // SIMD; holding the samples of a step in registers while its unit is listed
