@@ -13,6 +13,9 @@ namespace msh {
 enum Kind : int { K_INT64 = 0, K_F32 = 1, K_F64 = 2 };
 enum Method : int { MC = 0, MT = 1, SN = 2 };
 
+// waves (x planes) of a row emit's block
+constexpr int rows_emit_waves(int method) { return method == SN ? 2 : 4; }
+
 // Cells are (nx-1)*(ny-1)*(nz-1).  The emission order of the reference is
 // x outermost, z innermost (src/marching_cubes.jl:40).  A "unit" is one
 // z-row of cells (fixed x, y) cut into nzseg segments of zseg cells; units

@@ -210,23 +210,27 @@ __device__ __forceinline__ int64_t word_vertex(const VolArgs& a, int x, uint32_t
   return a.voff[a.ubase + u] + (int64_t)a.wpre[64 * (a.ubase + u) + (q & 63)];
 }
 
-// Emit tile t: kWaves x planes (one a wave, so the waves of a block read the
-// same lines) by a.ue units.  Tiles go over 8 blocks along x (32 planes, a
-// 128-byte line of Float32 samples), then along the planes, then to the next
-// 8 blocks, so the tiles in flight on an XCD share their lines in its L2.
+static_assert(rows_emit_waves(MC) == kWaves && rows_emit_waves(MT) == kWaves, "their blocks");
+
+// Emit tile t: W x planes (one a wave of the block, so its waves read the
+// same lines) by a.ue units.  Tiles go over 32 planes along x (a 128-byte line
+// of Float32 samples), then along the planes, then to the next 32, so the
+// tiles in flight on an XCD share their lines in its L2.
+template <int W>
 __device__ __forceinline__ void rows_tile(const VolArgs& a, int64_t t, int* x, int* g0) {
-  const uint32_t nxb = (uint32_t)(a.g.nx - 1 + kWaves - 1) / kWaves;
+  constexpr uint32_t G = 32 / W;  // blocks of 32 planes
+  const uint32_t nxb = (uint32_t)(a.g.nx - 1 + W - 1) / W;
   const uint32_t gb = (uint32_t)(a.upx + a.ue - 1) / (uint32_t)a.ue;
-  const uint32_t full = nxb / 8, rest = nxb - full * 8;
-  const uint32_t grp = (uint32_t)t / (8 * gb);
-  uint32_t r, n = 8, first = grp;
+  const uint32_t full = nxb / G, rest = nxb - full * G;
+  const uint32_t grp = (uint32_t)t / (G * gb);
+  uint32_t r, n = G, first = grp;
   if (grp >= full) {
     first = full;
     n = rest;
   }
-  r = (uint32_t)t - first * 8 * gb;
+  r = (uint32_t)t - first * G * gb;
   const uint32_t gi = r / n;
-  *x = (int)(first * 8 + (r - gi * n)) * kWaves + wave_id();
+  *x = (int)(first * G + (r - gi * n)) * W + wave_id();
   *g0 = (int)gi * a.ue;
 }
 
@@ -241,10 +245,12 @@ struct __attribute__((packed, aligned(sizeof(T)))) Pair {
 // of 32 in turn, so tiles that share lines meet in one L2 and a field whose
 // surface lies in a part of its planes still keeps every XCD busy (1024^3
 // Float32 sphere emit 158 -> 132 us; the 2048 blocks of a 256^3 gyroid are
-// 36 us in one run an XCD and 39 in turns).
-__device__ __forceinline__ int64_t rows_block_tile(int64_t b, int64_t nb) {
+// 36 us in one run an XCD and 39 in turns; surface nets of 384 x 320 x 448
+// Float64 noise, 13440 blocks of two waves, 458 and 430).  `few`: the blocks
+// from which a launch takes turns.
+__device__ __forceinline__ int64_t rows_block_tile(int64_t b, int64_t nb, int64_t few = 8192) {
   constexpr int64_t C = 32;
-  if (nb < 8192) return xcd_tile(b, nb);
+  if (nb < few) return xcd_tile(b, nb);
   if (b >= nb / (8 * C) * (8 * C)) return b;
   // (turned by one XCD a round: the y range of a plane is not one XCD's)
   const int64_t round = (b >> 3) / C, at = (b >> 3) % C;

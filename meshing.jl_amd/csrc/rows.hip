@@ -376,14 +376,14 @@ void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a) {
 // would each pay the way to the first sample for a few cells (1024^3 Float32
 // sphere, 12 vertices a unit: 8 units 158 us, 1 unit 349 us; 1024^3 Float64
 // value noise, 520 vertices a unit: 1 unit 5.4 ms, 8 units 6.0 ms), as long
-// as the blocks fill the device.  One where the vertices are not known yet
+// as the waves fill the device.  One where the vertices are not known yet
 // (a batch lays its tiles out before it counts): nverts < 0.
 void rows_emit_tiling(VolArgs* a, int64_t nverts) {
-  const int64_t nxb = (a->g.nx - 1 + kWaves - 1) / kWaves;
+  const int64_t waves = rows_emit_waves(a->method), nxb = (a->g.nx - 1 + waves - 1) / waves;
   const int64_t full = a->method == MC ? 256 : 64;  // about 64 cells
   a->ue = 1;
   while (nverts >= 0 && a->ue < kMaxUE && nverts * 2 * a->ue <= full * a->g.units &&
-         nxb * ((a->upx + 2 * a->ue - 1) / (2 * a->ue)) >= 8192)
+         waves * nxb * ((a->upx + 2 * a->ue - 1) / (2 * a->ue)) >= 32768)
     a->ue *= 2;
   a->ntiles = nxb * ((a->upx + a->ue - 1) / a->ue);
 }

@@ -193,7 +193,7 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
   const uint32_t rbytes = (uint32_t)g.nx * (uint32_t)sizeof(T);
   const int lane = lane_id();
   int x, g0;
-  rows_tile(a, t, &x, &g0);
+  rows_tile<kWaves>(a, t, &x, &g0);
   const int g1 = min(g0 + a.ue, a.upx);
   // lane i holds unit g0 + i's counts and output offsets
   uint32_t cnt = 0;

@@ -13,8 +13,8 @@
 // as in rows_mc.hip.  A unit that does not fit the queue is read again after
 // the emit, which so needs no registers for it.
 //
-// Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 114 -> 37 us,
-// 384 x 320 x 448 Float64 value noise 774 -> 482 us.  Bound by vector issue
+// Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 114 -> 34 us,
+// 384 x 320 x 448 Float64 value noise 774 -> 430 us.  Bound by vector issue
 // (58% of the cycles there, most of it the divisions and interpolations of
 // the edges) and by the latency of each step's look-ups at 3 to 4 waves a
 // SIMD; holding the samples of a step in registers while its unit is listed
@@ -27,6 +27,13 @@ namespace msh {
 namespace {
 
 constexpr int kCells = 256;  // cells queued at a time, per wave
+
+// Two waves a block: a block keeps its registers and LDS until its slowest
+// wave is done, and there are no tables to share (256^3 Float32 gyroid emit 37
+// us with four waves, 34 with two, 41 with one; 384 x 320 x 448 Float64 noise
+// 483, 427 and 438).
+constexpr int kSnWaves = rows_emit_waves(SN);
+constexpr int kSnBlock = kSnWaves * kWave;
 
 // The 12 cube edges in Marching Cubes order (src/lut/mc.jl _mc_edge_list),
 // corners in natural order (bits 0, 1, 2: dx, dy, dz).
@@ -48,13 +55,13 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
     uint32_t d10[kCells], d01[kCells], d11[kCells];  // how far back the vertices at -x, -y, both are
     uint32_t face[kCells];  // cells with faces: cell | axes << 8 | below << 11 | slot << 12
   };
-  __shared__ __align__(16) Wave waves[kWaves];
+  __shared__ __align__(16) Wave waves[kSnWaves];
   const Geom g = a.g;
   const uint32_t pbytes = (uint32_t)((int64_t)g.nx * g.ny * (int64_t)sizeof(T));
   const uint32_t rbytes = (uint32_t)g.nx * (uint32_t)sizeof(T);
   const int lane = lane_id();
   int x, g0;
-  rows_tile(a, t, &x, &g0);
+  rows_tile<kSnWaves>(a, t, &x, &g0);
   const int g1 = min(g0 + a.ue, a.upx);
   // lane i holds unit g0 + i's counts and output offsets
   uint32_t cnt = 0;
@@ -271,15 +278,17 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
 }
 
 template <typename T, typename M, typename Out, int CXM>
-__global__ __launch_bounds__(kBlock) void k_rows_sn(VolArgs a) {
+__global__ __launch_bounds__(kSnBlock) void k_rows_sn(VolArgs a) {
   rows_sn_tile<T, M, Out, CXM>(a, rows_block_tile(blockIdx.x, a.ntiles));
 }
 
-// Batched: a block per tile of the launch; the map names its volume.
+// Batched: a block per tile of the launch; the map names its volume.  Turns
+// over the XCDs from 16384 blocks, as many waves as in the other methods'
+// batches (32 mixed volumes 605 us a batch, 624 with turns from 8192).
 template <typename T, typename M, typename Out, int CXM>
-__global__ __launch_bounds__(kBlock) void k_rows_sn_b(const VolArgs* __restrict__ vols,
+__global__ __launch_bounds__(kSnBlock) void k_rows_sn_b(const VolArgs* __restrict__ vols,
                                                   const int32_t* __restrict__ emap, int64_t gbase) {
-  const int64_t b = gbase + rows_block_tile(blockIdx.x, gridDim.x);
+  const int64_t b = gbase + rows_block_tile(blockIdx.x, gridDim.x, 16384);
   const VolArgs a = vols[__builtin_amdgcn_readfirstlane(emap[b])];
   rows_sn_tile<T, M, Out, CXM>(a, b - a.eblk0);
 }
@@ -292,10 +301,10 @@ __global__ __launch_bounds__(kBlock) void k_rows_sn_b(const VolArgs* __restrict_
 template <typename T, typename M, typename Out, int CXM>
 static hipError_t rows_sn_cx(const VolArgs& a, const RowsBatch* b, hipStream_t st) {
   if (b)
-    hipLaunchKernelGGL((k_rows_sn_b<T, M, Out, CXM>), dim3((unsigned)b->nblocks), dim3(kBlock), 0, st, b->vols,
+    hipLaunchKernelGGL((k_rows_sn_b<T, M, Out, CXM>), dim3((unsigned)b->nblocks), dim3(kSnBlock), 0, st, b->vols,
                        b->map, b->gbase);
   else
-    hipLaunchKernelGGL((k_rows_sn<T, M, Out, CXM>), dim3((unsigned)a.ntiles), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_rows_sn<T, M, Out, CXM>), dim3((unsigned)a.ntiles), dim3(kSnBlock), 0, st, a);
   return hipGetLastError();
 }
 
