@@ -491,6 +491,17 @@ int setup_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t
 // The row kernels serve the default family and family 2.
 bool rows_family(const Plan& p) { return p.family < 0 || p.family == 2; }
 
+// By default a single volume goes to them from a number of units on in
+// Marching Tetrahedra, whose waves are the longest: with few units a dense
+// one leaves most of the device idle, where the tiles of the lanes-along-x
+// kernel are smaller (value noise, whole call: 110 x 100 x 120 Float32, 763
+// units, 257 us by rows and 210 by lanes along x; 160^3 Float32, 2067 units,
+// 262 and 218; 165 x 160 x 170 Float64, 2460 units, 246 and 323; 180^3
+// Float32, 3043 units, 258 and 319).  The other methods gain at every size.
+bool rows_single(const Plan& p, const Geom& rows) {
+  return p.method != MT || p.family == 2 || rows.units >= 2304;
+}
+
 bool same_call(const Ctx* c, const msh_field* f, const msh_params* p) {
   return c->have && memcmp(&c->field, f, sizeof(*f)) == 0 &&
          memcmp(&c->params, p, sizeof(*p)) == 0;
@@ -628,7 +639,7 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
   RowsGeom rg{};
   Geom gr = g;
   void* bits = nullptr;
-  if (rows_family(pl) && rows_geom(pl, &gr, &rg)) {
+  if (rows_family(pl) && rows_geom(pl, &gr, &rg) && rows_single(pl, gr)) {
     // with no room for the sample bits the other kernels, which need less,
     // take the volume
     if (setup_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr),
