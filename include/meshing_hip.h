@@ -163,6 +163,16 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
                        int32_t* chosen);
 int msh_set_kernel_family(void* ctx, int32_t method, int32_t dtype, int32_t family);
 
+/* Limits of a context.  Results do not depend on them.
+ * MSH_LIMIT_SAMPLE_BITS: the most bytes of workspace that a call's row
+ * kernels may take for their sample bits and what goes with them (a bit per
+ * sample, and for tetrahedra and surface nets 2 bytes per 32 cells);
+ * negative, the default: no limit.  A call over it takes the other kernels,
+ * as one does for whose bits the device has no room.
+ * No counterpart in the reference. */
+typedef enum { MSH_LIMIT_SAMPLE_BITS = 0 } msh_limit;
+int msh_set_limit(void* ctx, int32_t what, int64_t value);
+
 /* Vertex welding, the opt-in step after extraction: vertices whose three
  * coordinates have identical bit patterns merge into their first
  * appearance, the welded vertices keep first-appearance order, and the

@@ -15,13 +15,14 @@ MSH_OK, MSH_ERR_ARGUMENT, MSH_ERR_OUT_OF_MEMORY, MSH_ERR_DEVICE, MSH_ERR_STATE, 
 MSH_MARCHING_CUBES, MSH_MARCHING_TETRAHEDRA, MSH_NAIVE_SURFACE_NETS = range(3)
 MSH_INT64, MSH_FLOAT32, MSH_FLOAT64 = range(3)
 MSH_HOST, MSH_DEVICE = range(2)
+MSH_LIMIT_SAMPLE_BITS = 0
 
 # every symbol the header declares; checked by the CPU test suite
 EXPORTS = ("msh_create", "msh_destroy", "msh_set_stream", "msh_synchronize",
            "msh_last_error", "msh_output_kind", "msh_count", "msh_extract",
            "msh_batch_count", "msh_batch_extract", "msh_autotune", "msh_set_kernel_family",
            "msh_generate_field", "msh_weld", "msh_weld_to", "msh_isosurface_noalloc",
-           "msh_batch_graph_launches", "msh_autotune_batch")
+           "msh_batch_graph_launches", "msh_autotune_batch", "msh_set_limit")
 
 
 class MshField(ctypes.Structure):
@@ -100,6 +101,7 @@ def lib():
             L.msh_isosurface_noalloc.argtypes = [vp, pf, pp, vp, i64, vp, i64, vp]
             L.msh_batch_graph_launches.argtypes = [vp, ctypes.POINTER(i64), ctypes.POINTER(i64)]
             L.msh_autotune_batch.argtypes = [vp, i32, pf, pp, ctypes.POINTER(i32)]
+            L.msh_set_limit.argtypes = [vp, i32, i64]
             for name in EXPORTS:
                 f = getattr(L, name)
                 if name != "msh_last_error":

@@ -114,6 +114,7 @@ struct Ctx {
   // emit kernel family per (method, element type, size class), -1 = default
   // order; set by msh_autotune or msh_set_kernel_family
   int family[3][3][kSizeClasses];
+  int64_t bits_limit = -1;  // msh_set_limit: bytes for sample bits, negative: any
   Ctx() {
     for (auto& m : family)
       for (auto& t : m)
@@ -460,6 +461,15 @@ int make_plan(Ctx* c, const msh_field* f, const msh_params* p, Plan* out) {
   return msh::make_plan(c ? &c->err : nullptr, f, p, out);
 }
 
+// What a batch's launches are derived from besides the arguments, the kernel
+// family choices and the buffers' addresses: which kernels the call takes
+// also depends on the room there was and on the limits (two layouts of one
+// batch may meet at one address, one after the other).
+void key_layout(std::vector<char>* k, const Ctx* c, int64_t units) {
+  const int64_t v[4] = {c->batch.rows, units, (int64_t)c->ws_bytes, (int64_t)c->bws_bytes};
+  key_add(k, v, 4);
+}
+
 int grow(Ctx* c, void** buf, size_t* have, size_t need, const char* what) {
   if (need <= *have) return MSH_OK;
   if (*buf) {
@@ -477,7 +487,8 @@ int grow(Ctx* c, void** buf, size_t* have, size_t need, const char* what) {
   return MSH_OK;
 }
 
-// extra: room for the sample bits of the row kernels, at *bits
+// extra: room for the sample bits of the row kernels (and what goes with
+// them), at *bits
 int setup_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t extra = 0,
                     void** bits = nullptr) {
   const size_t need = workspace_layout(units, ncoords, nullptr, nullptr);
@@ -486,6 +497,17 @@ int setup_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t
   workspace_layout(units, ncoords, c->ws, w);
   if (bits) *bits = (char*)c->ws + need;
   return MSH_OK;
+}
+
+// Workspace with the sample bits of the row kernels; false, with no error
+// left, where they are not to take that much (msh_set_limit) or the device
+// has no room: the other kernels, which need less, take the call then.
+bool rows_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t extra, void** bits) {
+  if (c->bits_limit >= 0 && extra > (size_t)c->bits_limit) return false;
+  if (setup_workspace(c, units, ncoords, w, extra, bits) == MSH_OK) return true;
+  *bits = nullptr;
+  (void)hipGetLastError();
+  return false;
 }
 
 // The row kernels serve the default family and family 2.
@@ -639,15 +661,9 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
   RowsGeom rg{};
   Geom gr = g;
   void* bits = nullptr;
-  if (rows_family(pl) && rows_geom(pl, &gr, &rg) && rows_single(pl, gr)) {
-    // with no room for the sample bits the other kernels, which need less,
-    // take the volume
-    if (setup_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr),
-                        &bits) == MSH_OK)
-      g = gr;
-    else
-      (void)hipGetLastError();
-  }
+  if (rows_family(pl) && rows_geom(pl, &gr, &rg) && rows_single(pl, gr) &&
+      rows_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr), &bits))
+    g = gr;
   if (!bits) rc = setup_workspace(c, g.units, ncoords, &w);
   if (rc) return rc;
   int64_t nv = 0, nfc = 0;
@@ -845,13 +861,10 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
       runits += rgeoms[v].units;
       extra += rows_bytes(rgeoms[v], rows[v]);
     }
-    // (with no room for the sample bits the other kernels take the batch)
     extra += align256((size_t)runits * 64 * sizeof(uint16_t));
-    if (setup_workspace(c, runits, ncoords, &w, extra, &bits) == MSH_OK) {
+    if (rows_workspace(c, runits, ncoords, &w, extra, &bits)) {
       units = runits;
       geoms = rgeoms;
-    } else {
-      (void)hipGetLastError();
     }
   }
   b.rows = bits != nullptr;
@@ -1033,13 +1046,14 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     return e;
   };
   // everything the launches and copies above are derived from: the
-  // arguments, the kernel family choices and the buffers
+  // arguments, the kernel family choices, the buffers and the layout in them
   std::vector<char> key;
   key_add(&key, fields, (size_t)n);
   key_add(&key, params, (size_t)n);
   key_add(&key, &c->family[0][0][0], 9 * kSizeClasses);
   const void* bufs[5] = {c->ws, c->bws, c->hbatch, c->fstage, (const void*)c->stream};
   key_add(&key, bufs, 5);
+  key_layout(&key, c, units);
   hipError_t e = run_phase(c, &c->gcount, std::move(key), !host_fields && c->stream != nullptr,
                            enqueue);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1137,6 +1151,7 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
   const void* bufs[5] = {c->ws, c->bws, c->hbatch, (const void*)c->stream,
                          (const void*)c->upload};
   key_add(&key, bufs, 5);
+  key_layout(&key, c, b.units);
   hipError_t e = run_phase(c, &c->gemit, std::move(key),
                            out_memory == MSH_DEVICE && c->stream != nullptr, enqueue);
   if (e == hipSuccess) c->upload_pending = true;
@@ -1168,6 +1183,16 @@ int msh_set_kernel_family(void* ctx, int32_t method, int32_t dtype, int32_t fami
       family > 3)
     return fail(c, MSH_ERR_ARGUMENT, "method, dtype or kernel family out of range");
   for (int& f : c->family[method][dtype]) f = family;
+  c->have = false;
+  c->batch.have = false;
+  return MSH_OK;
+}
+
+int msh_set_limit(void* ctx, int32_t what, int64_t value) {
+  Ctx* c = (Ctx*)ctx;
+  if (!c) return MSH_ERR_ARGUMENT;
+  if (what != MSH_LIMIT_SAMPLE_BITS) return fail(c, MSH_ERR_ARGUMENT, "unknown limit");
+  c->bits_limit = value;
   c->have = false;
   c->batch.have = false;
   return MSH_OK;

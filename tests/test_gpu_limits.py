@@ -1,0 +1,54 @@
+"""Calls that go from the row kernels to the others and back because of the room
+for the sample bits, at the same buffers: the meshes stay those of the
+oracle.  Exact."""
+import numpy as np
+import pytest
+
+from helpers import assert_same_mesh, dev_field, noise
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def set_limit(pkg):
+    from importlib import import_module
+    capi = import_module(pkg.__name__ + "._capi")
+    ctx = capi.context(0)
+
+    def set_to(what, value):
+        with ctx.lock:
+            ctx.check(capi.lib().msh_set_limit(ctx.handle, what, value))
+
+    yield set_to
+    set_to(capi.MSH_LIMIT_SAMPLE_BITS, -1)
+
+
+def test_unknown_limit_is_refused(set_limit):
+    with pytest.raises(ValueError):
+        set_limit(9, 0)
+
+
+def test_repeated_batch_changes_kernels(pkg, oracle, set_limit):
+    # the same batch by the row kernels, then with no room for their bits,
+    # then with room again, each often enough to be captured and replayed;
+    # the workspaces keep their addresses (they only grow)
+    import torch
+    shapes = [(33, 34, 35), (20, 50, 70), (64, 9, 40), (2, 3, 130)]
+    names = ["mc", "mt", "sn", "mc"]
+    methods = [pkg.MarchingCubes(iso=0), pkg.MarchingTetrahedra(iso=0), pkg.NaiveSurfaceNets(iso=0),
+               pkg.MarchingCubes(iso=0)]
+    host = [noise(s, i, np.float32 if i % 2 else np.float64) for i, s in enumerate(shapes)]
+    want = [oracle.isosurface(f, n, iso=0) for f, n in zip(host, names)]
+    fields = [dev_field(f) for f in host]
+    stream = torch.cuda.Stream()  # (the null stream is never captured)
+    torch.cuda.synchronize()
+    for limit in (-1, 0, -1, 0):
+        set_limit(0, limit)
+        for rep in range(4):
+            with torch.cuda.stream(stream):
+                res = pkg.isosurface_batch(fields, methods)
+            stream.synchronize()
+            for (V, F), (Vo, Fo) in zip(res, want):
+                assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
+            del res
+            torch.cuda.synchronize()
