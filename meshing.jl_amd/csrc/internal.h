@@ -173,7 +173,8 @@ struct CoordArgs {
 CoordArgs coord_args(const Plan& p, const Geom& g, double* coords);
 
 // The row kernels (rows.h): Geom::units in their units, and the layout of
-// the sample bits; false when they do not take the volume.
+// the sample bits; false when they do not take the volume (its sizes, or axes
+// without finite ends in surface nets).
 struct RowsGeom {
   int64_t xs;
   int32_t sw, cw, upx;

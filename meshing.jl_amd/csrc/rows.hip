@@ -3,6 +3,7 @@
 // unit from the bits.  Their scan is the one of the other kernels
 // (kernels.hip) over these units.
 #include <algorithm>
+#include <cmath>
 
 #include "rows.h"
 
@@ -339,6 +340,11 @@ bool rows_geom(const Plan& p, Geom* g, RowsGeom* r) {
   // (a cell owns at most 13)
   if (p.method != MC && (int64_t)(g->ny + 1) * g->nz * (p.method == MT ? 13 : 1) >= (1ll << 31))
     return false;
+  // the surface nets emit leaves p + mu (p - p) out for a finite p
+  // (rows_sn.hip): every coordinate is finite between ends of this size
+  if (p.method == SN)
+    for (int k = 0; k < 3; ++k)
+      if (!(std::fabs(p.a[k]) <= 0x1p1022 && std::fabs(p.b[k]) <= 0x1p1022)) return false;
   r->upx = (int32_t)((words + 63) / 64);
   r->xs = (plane + 31) / 32 * 32;
   const int64_t units = (int64_t)(g->nx - 1) * r->upx;

@@ -136,7 +136,8 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
         if (((r.cs >> ca) ^ (r.cs >> cb)) & 1) {
           const M mu = (iso - (M)v[ca]) / (M)(v[cb] - v[ca]);
           // along an axis on which the edge's ends agree p1 + mu * (p2 - p1)
-          // is the end itself, or NaN where mu is not finite
+          // is the end itself, or NaN where mu is not finite (an infinite
+          // end would make it NaN too: rows_geom takes finite ones only)
           const double nz = (double)(mu * (M)0);
           const int ax = ca ^ cb;  // 1, 2, 4: the edge's axis
           const double qx = ax == 1 ? lerp_axis<M>(cx32, mu, px[ca & 1], px[cb & 1]) : px[ca & 1] + nz;

@@ -1,6 +1,6 @@
-"""Calls that go from the row kernels to the others and back because of the room
-for the sample bits, at the same buffers: the meshes stay those of the
-oracle.  Exact."""
+"""Which kernels a call takes: from the row kernels to the others and back because
+of the room for the sample bits, at the same buffers, and because of the axes;
+the meshes stay those of the oracle.  Exact."""
 import numpy as np
 import pytest
 
@@ -52,3 +52,23 @@ def test_repeated_batch_changes_kernels(pkg, oracle, set_limit):
                 assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
             del res
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("limit", [-1, 0])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("name", ["mc", "mt", "sn"])
+def test_axes_without_finite_ends(pkg, oracle, set_limit, name, dtype, limit):
+    # p + mu * (p - p) is NaN for an infinite p, whatever mu is
+    set_limit(0, limit)
+    m = {"mc": pkg.MarchingCubes(iso=0), "mt": pkg.MarchingTetrahedra(iso=0),
+         "sn": pkg.NaiveSurfaceNets(iso=0)}[name]
+    f = noise((9, 10, 40), 5, dtype)
+    inf, one, big = np.inf, (-1, 1), np.finfo(np.float64).max
+    for ax in (((-1.0, inf), one, one), (one, (-inf, 1.0), (np.float32(-1), np.float32(inf))),
+               (one, one, (np.nan, 1.0)), ((-big, big), one, (-inf, inf)),
+               ((np.float32(-3e38), np.float32(3e38)), one, one)):
+        Vo, Fo = oracle.isosurface(f, name, iso=0, X=ax[0], Y=ax[1], Z=ax[2])
+        V, F = pkg.isosurface(dev_field(f), m, *ax)
+        assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
+        (V, F), = pkg.isosurface_batch([dev_field(f)], m, [ax])
+        assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
