@@ -169,8 +169,11 @@ int msh_set_kernel_family(void* ctx, int32_t method, int32_t dtype, int32_t fami
  * sample, and for tetrahedra and surface nets 2 bytes per 32 cells);
  * negative, the default: no limit.  A call over it takes the other kernels,
  * as one does for whose bits the device has no room.
+ * MSH_LIMIT_WELD_INDEX32: the most vertices that msh_weld welds with 32-bit
+ * indices in its workspace; 2^31 by default and at most (also for a negative
+ * value).  A larger mesh takes 64-bit ones.
  * No counterpart in the reference. */
-typedef enum { MSH_LIMIT_SAMPLE_BITS = 0 } msh_limit;
+typedef enum { MSH_LIMIT_SAMPLE_BITS = 0, MSH_LIMIT_WELD_INDEX32 = 1 } msh_limit;
 int msh_set_limit(void* ctx, int32_t what, int64_t value);
 
 /* Vertex welding, the opt-in step after extraction: vertices whose three

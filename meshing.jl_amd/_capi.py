@@ -15,7 +15,7 @@ MSH_OK, MSH_ERR_ARGUMENT, MSH_ERR_OUT_OF_MEMORY, MSH_ERR_DEVICE, MSH_ERR_STATE, 
 MSH_MARCHING_CUBES, MSH_MARCHING_TETRAHEDRA, MSH_NAIVE_SURFACE_NETS = range(3)
 MSH_INT64, MSH_FLOAT32, MSH_FLOAT64 = range(3)
 MSH_HOST, MSH_DEVICE = range(2)
-MSH_LIMIT_SAMPLE_BITS = 0
+MSH_LIMIT_SAMPLE_BITS, MSH_LIMIT_WELD_INDEX32 = range(2)
 
 # every symbol the header declares; checked by the CPU test suite
 EXPORTS = ("msh_create", "msh_destroy", "msh_set_stream", "msh_synchronize",

@@ -115,6 +115,7 @@ struct Ctx {
   // order; set by msh_autotune or msh_set_kernel_family
   int family[3][3][kSizeClasses];
   int64_t bits_limit = -1;  // msh_set_limit: bytes for sample bits, negative: any
+  int64_t weld32 = kWeldIndex32;  // .. vertices welded with 32-bit indices
   Ctx() {
     for (auto& m : family)
       for (auto& t : m)
@@ -1191,8 +1192,12 @@ int msh_set_kernel_family(void* ctx, int32_t method, int32_t dtype, int32_t fami
 int msh_set_limit(void* ctx, int32_t what, int64_t value) {
   Ctx* c = (Ctx*)ctx;
   if (!c) return MSH_ERR_ARGUMENT;
-  if (what != MSH_LIMIT_SAMPLE_BITS) return fail(c, MSH_ERR_ARGUMENT, "unknown limit");
-  c->bits_limit = value;
+  if (what == MSH_LIMIT_SAMPLE_BITS)
+    c->bits_limit = value;
+  else if (what == MSH_LIMIT_WELD_INDEX32)
+    c->weld32 = value < 0 || value > kWeldIndex32 ? kWeldIndex32 : value;
+  else
+    return fail(c, MSH_ERR_ARGUMENT, "unknown limit");
   c->have = false;
   c->batch.have = false;
   return MSH_OK;
@@ -1485,7 +1490,7 @@ int msh_weld_to(void* ctx, int32_t kind, int64_t nverts, const void* verts, int6
   while (nslots < nverts + nverts / 4 + 1) nslots <<= 1;
   const int64_t U = nverts > 0 ? nverts : 1;
   const int64_t T = (U + 4095) / 4096;
-  const size_t isz = weld_index_bytes(nverts);
+  const size_t isz = nverts <= c->weld32 ? 4 : 8;
   const size_t b_idx = align256((size_t)U * isz), b_slot = align256((size_t)U * 4);
   const size_t b_lrep = align256((size_t)U * 2);
   const size_t b_tcnt = align256((size_t)(T + 1) * 4), b_toff = align256((size_t)T * 8);
@@ -1522,6 +1527,7 @@ int msh_weld_to(void* ctx, int32_t kind, int64_t nverts, const void* verts, int6
   a.faces = faces;
   a.faces_out = faces_out;
   a.nslots = nslots;
+  a.index_bytes = (int)isz;
   hipError_t e = launch_weld(a, c->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(c->pinned, sizes, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);

@@ -248,6 +248,7 @@ hipError_t launch_emit_batch(const Plan& p, int variant, const VolArgs* vols,
 // Zero n 32-bit words (the work-queue counters) with a kernel.
 hipError_t launch_zero_u32(uint32_t* p, int64_t n, hipStream_t st);
 // Exact-coordinate vertex welding (weld.hip).
+constexpr int64_t kWeldIndex32 = (int64_t)1 << 31;  // vertices that 32-bit indices serve
 struct WeldArgs {
   int out_kind;          // K_F32 or K_F64: element type of the coordinates
   int64_t nverts, nfaces;
@@ -255,7 +256,8 @@ struct WeldArgs {
   void* verts_out;       // welded vertices, room for nverts x 3
   const int64_t* faces;  // nfaces x 3, 1-based
   int64_t* faces_out;    // renumbered (may be faces itself)
-  int64_t* table;        // hash slots: a power of two >= 1.25 nverts, weld_index_bytes each
+  int index_bytes;       // of a vertex index below: 4 (up to kWeldIndex32 vertices) or 8
+  int64_t* table;        // hash slots: a power of two >= 1.25 nverts, an index each
   int64_t nslots;
   uint64_t* bounds;      // room for 63 x-region bounds of a large table
   void* rep;             // nverts indices: the vertex's first appearance
@@ -267,8 +269,6 @@ struct WeldArgs {
   int64_t* total;        // welded count
   int64_t* bad;          // count of face indices outside 1..nverts
 };
-// bytes of a vertex index in the weld's workspace
-size_t weld_index_bytes(int64_t nverts);
 hipError_t launch_weld(const WeldArgs& a, hipStream_t st);
 
 hipError_t launch_generate(int kind, int dtype, int64_t nx, int64_t ny, int64_t nz,

@@ -433,10 +433,8 @@ hipError_t weld_t(const WeldArgs& a, hipStream_t st) {
 
 }  // namespace
 
-size_t weld_index_bytes(int64_t nverts) { return nverts <= ((int64_t)1 << 31) ? 4 : 8; }
-
 hipError_t launch_weld(const WeldArgs& a, hipStream_t st) {
-  const bool narrow = weld_index_bytes(a.nverts) == 4;
+  const bool narrow = a.index_bytes == 4;
   if (a.out_kind == K_F32)
     return narrow ? weld_t<uint32_t, uint32_t>(a, st) : weld_t<uint32_t, uint64_t>(a, st);
   return narrow ? weld_t<uint64_t, uint32_t>(a, st) : weld_t<uint64_t, uint64_t>(a, st);
