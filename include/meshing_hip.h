@@ -191,7 +191,7 @@ int msh_set_limit(void* ctx, int32_t what, int64_t value);
 int msh_weld(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t nfaces,
              int64_t* faces, void* verts_out, int64_t* nunique);
 /* msh_weld with the renumbered faces written to faces_out instead (room for
- * nfaces x 3; faces itself, or apart from it); faces outside 1..nverts are
+ * nfaces x 3; faces itself, or apart from it: MSH_ERR_ARGUMENT otherwise); faces outside 1..nverts are
  * copied as they are. */
 int msh_weld_to(void* ctx, int32_t kind, int64_t nverts, const void* verts, int64_t nfaces,
                 const int64_t* faces, int64_t* faces_out, void* verts_out, int64_t* nunique);

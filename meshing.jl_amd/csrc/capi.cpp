@@ -1480,6 +1480,10 @@ int msh_weld_to(void* ctx, int32_t kind, int64_t nverts, const void* verts, int6
   if (nverts > 0 && (const char*)verts_out < (const char*)verts + vbytes &&
       (const char*)verts < (const char*)verts_out + vbytes)
     return fail(c, MSH_ERR_ARGUMENT, "verts_out overlaps verts");
+  const size_t fbytes = (size_t)nfaces * 3 * sizeof(int64_t);
+  if (faces_out != faces && (const char*)faces_out < (const char*)faces + fbytes &&
+      (const char*)faces < (const char*)faces_out + fbytes)
+    return fail(c, MSH_ERR_ARGUMENT, "faces_out overlaps faces without being faces");
   // hash slots are noted as 32-bit numbers: at most 2^32 slots
   if (nverts > ((int64_t)3 << 30) || nfaces > (int64_t)1 << 40)
     return fail(c, MSH_ERR_ARGUMENT, "mesh too large (at most 3 * 2^30 vertices)");
