@@ -120,11 +120,10 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
  * stream other than the null stream) runs each phase from a hipGraph: the
  * second such call captures the phase's copies and launches, later calls
  * replay it (new output pointers travel through the descriptor copy, so
- * they may change).  A batch whose volumes all take the row kernels runs them
- * with a block per tile; in any other, the count and emit kernels are
- * persistent: as many blocks as fit on the device take the batch's tiles
- * from a work queue.  msh_batch_graph_launches reports how many times each phase has run
- * from a graph on this context.  No counterpart in the reference. */
+ * they may change).  The row kernels run with a block per tile; the other count
+ * and emit kernels of a batch are persistent: as many blocks as fit on the
+ * device take the tiles from a work queue.  msh_batch_graph_launches reports
+ * how many times each phase has run from a graph on this context.  No counterpart in the reference. */
 int msh_batch_graph_launches(void* ctx, int64_t* count_phase, int64_t* emit_phase);
 
 /* Kernel choice.  There are kernel families per method: 2 the row kernels

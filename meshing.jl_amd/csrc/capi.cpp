@@ -30,6 +30,7 @@ namespace {
 struct Launch {
   Plan plan;                // types (and method) of the group
   int variant = 0;          // emit variant (emit launches only)
+  bool rows = false;        // of the row kernels: a block per tile, no work queue
   int64_t gbase = 0;        // first block in the block -> volume map
   int64_t nblocks = 0;
   double cost = 0;          // estimated work: cells weighted by method
@@ -49,6 +50,10 @@ double cell_cost(const VolArgs& v, const Plan& p, bool emit) {
 
 // Launch order for spreading: most work first (each goes to the stream with
 // the least work so far, so the short launches fill in at the end).
+bool work_queues(const std::vector<Launch>& ls) {
+  return std::any_of(ls.begin(), ls.end(), [](const Launch& l) { return !l.rows; });
+}
+
 std::vector<size_t> by_cost(const std::vector<Launch>& ls) {
   std::vector<size_t> o(ls.size());
   for (size_t i = 0; i < o.size(); ++i) o[i] = i;
@@ -75,7 +80,7 @@ struct BatchState {
   std::vector<Plan> plans;
   std::vector<VolArgs> vols;       // host copy of the device descriptors
   std::vector<Launch> bits, counts, emits;  // bits: sample-bit launches of the row kernels
-  bool rows = false;               // every volume goes through the row kernels
+  std::vector<char> rows;          // per volume: goes through the row kernels
   std::vector<int64_t> sizes;      // 4 per volume: first vertex, nverts, first face, nfaces
   int64_t units = 0, ncoords = 0, cblocks = 0, eblocks = 0, bblocks = 0;
   size_t ctr_off = 0;              // work-queue counters in the batch workspace: 8 per
@@ -467,8 +472,9 @@ int make_plan(Ctx* c, const msh_field* f, const msh_params* p, Plan* out) {
 // also depends on the room there was and on the limits (two layouts of one
 // batch may meet at one address, one after the other).
 void key_layout(std::vector<char>* k, const Ctx* c, int64_t units) {
-  const int64_t v[4] = {c->batch.rows, units, (int64_t)c->ws_bytes, (int64_t)c->bws_bytes};
-  key_add(k, v, 4);
+  const int64_t v[3] = {units, (int64_t)c->ws_bytes, (int64_t)c->bws_bytes};
+  key_add(k, v, 3);
+  key_add(k, c->batch.rows.data(), c->batch.rows.size());
 }
 
 int grow(Ctx* c, void** buf, size_t* have, size_t need, const char* what) {
@@ -818,11 +824,11 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   if (rc) return rc;
   b.plans.assign((size_t)n, Plan{});
   std::vector<Geom> geoms((size_t)n);
-  // the row kernels take the batch when they take every volume of it (its
-  // units are scanned together)
+  // each volume by the row kernels, or not: the scan takes units of both
+  // kinds in one sequence
   std::vector<Geom> rgeoms((size_t)n);
   std::vector<RowsGeom> rows((size_t)n);
-  b.rows = true;
+  b.rows.assign((size_t)n, 0);
   for (int v = 0; v < n; ++v) {
     rc = make_plan(c, &fields[v], &params[v], &b.plans[v]);
     if (rc) {
@@ -834,8 +840,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (geoms[v].units > 0 && !fields[v].data)
       return fail(c, MSH_ERR_ARGUMENT, "volume " + std::to_string(v) + ": null field data");
     rgeoms[v] = geoms[v];
-    if (geoms[v].units > 0)
-      b.rows = b.rows && rows_family(b.plans[v]) && rows_geom(b.plans[v], &rgeoms[v], &rows[v]);
+    b.rows[v] = rows_family(b.plans[v]) && rows_geom(b.plans[v], &rgeoms[v], &rows[v]);
   }
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, MSH_ERR_DEVICE, "hipSetDevice");
 
@@ -854,21 +859,20 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   }
   Workspace w{};
   void* bits = nullptr;
-  if (b.rows && units > 0) {
-    int64_t runits = 0;
-    size_t extra = 0;
-    for (int v = 0; v < n; ++v) {
-      if (geoms[v].units == 0) continue;
-      runits += rgeoms[v].units;
-      extra += rows_bytes(rgeoms[v], rows[v]);
-    }
-    extra += align256((size_t)runits * 64 * sizeof(uint16_t));
-    if (rows_workspace(c, runits, ncoords, &w, extra, &bits)) {
-      units = runits;
-      geoms = rgeoms;
-    }
+  int64_t runits = units;
+  size_t extra = 0;
+  for (int v = 0; v < n; ++v) {
+    if (!b.rows[v]) continue;
+    runits += rgeoms[v].units - geoms[v].units;
+    extra += rows_bytes(rgeoms[v], rows[v]) + rows_prefix_bytes(b.plans[v], rgeoms[v]);
   }
-  b.rows = bits != nullptr;
+  if (extra > 0 && rows_workspace(c, runits, ncoords, &w, extra, &bits)) {
+    units = runits;
+    for (int v = 0; v < n; ++v)
+      if (b.rows[v]) geoms[v] = rgeoms[v];
+  } else {
+    b.rows.assign((size_t)n, 0);
+  }
   if (!bits) rc = setup_workspace(c, units, ncoords, &w);
   if (rc) return rc;
   if (hbytes) {
@@ -881,8 +885,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   b.vols.assign((size_t)n, VolArgs{});
   std::vector<int> emit_var((size_t)n, 0);
   int64_t ubase = 0, cbase = 0;
-  uint16_t* wpre = (uint16_t*)bits;
-  char* vbits = (char*)bits + align256((size_t)units * 64 * sizeof(uint16_t));
+  char* vbits = (char*)bits;
   for (int v = 0; v < n; ++v) {
     const void* df = fields[v].data;
     if (fields[v].memory == MSH_HOST && geoms[v].units > 0) df = (char*)c->fstage + hoff[v];
@@ -892,10 +895,11 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     a.ubase = ubase;
     a.sz = nullptr;  // set below, once the sizes array is placed
     emit_var[v] = emit_variant(b.plans[v], &a);
-    if (bits && geoms[v].units > 0) {
+    if (b.rows[v]) {
+      char* const wpre = vbits + rows_bytes(geoms[v], rows[v]);
       rows_vol(rows[v], vbits, wpre, &a);
       rows_emit_tiling(&a, -1);
-      vbits += rows_bytes(geoms[v], rows[v]);
+      vbits = wpre + rows_prefix_bytes(b.plans[v], geoms[v]);
       emit_var[v] = kRowsVariant + cx_class(a);
     }
     if (geoms[v].units == 0) {
@@ -919,29 +923,30 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
                    [&](int x, int y) { return geoms[x].nz > geoms[y].nz; });
   std::vector<char> done((size_t)n, 0);
   int64_t bblocks = 0;
-  if (b.rows)
-    for (int T : {(int)K_F32, (int)K_F64}) {
-      Launch L;
-      L.plan.T = T;
-      L.gbase = bblocks;
-      for (int u : ord) {
-        if (b.plans[u].T != T) continue;
-        b.vols[u].bblk0 = bblocks;
-        bblocks += b.vols[u].bntiles;
-      }
-      L.nblocks = bblocks - L.gbase;
-      L.cost = (double)L.nblocks * (T == K_F64 ? 2.0 : 1.0);
-      if (L.nblocks) b.bits.push_back(L);
+  for (int T : {(int)K_F32, (int)K_F64}) {
+    Launch L;
+    L.plan.T = T;
+    L.gbase = bblocks;
+    for (int u : ord) {
+      if (!b.rows[u] || b.plans[u].T != T) continue;
+      b.vols[u].bblk0 = bblocks;
+      bblocks += b.vols[u].bntiles;
     }
+    L.nblocks = bblocks - L.gbase;
+    L.cost = (double)L.nblocks * (T == K_F64 ? 2.0 : 1.0);
+    if (L.nblocks) b.bits.push_back(L);
+  }
   int64_t cblocks = 0;
   for (int v : ord) {
     if (done[v]) continue;
     Launch L;
     L.plan = b.plans[v];
+    L.rows = b.rows[v];
     L.gbase = cblocks;
     for (int u : ord) {
       // (the row kernels count from the bits, whatever the element type)
-      if (done[u] || (!b.rows && b.plans[u].T != L.plan.T) || b.plans[u].method != L.plan.method)
+      if (done[u] || b.rows[u] != b.rows[v] || b.plans[u].method != L.plan.method ||
+          (!L.rows && b.plans[u].T != L.plan.T))
         continue;
       done[u] = 1;
       b.vols[u].cblk0 = cblocks;
@@ -958,6 +963,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     Launch L;
     L.plan = b.plans[v];
     L.variant = emit_var[v];
+    L.rows = b.rows[v];
     L.gbase = eblocks;
     for (int u : ord) {
       if (done[u] || emit_var[u] != L.variant || !same_plan_types(b.plans[u], L.plan)) continue;
@@ -976,7 +982,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   const size_t b_vols = align256(sizeof(VolArgs) * (size_t)(n > 0 ? n : 1));
   const size_t b_cmap = align256(4 * (size_t)(cblocks + 1));
   const size_t b_emap = align256(4 * (size_t)(eblocks + 1));
-  const size_t b_bmap = b.rows ? align256(4 * (size_t)(bblocks + 1)) : 0;
+  const size_t b_bmap = bits ? align256(4 * (size_t)(bblocks + 1)) : 0;
   const size_t b_sizes = align256(32 * (size_t)(n > 0 ? n : 1));
   const size_t nctr = 8 * (b.counts.size() + b.emits.size());
   const size_t b_ctr = align256(4 * (nctr + 1));
@@ -989,7 +995,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   int64_t* dsizes = (int64_t*)((char*)emap + b_emap);
   b.ctr_off = b_vols + b_cmap + b_emap + b_sizes;
   uint32_t* ctrs = (uint32_t*)((char*)c->bws + b.ctr_off);
-  int32_t* bmap = b.rows ? (int32_t*)((char*)ctrs + b_ctr) : nullptr;
+  int32_t* bmap = bits ? (int32_t*)((char*)ctrs + b_ctr) : nullptr;
   for (int v = 0; v < n; ++v) b.vols[v].sz = dsizes + 4 * v;
   // pinned host side: descriptors | sizes
   if (c->hbatch_bytes < b_vols + b_sizes) {
@@ -1018,7 +1024,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
                          c->stream);
     if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, c->stream);
     if (e == hipSuccess) e = launch_coords_batch(dvols, n, c->stream);
-    if (e == hipSuccess && !b.rows)
+    if (e == hipSuccess && work_queues(b.counts))
       e = launch_zero_u32(ctrs, (int64_t)(8 * b.counts.size()), c->stream);
     for (const Launch& L : b.bits)
       if (e == hipSuccess)
@@ -1027,7 +1033,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess) e = sp.start((int)b.counts.size());
     for (size_t k : by_cost(b.counts)) {
       if (e != hipSuccess) break;
-      if (b.rows)
+      if (b.counts[k].rows)
         e = launch_rows_count_batch(b.counts[k].plan.method,
                                     RowsBatch{dvols, cmap, b.counts[k].gbase, b.counts[k].nblocks},
                                     sp.next(b.counts[k].cost));
@@ -1132,7 +1138,7 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
     hipError_t e = hipMemcpyAsync(dvols, c->hbatch, sizeof(VolArgs) * (size_t)n,
                                   hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipEventRecord(c->upload, c->stream);
-    if (e == hipSuccess && !b.rows)
+    if (e == hipSuccess && work_queues(b.emits))
       e = launch_zero_u32(ectr, (int64_t)(8 * b.emits.size()), c->stream);
     Spread sp{c};
     if (e == hipSuccess) e = sp.start((int)b.emits.size());
@@ -1411,23 +1417,6 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
     float cur = 0.f;
     bool took = true;
     rc = time_all(-1, 0, &cur, &took);
-    // the row kernels take a batch only as a whole: every group on them
-    if (rc == MSH_OK && !no_room && std::any_of(best.begin(), best.end(), [](int f) { return f != 2; })) {
-      auto set_all = [&](bool rows) {
-        for (size_t g = 0; g < gkey.size(); ++g)
-          c->family[gkey[g] / (3 * kSizeClasses)][(gkey[g] / kSizeClasses) % 3][gkey[g] % kSizeClasses] =
-              rows ? 2 : best[g];
-      };
-      set_all(true);
-      float ms = 0.f;
-      rc = time_all(-1, 2, &ms, &took);
-      if (rc == MSH_OK && !no_room && ms < cur) {
-        std::fill(best.begin(), best.end(), 2);
-        cur = ms;
-      } else {
-        set_all(false);
-      }
-    }
     // (with no room for the whole batch there is nothing to compare against)
     std::vector<size_t> gord(rc == MSH_OK && !no_room ? gkey.size() : 0);
     for (size_t g = 0; g < gord.size(); ++g) gord[g] = g;

@@ -95,8 +95,8 @@ struct VolArgs {
   int64_t cblk0;           // first count block of this volume in a batched launch
   // the row kernels (rows.h); bits is null for the other kernels
   uint32_t* bits;          // sample bits, 32 samples along z a word
-  uint16_t* wpre;          // per cell word of a unit: vertices before it in the unit
-                           // (tetrahedra and surface nets), from ubase
+  uint16_t* wpre;          // per cell word of the volume's units: vertices before it
+                           // in the unit (tetrahedra and surface nets)
   int64_t xs;              // words of an x plane
   int32_t sw, cw;          // words of a column of samples, of a row of cells
   int32_t upx;             // units of an x plane

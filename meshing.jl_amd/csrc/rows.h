@@ -207,7 +207,7 @@ __device__ __forceinline__ uint32_t active_of(const Col& a, const Col& b, const 
 // First vertex (in the volume's numbering) of cell word q of x plane x.
 __device__ __forceinline__ int64_t word_vertex(const VolArgs& a, int x, uint32_t q) {
   const int64_t u = (int64_t)x * a.upx + (q >> 6);
-  return a.voff[a.ubase + u] + (int64_t)a.wpre[64 * (a.ubase + u) + (q & 63)];
+  return a.voff[a.ubase + u] + (int64_t)a.wpre[64 * u + (q & 63)];
 }
 
 static_assert(rows_emit_waves(MC) == kWaves && rows_emit_waves(MT) == kWaves, "their blocks");

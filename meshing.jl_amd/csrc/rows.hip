@@ -229,7 +229,7 @@ __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, con
     const uint32_t incl = wave_scan_dpp(n);
     if (lane == kWave - 1) cnt[u] = incl;
     if constexpr (METHOD != MC)
-      a.wpre[64 * (a.ubase + u) + lane] = (uint16_t)((incl - n) & 0xFFFF);
+      a.wpre[64 * (int64_t)u + lane] = (uint16_t)((incl - n) & 0xFFFF);
   }
 }
 

@@ -453,7 +453,7 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
       {
         const uint32_t q = (uint32_t)gi * 64u + (uint32_t)lane, cw = (uint32_t)a.cw;
         if (act != 0) {
-          pre = a.wpre[64 * (a.ubase + (int64_t)x * a.upx + gi) + lane];
+          pre = a.wpre[64 * ((int64_t)x * a.upx + gi) + lane];
           const int64_t mine = readlane64(voff, gi - g0) + a.sz[0] + (int64_t)pre;
           if (x > 0) w10 = (uint32_t)(mine - word_vertex(a, x - 1, q));
           if (y > 0) w01 = (uint32_t)(mine - word_vertex(a, x, q - cw));

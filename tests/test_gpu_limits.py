@@ -72,3 +72,31 @@ def test_axes_without_finite_ends(pkg, oracle, set_limit, name, dtype, limit):
         assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
         (V, F), = pkg.isosurface_batch([dev_field(f)], m, [ax])
         assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
+
+
+def test_families_mix_in_a_batch(pkg, oracle):
+    # each volume of a batch runs its own class's family: the row kernels for
+    # some, every other family beside them, and a volume nothing crosses
+    import torch
+    make = {"mc": pkg.MarchingCubes, "mt": pkg.MarchingTetrahedra, "sn": pkg.NaiveSurfaceNets}
+    types = [(n, t) for n in make for t in ("float32", "float64")]
+    host = [noise((20 + 3 * i, 33 + i, 30 + 7 * i), i, t) for i, (n, t) in enumerate(types * 2)]
+    host.append(np.ones((9, 8, 70), np.float32))
+    names = [n for n, _ in types * 2] + ["mt"]
+    fields, methods = [dev_field(f) for f in host], [make[n](iso=0) for n in names]
+    want = [oracle.isosurface(f, n, iso=0) for f, n in zip(host, names)]
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    try:
+        for shift in range(4):
+            for i, (n, t) in enumerate(types):
+                pkg.set_kernel_family(make[n](iso=0), t, [-1, 0, 2, 1, -1, 3][(i + shift) % 6])
+            for rep in range(3):
+                with torch.cuda.stream(stream):
+                    res = pkg.isosurface_batch(fields, methods)
+                stream.synchronize()
+                for (V, F), (Vo, Fo) in zip(res, want):
+                    assert_same_mesh(V.cpu().numpy(), F.cpu().numpy(), Vo, Fo)
+    finally:
+        for n, t in types:
+            pkg.set_kernel_family(make[n](iso=0), t, -1)
