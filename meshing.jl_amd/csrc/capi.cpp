@@ -34,6 +34,10 @@ struct Launch {
   int64_t gbase = 0;        // first block in the block -> volume map
   int64_t nblocks = 0;
   double cost = 0;          // estimated work: cells weighted by method
+  // emits of the row kernels: the launch's shared units (RowsGroup)
+  RowsGroup* groups = nullptr;
+  uint32_t* ngroups = nullptr;
+  int32_t xblocks = 0;
 };
 
 // Estimated work of a volume in a batched launch, for spreading the launches
@@ -82,6 +86,7 @@ struct BatchState {
   std::vector<Launch> bits, counts, emits;  // bits: sample-bit launches of the row kernels
   std::vector<char> rows;          // per volume: goes through the row kernels
   std::vector<int64_t> sizes;      // 4 per volume: first vertex, nverts, first face, nfaces
+  std::vector<uint32_t> ngroups;   // per emit launch: groups of shared units
   int64_t units = 0, ncoords = 0, cblocks = 0, eblocks = 0, bblocks = 0;
   size_t ctr_off = 0;              // work-queue counters in the batch workspace: 8 per
                                    // count launch, then 8 per emit launch
@@ -523,10 +528,12 @@ bool rows_family(const Plan& p) { return p.family < 0 || p.family == 2; }
 // By default a single volume goes to them from a number of units on in
 // Marching Tetrahedra, whose waves are the longest: with few units a dense
 // one leaves most of the device idle, where the tiles of the lanes-along-x
-// kernel are smaller (value noise, whole call: 110 x 100 x 120 Float32, 763
-// units, 257 us by rows and 210 by lanes along x; 160^3 Float32, 2067 units,
-// 262 and 218; 165 x 160 x 170 Float64, 2460 units, 246 and 323; 180^3
-// Float32, 3043 units, 258 and 319).  The other methods gain at every size.
+// kernel are smaller (whole calls, lanes along x and by rows: value noise of
+// 128^3 Float32, 1016 units, 265 and 336 us, of 160^3, 2067 units, 229 and
+// 282; a gentle surface across x in 160^3 91 and 109; but 180^3 noise, 3043
+// units, 319 and 258).  Where the dense units are few, waves share them and
+// smaller volumes gain too (a 96^3 sphere 115 and 72 us); which these are is
+// known only after the count.
 bool rows_single(const Plan& p, const Geom& rows) {
   return p.method != MT || p.family == 2 || rows.units >= 2304;
 }
@@ -667,9 +674,11 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
   const int64_t ncoords = (int64_t)g.nx + g.ny + g.nz;
   RowsGeom rg{};
   Geom gr = g;
-  void* bits = nullptr;
+  void* bits = nullptr;  // sample bits | vertex prefixes | counter of shared units | their groups
   if (rows_family(pl) && rows_geom(pl, &gr, &rg) && rows_single(pl, gr) &&
-      rows_workspace(c, gr.units, ncoords, &w, rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr), &bits))
+      rows_workspace(c, gr.units, ncoords, &w,
+                     rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr) + rows_groups_bytes(pl.method),
+                     &bits))
     g = gr;
   if (!bits) rc = setup_workspace(c, g.units, ncoords, &w);
   if (rc) return rc;
@@ -687,8 +696,15 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
       dfield = c->fstage;
     }
     VolArgs a = make_vol(pl, g, dfield, w);
-    if (bits) rows_vol(rg, bits, (char*)bits + rows_bytes(gr, rg), &a);
-    c->pinned[1] = c->pinned[3] = -1;
+    if (bits) {
+      char* const wpre = (char*)bits + rows_bytes(gr, rg);
+      char* const shared = wpre + rows_prefix_bytes(pl, gr);
+      rows_vol(rg, bits, wpre, &a);
+      a.ngroups = (uint32_t*)shared;
+      a.groups = (RowsGroup*)(shared + kGroupsAt);
+      a.gcap = rows_group_cap(pl.method);
+    }
+    c->pinned[0] = c->pinned[1] = c->pinned[3] = -1;
     const CoordArgs ca = coord_args(pl, g, w.coords);
     // a volume of one scan tile is scanned by the count's last block
     const bool tail = bits && g.units <= kScanTile;
@@ -698,9 +714,10 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
     // the scan also fills the coordinate tables and writes the sizes into
     // the pinned host words itself; a negative word afterwards (not
     // written) is read back by a copy
-    if (e == hipSuccess && !tail) e = launch_scan(g, w, c->stream, c->pinned, &ca);
+    if (e == hipSuccess && !tail) e = launch_scan(g, w, c->stream, c->pinned, &ca, bits ? &a : nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess && (c->pinned[1] < 0 || c->pinned[3] < 0)) {
+    if (e == hipSuccess && (c->pinned[0] < 0 || c->pinned[1] < 0 || c->pinned[3] < 0)) {
+      // (totals[0] is 0: no unit is shared then)
       e = hipMemcpyAsync(c->pinned, w.totals, 4 * sizeof(int64_t), hipMemcpyDeviceToHost,
                          c->stream);
       if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -708,7 +725,11 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
     if (e != hipSuccess) return hip_fail(c, e, "count/scan");
     nv = c->pinned[1];
     nfc = c->pinned[3];
-    if (bits) rows_emit_tiling(&a, nv);
+    if (bits) {
+      rows_emit_tiling(&a, nv);
+      a.shared = (uint32_t)c->pinned[0];
+      a.xblocks = rows_xblocks(a.shared, a.gcap);
+    }
     c->vol = a;
   }
   c->field = *f;
@@ -884,6 +905,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   // by the full instantiation (types + variant)
   b.vols.assign((size_t)n, VolArgs{});
   std::vector<int> emit_var((size_t)n, 0);
+  std::vector<size_t> emit_of((size_t)n, 0);  // emit launch
   int64_t ubase = 0, cbase = 0;
   char* vbits = (char*)bits;
   for (int v = 0; v < n; ++v) {
@@ -968,6 +990,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     for (int u : ord) {
       if (done[u] || emit_var[u] != L.variant || !same_plan_types(b.plans[u], L.plan)) continue;
       done[u] = 1;
+      emit_of[u] = b.emits.size();
       b.vols[u].eblk0 = eblocks;
       eblocks += b.vols[u].ntiles;
       L.cost += cell_cost(b.vols[u], b.plans[u], true);
@@ -978,15 +1001,19 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   if (cblocks > INT32_MAX || eblocks > INT32_MAX || bblocks > INT32_MAX)
     return fail(c, MSH_ERR_ARGUMENT, "batch too large for one launch");
 
-  // device side: descriptors | cmap | emap | sizes
+  // device side: descriptors | cmap | emap | sizes, numbers of groups of shared
+  // units | work queues | bmap | these groups
   const size_t b_vols = align256(sizeof(VolArgs) * (size_t)(n > 0 ? n : 1));
   const size_t b_cmap = align256(4 * (size_t)(cblocks + 1));
   const size_t b_emap = align256(4 * (size_t)(eblocks + 1));
   const size_t b_bmap = bits ? align256(4 * (size_t)(bblocks + 1)) : 0;
-  const size_t b_sizes = align256(32 * (size_t)(n > 0 ? n : 1));
+  const size_t b_sizes = align256(32 * (size_t)(n > 0 ? n : 1) + 4 * b.emits.size());
+  size_t b_groups = 0;
+  for (const Launch& L : b.emits)
+    if (L.rows) b_groups += rows_group_cap(L.plan.method) * sizeof(RowsGroup);
   const size_t nctr = 8 * (b.counts.size() + b.emits.size());
   const size_t b_ctr = align256(4 * (nctr + 1));
-  rc = grow(c, &c->bws, &c->bws_bytes, b_vols + b_cmap + b_emap + b_sizes + b_ctr + b_bmap,
+  rc = grow(c, &c->bws, &c->bws_bytes, b_vols + b_cmap + b_emap + b_sizes + b_ctr + b_bmap + b_groups,
             "batch workspace");
   if (rc) return rc;
   VolArgs* dvols = (VolArgs*)c->bws;
@@ -996,7 +1023,23 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   b.ctr_off = b_vols + b_cmap + b_emap + b_sizes;
   uint32_t* ctrs = (uint32_t*)((char*)c->bws + b.ctr_off);
   int32_t* bmap = bits ? (int32_t*)((char*)ctrs + b_ctr) : nullptr;
-  for (int v = 0; v < n; ++v) b.vols[v].sz = dsizes + 4 * v;
+  uint32_t* const ngroups = (uint32_t*)(dsizes + 4 * n);
+  RowsGroup* groups = (RowsGroup*)((char*)ctrs + b_ctr + b_bmap);
+  for (size_t k = 0; k < b.emits.size(); ++k) {
+    Launch& L = b.emits[k];
+    if (!L.rows) continue;
+    L.ngroups = ngroups + k;
+    L.groups = groups;
+    groups += rows_group_cap(L.plan.method);
+  }
+  for (int v = 0; v < n; ++v) {
+    b.vols[v].sz = dsizes + 4 * v;
+    b.vols[v].self = v;
+    if (!b.rows[v]) continue;
+    b.vols[v].ngroups = b.emits[emit_of[v]].ngroups;
+    b.vols[v].groups = b.emits[emit_of[v]].groups;
+    b.vols[v].gcap = rows_group_cap(b.plans[v].method);
+  }
   // pinned host side: descriptors | sizes
   if (c->hbatch_bytes < b_vols + b_sizes) {
     if (c->hbatch) (void)hipHostFree(c->hbatch);
@@ -1022,7 +1065,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess && n > 0)
       e = hipMemcpyAsync(dvols, c->hbatch, sizeof(VolArgs) * (size_t)n, hipMemcpyHostToDevice,
                          c->stream);
-    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, c->stream);
+    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, ngroups, (int)b.emits.size(), c->stream);
     if (e == hipSuccess) e = launch_coords_batch(dvols, n, c->stream);
     if (e == hipSuccess && work_queues(b.counts))
       e = launch_zero_u32(ctrs, (int64_t)(8 * b.counts.size()), c->stream);
@@ -1049,7 +1092,8 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess && units > 0)
       e = launch_sizes_batch(dvols, n, w, units, dsizes, c->stream);
     if (e == hipSuccess && units > 0)
-      e = hipMemcpyAsync(hsizes, dsizes, 32 * (size_t)n, hipMemcpyDeviceToHost, c->stream);
+      e = hipMemcpyAsync(hsizes, dsizes, 32 * (size_t)n + 4 * b.emits.size(), hipMemcpyDeviceToHost,
+                         c->stream);
     return e;
   };
   // everything the launches and copies above are derived from: the
@@ -1067,7 +1111,11 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   if (e != hipSuccess) return hip_fail(c, e, "batched count/scan");
 
   b.sizes.assign(4 * (size_t)n, 0);
-  if (units > 0) memcpy(b.sizes.data(), hsizes, 32 * (size_t)n);
+  b.ngroups.assign(b.emits.size(), 0);
+  if (units > 0) {
+    memcpy(b.sizes.data(), hsizes, 32 * (size_t)n);
+    memcpy(b.ngroups.data(), hsizes + 4 * n, 4 * b.emits.size());
+  }
   for (int v = 0; v < n; ++v) {
     if (nverts) nverts[v] = b.sizes[4 * v + 1];
     if (nfaces) nfaces[v] = b.sizes[4 * v + 3];
@@ -1132,6 +1180,22 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
   int32_t* emap = (int32_t*)((char*)c->bws + b_vols + b_cmap);
   memcpy(c->hbatch, b.vols.data(), sizeof(VolArgs) * (size_t)n);
   uint32_t* ectr = (uint32_t*)((char*)c->bws + b.ctr_off) + 8 * b.counts.size();
+  // blocks for the shared units: their number in steps, so that a repeated
+  // batch with new values in its fields still repeats its launches
+  std::vector<int32_t> xblocks(b.emits.size(), 0);
+  for (size_t k = 0; k < b.emits.size(); ++k) {
+    if (!b.emits[k].rows) continue;
+    const int32_t x = rows_xblocks(b.ngroups[k], rows_group_cap(b.emits[k].plan.method));
+    while (xblocks[k] < x) xblocks[k] = xblocks[k] ? 4 * xblocks[k] : 32;
+    b.emits[k].xblocks = xblocks[k];
+  }
+  auto shared_blocks = [](const Launch& L) {
+    RowsBatch r{};
+    r.groups = L.groups;
+    r.ngroups = L.ngroups;
+    r.xblocks = L.xblocks;
+    return r;
+  };
   // the output pointers travel in the descriptors (copied from hbatch by
   // the first operation), so a captured emit phase serves new outputs
   auto enqueue = [&]() -> hipError_t {
@@ -1145,7 +1209,8 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
     for (size_t k : by_cost(b.emits)) {
       if (e != hipSuccess) break;
       e = launch_emit_batch(b.emits[k].plan, b.emits[k].variant, dvols, emap, b.emits[k].gbase,
-                            b.emits[k].nblocks, ectr + 8 * k, sp.next(b.emits[k].cost));
+                            b.emits[k].nblocks, ectr + 8 * k, shared_blocks(b.emits[k]),
+                            sp.next(b.emits[k].cost));
     }
     const hipError_t ej = sp.finish();
     if (e == hipSuccess) e = ej;
@@ -1159,6 +1224,7 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
                          (const void*)c->upload};
   key_add(&key, bufs, 5);
   key_layout(&key, c, b.units);
+  key_add(&key, xblocks.data(), xblocks.size());
   hipError_t e = run_phase(c, &c->gemit, std::move(key),
                            out_memory == MSH_DEVICE && c->stream != nullptr, enqueue);
   if (e == hipSuccess) c->upload_pending = true;

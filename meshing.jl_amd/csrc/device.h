@@ -284,6 +284,66 @@ __device__ __forceinline__ double coord_at(const CoordArgs& c, int i) {
   return lerpi(j, n, c.a[axis], c.b[axis], (c.mask >> axis) & 1);
 }
 
+// The shared units of a volume of the row kernels among kScanTile units, of
+// which this thread of the block holds kScanItems, c of units first on: the
+// block counts their groups before a barrier that it has anyway (share_count),
+// and lists them after it (share_list) behind those that *o.ngroups counts, or
+// with `alone` as the only ones.  One entry of the counter a tile: one a unit
+// from the count, 9 ns each, cost 256^3 Float32 value noise, whose units are
+// all full, 76 us.
+struct ShareOut {
+  RowsGroup* groups;
+  uint32_t* ngroups;
+  uint32_t cap, waves;  // waves of an emit block: parts of a group
+  RowsCuts cuts;
+  uint32_t vol;
+};
+__host__ __device__ inline ShareOut share_out(const VolArgs& a, int vol) {
+  return {a.groups, a.ngroups, a.gcap, (uint32_t)rows_emit_waves(a.method), rows_cuts(a.method),
+          (uint32_t)vol};
+}
+struct ShareSums {
+  uint32_t w[kWaves], base;
+};
+__device__ __forceinline__ uint32_t share_count(const ShareOut& o, const uint32_t (&c)[kScanItems],
+                                                ShareSums* s) {
+  uint32_t mine = 0;
+#pragma unroll
+  for (int q = 0; q < kScanItems; ++q) mine += rows_parts(o.cuts, c[q] & 0xFFFF);
+  mine /= o.waves;  // (a power of two, which the parts are multiples of)
+  const uint32_t incl = wave_scan_dpp(mine);
+  if (lane_id() == kWave - 1) s->w[wave_id()] = incl;
+  return incl - mine;
+}
+// (before: share_count's; returns the tile's groups)
+__device__ __forceinline__ uint32_t share_list(const ShareOut& o, int64_t first,
+                                               const uint32_t (&c)[kScanItems], ShareSums* s,
+                                               uint32_t before, bool alone) {
+  uint32_t at = before, all = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    at += w < wave_id() ? s->w[w] : 0u;
+    all += s->w[w];
+  }
+  if (__builtin_expect(all == 0, 1)) return 0;
+  if (!alone) {
+    if (threadIdx.x == 0) s->base = atomicAdd(o.ngroups, all);
+    __syncthreads();
+    if (s->base >= o.cap) return all;
+    at += s->base;
+  }
+#pragma unroll 1
+  for (int q = 0; q < kScanItems; ++q) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) v = i == q ? c[i] & 0xFFFF : v;
+    const uint32_t p = rows_parts(o.cuts, v);
+    for (uint32_t k = 0; k < p; k += o.waves, ++at)
+      if (at < o.cap) o.groups[at] = {o.vol, (uint32_t)first + (uint32_t)q, k, p};
+  }
+  return all;
+}
+
 // Raw buffer resource over `bytes` bytes at p (32-bit data format, so
 // loads past `bytes` return 0 instead of touching memory).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* p, uint32_t bytes) {

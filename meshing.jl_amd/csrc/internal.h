@@ -16,6 +16,37 @@ enum Method : int { MC = 0, MT = 1, SN = 2 };
 // waves (x planes) of a row emit's block
 constexpr int rows_emit_waves(int method) { return method == SN ? 2 : 4; }
 
+// Part of a full unit of the row kernels (rows.h): `waves of a block`
+// neighbouring parts of its words, for a block of the emit beside its tiles.
+struct RowsGroup {
+  uint32_t vol;     // volume, in a batch
+  uint32_t unit;
+  uint32_t first;   // its first part ..
+  uint32_t parts;   // .. of this many
+};
+constexpr int kMaxParts = 16;
+// Where the parts of a unit start.
+struct RowsParts {
+  uint32_t pre[kMaxParts];  // the unit's vertices | faces << 16 before it
+  uint8_t word[kMaxParts];  // its first word of the unit
+};
+// Groups of an emit launch, at most: two rounds of the device's waves (with one,
+// 4096 parts, surface nets of 128^3 Float32 value noise take 141 us a call
+// instead of 100, tetrahedra of a 512^3 box 536 instead of 335).
+constexpr uint32_t rows_group_cap(int method) { return 8192 / rows_emit_waves(method); }
+// Vertices from which a unit has 4, 8 and 16 parts (about 128 cells each).
+struct RowsCuts {
+  uint32_t four, eight, sixteen;
+};
+__host__ __device__ constexpr RowsCuts rows_cuts(int method) {
+  return method == MC ? RowsCuts{1024, 4096, 8192} : method == MT ? RowsCuts{768, 1536, 3072}
+                                                                  : RowsCuts{256, 1024, 1792};
+}
+// Parts of a unit of v vertices, 0 if it is not shared.
+__host__ __device__ constexpr uint32_t rows_parts(const RowsCuts& k, uint32_t v) {
+  return (v >= k.four ? 4u : 0u) + (v >= k.eight ? 4u : 0u) + (v >= k.sixteen ? 8u : 0u);
+}
+
 // Cells are (nx-1)*(ny-1)*(nz-1).  The emission order of the reference is
 // x outermost, z innermost (src/marching_cubes.jl:40).  A "unit" is one
 // z-row of cells (fixed x, y) cut into nzseg segments of zseg cells; units
@@ -101,6 +132,13 @@ struct VolArgs {
   int32_t sw, cw;          // words of a column of samples, of a row of cells
   int32_t upx;             // units of an x plane
   int32_t ue;              // units a wave emits one after another
+  int32_t self;            // this volume's number in a batch
+  int32_t xblocks;         // blocks of groups before the tiles of a single emit ..
+  uint32_t shared;         // .. and their groups
+  RowsParts* parts;        // per unit, of the shared ones
+  RowsGroup* groups;       // room for gcap
+  uint32_t* ngroups;       // their number, while the scan counts them; above gcap no unit is shared
+  uint32_t gcap;
   int64_t bntiles, bblk0;  // sample-bit tiles in a batched launch, its first block there
   uint32_t cwm, cwn;       // 2^32 / cw and 2^16 / cw, rounded down and up (word_pos)
   int32_t nti, ntj;        // emit tiles along x and y
@@ -182,8 +220,8 @@ struct RowsGeom {
 bool rows_geom(const Plan& p, Geom* g, RowsGeom* r);
 // bytes of the sample bits, and VolArgs of a volume with its bits there
 size_t rows_bytes(const Geom& g, const RowsGeom& r);
-size_t rows_prefix_bytes(const Plan& p, const Geom& g);  // .. of VolArgs::wpre
-void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a);
+size_t rows_prefix_bytes(const Plan& p, const Geom& g);  // .. of VolArgs::wpre and parts
+void rows_vol(const RowsGeom& r, void* bits, void* prefixes, VolArgs* a);
 // emit tiling, from the number of vertices (negative: not known yet)
 void rows_emit_tiling(VolArgs* a, int64_t nverts);
 // The count's last block to finish also scans the units (one scan tile of
@@ -193,6 +231,15 @@ struct ScanTail {
   int64_t *voff, *foff, *totals, *host;
   CoordArgs coords;
 };
+// bytes of the group list of a launch, its counter first
+constexpr size_t kGroupsAt = 256;
+constexpr size_t rows_groups_bytes(int method) {
+  return kGroupsAt + rows_group_cap(method) * sizeof(RowsGroup);
+}
+// blocks for n groups: none when there are too many
+inline int32_t rows_xblocks(uint32_t n, uint32_t gcap) {
+  return n > gcap ? 0 : (int32_t)((n + 7) / 8 * 8);
+}
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, const ScanTail& tail, hipStream_t st);
 // A batched launch: tiles gbase .. gbase + nblocks of the batch, whose volumes
 // the map names.
@@ -200,6 +247,10 @@ struct RowsBatch {
   const VolArgs* vols;
   const int32_t* map;
   int64_t gbase, nblocks;
+  // emits: the launch's groups, and the blocks for them before its tiles
+  const RowsGroup* groups = nullptr;
+  const uint32_t* ngroups = nullptr;
+  int32_t xblocks = 0;
 };
 // axis types: 1 all Float64, 2 all Float32, 0 mixed
 inline int cx_class(const VolArgs& a) { return a.cxmask == 0 ? 1 : a.cxmask == 7 ? 2 : 0; }
@@ -221,11 +272,12 @@ hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st,
                         const ScanTail& tail = ScanTail{});
 // host: pinned host words that also receive the vertex and face totals
-// (at [1] and [3]), or null; coords: coordinate tables the scan also fills
-// (in its one-block tile scan, or block 0 of the fused apply) instead of a
-// launch of their own, or null
+// (at [1] and [3]) and the number of groups of shared units (at [0]), or null;
+// coords: coordinate tables the scan also fills (in its one-block tile scan,
+// or block 0 of the fused apply) instead of a launch of their own, or null;
+// rows: a volume of the row kernels, whose shared units are listed, or null
 hipError_t launch_scan(const Geom& g, const Workspace& w, hipStream_t st, int64_t* host = nullptr,
-                       const CoordArgs* coords = nullptr);
+                       const CoordArgs* coords = nullptr, const VolArgs* rows = nullptr);
 hipError_t launch_emit(const Plan& p, const VolArgs& a, hipStream_t st);
 
 // Batched launches over n volumes whose VolArgs are in device memory.
@@ -233,18 +285,20 @@ hipError_t launch_emit(const Plan& p, const VolArgs& a, hipStream_t st);
 // Plan types and emit variant); gbase is the launch's first block in the
 // block->volume maps.
 hipError_t launch_coords_batch(const VolArgs* vols, int n, hipStream_t st);
-// (bmap: sample-bit tiles of the row kernels, or null)
+// (bmap: sample-bit tiles of the row kernels, or null; also clears nz words at zero)
 hipError_t launch_fill_maps(const VolArgs* vols, int n, int32_t* cmap, int32_t* emap, int32_t* bmap,
-                            hipStream_t st);
+                            uint32_t* zero, int nz, hipStream_t st);
 // Persistent count and emit launches (families 2 and 3) take their tiles
 // from 8 work-queue counters at ctr, which must be zero at launch.
 hipError_t launch_count_batch(const Plan& p, const VolArgs* vols, const int32_t* cmap,
                               int64_t gbase, int64_t nblocks, uint32_t* ctr, hipStream_t st);
+// (and the groups of shared units)
 hipError_t launch_sizes_batch(const VolArgs* vols, int n, const Workspace& w, int64_t units,
                               int64_t* sizes, hipStream_t st);
+// (b: the groups of a launch of the row kernels, its other fields unused)
 hipError_t launch_emit_batch(const Plan& p, int variant, const VolArgs* vols,
                              const int32_t* emap, int64_t gbase, int64_t nblocks, uint32_t* ctr,
-                             hipStream_t st);
+                             const RowsBatch& b, hipStream_t st);
 // Zero n 32-bit words (the work-queue counters) with a kernel.
 hipError_t launch_zero_u32(uint32_t* p, int64_t n, hipStream_t st);
 // Exact-coordinate vertex welding (weld.hip).

@@ -55,31 +55,16 @@ __global__ void k_coords_b(const VolArgs* __restrict__ vols) {
 
 // Block -> volume maps of a batch: one block per volume fills its ranges.
 __global__ void k_fill_maps(const VolArgs* __restrict__ vols, int32_t* __restrict__ cmap,
-                            int32_t* __restrict__ emap, int32_t* __restrict__ bmap) {
+                            int32_t* __restrict__ emap, int32_t* __restrict__ bmap,
+                            uint32_t* __restrict__ zero, int nz) {
   const int v = blockIdx.x;
+  if (v == 0)
+    for (int i = threadIdx.x; i < nz; i += blockDim.x) zero[i] = 0;
   const VolArgs& a = vols[v];
   for (int64_t i = threadIdx.x; i < a.cntiles; i += blockDim.x) cmap[a.cblk0 + i] = v;
   for (int64_t i = threadIdx.x; i < a.ntiles; i += blockDim.x) emap[a.eblk0 + i] = v;
   if (bmap)
     for (int64_t i = threadIdx.x; i < a.bntiles; i += blockDim.x) bmap[a.bblk0 + i] = v;
-}
-
-// Per-volume sizes of a batch from the scan over all volumes' units (volume
-// v's units start at ubase and volumes are stored in unit order):
-// (first vertex, nverts, first face, nfaces).
-__global__ void k_sizes(const VolArgs* __restrict__ vols, int n, const int64_t* __restrict__ voff,
-                        const int64_t* __restrict__ foff, const int64_t* __restrict__ totals,
-                        int64_t units, int64_t* __restrict__ sizes) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const int64_t ub = vols[v].ubase;
-  const int64_t ue = v + 1 < n ? vols[v + 1].ubase : units;
-  const int64_t vb = ub < units ? voff[ub] : totals[1], fb = ub < units ? foff[ub] : totals[3];
-  const int64_t ve = ue < units ? voff[ue] : totals[1], fe = ue < units ? foff[ue] : totals[3];
-  sizes[4 * v + 0] = vb;
-  sizes[4 * v + 1] = ve - vb;
-  sizes[4 * v + 2] = fb;
-  sizes[4 * v + 3] = fe - fb;
 }
 
 __global__ void k_zero_u32(uint32_t* __restrict__ p, int64_t n) {
@@ -111,13 +96,54 @@ __device__ __forceinline__ uint64_t scan_load(const uint32_t* __restrict__ cnt, 
   return sum;
 }
 
+// Per-volume sizes of a batch from the scan over all volumes' units (volume
+// v's units start at ubase and volumes are stored in unit order):
+// (first vertex, nverts, first face, nfaces); and the groups of its shared
+// units, by 16 more blocks a volume.
+__global__ __launch_bounds__(kBlock) void k_sizes(const VolArgs* __restrict__ vols, int n,
+                                                  const int64_t* __restrict__ voff,
+                                                  const int64_t* __restrict__ foff,
+                                                  const int64_t* __restrict__ totals,
+                                                  int64_t units, int64_t* __restrict__ sizes) {
+  const int v = blockIdx.x;
+  const VolArgs& a = vols[v];
+  const int64_t ub = a.ubase;
+  const int64_t ue = v + 1 < n ? vols[v + 1].ubase : units;
+  __shared__ ShareSums sums;
+  if (blockIdx.y > 0) {
+    if (!a.bits) return;
+    for (int64_t t = ub + (int64_t)(blockIdx.y - 1) * kScanTile; t < ue;
+         t += (int64_t)(gridDim.y - 1) * kScanTile) {
+      const int64_t first = t + (int64_t)threadIdx.x * kScanItems;
+      uint32_t c[kScanItems];
+      (void)scan_load(a.cnt, ue, first, c);
+      const ShareOut share = share_out(a, v);
+      const uint32_t before = share_count(share, c, &sums);
+      __syncthreads();
+      (void)share_list(share, first - ub, c, &sums, before, false);
+      __syncthreads();
+    }
+    return;
+  }
+  if (threadIdx.x != 0) return;
+  const int64_t vb = ub < units ? voff[ub] : totals[1], fb = ub < units ? foff[ub] : totals[3];
+  const int64_t ve = ue < units ? voff[ue] : totals[1], fe = ue < units ? foff[ue] : totals[3];
+  sizes[4 * v + 0] = vb;
+  sizes[4 * v + 1] = ve - vb;
+  sizes[4 * v + 2] = fb;
+  sizes[4 * v + 3] = fe - fb;
+}
+
 __global__ __launch_bounds__(kBlock) void k_scan_reduce(const uint32_t* __restrict__ cnt,
                                                         int64_t units,
-                                                        uint64_t* __restrict__ tilesum) {
+                                                        uint64_t* __restrict__ tilesum,
+                                                        ShareOut share) {
   __shared__ uint64_t s_w[kWaves];
   uint32_t c[kScanItems];
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
   const uint64_t incl = wave_incl_scan64(scan_load(cnt, units, base, c));
+  __shared__ ShareSums sums;
+  const uint32_t before = share.groups ? share_count(share, c, &sums) : 0u;
   if (lane_id() == kWave - 1) s_w[wave_id()] = incl;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -126,19 +152,22 @@ __global__ __launch_bounds__(kBlock) void k_scan_reduce(const uint32_t* __restri
     for (int q = 0; q < kWaves; ++q) agg += s_w[q];
     tilesum[blockIdx.x] = agg;
   }
+  if (share.groups) (void)share_list(share, base, c, &sums, before, false);
 }
 
 constexpr int kScanTilesBlock = 1024;
 
 __global__ __launch_bounds__(kScanTilesBlock) void k_scan_tiles(
     const uint64_t* __restrict__ tilesum, int64_t ntiles, int64_t* __restrict__ tileoff,
-    int64_t* __restrict__ totals, int64_t* __restrict__ host, CoordArgs coords) {
+    int64_t* __restrict__ totals, int64_t* __restrict__ host, CoordArgs coords,
+    const uint32_t* __restrict__ ngroups) {
   // the volume's coordinate tables, when asked for: one launch fewer
   if (coords.out)
     for (int i = threadIdx.x; i < coords.nx + coords.ny + coords.nz; i += kScanTilesBlock)
       coords.out[i] = coord_at(coords, i);
   __shared__ int64_t s_v[kScanTilesBlock / kWave], s_f[kScanTilesBlock / kWave];
   const int t = threadIdx.x, lane = lane_id(), wv = t / kWave;
+  const int64_t shared = ngroups ? (int64_t)*ngroups : 0;
   const int64_t per = (ntiles + kScanTilesBlock - 1) / kScanTilesBlock;
   const int64_t lo = t * per, hi = lo + per < ntiles ? lo + per : ntiles;
   int64_t sv = 0, sf = 0;  // int64: the sums over many tiles outgrow 32 bits
@@ -173,6 +202,7 @@ __global__ __launch_bounds__(kScanTilesBlock) void k_scan_tiles(
     if (host) {
       // the sizes straight into the caller's pinned host words (no copy
       // after the scan), made visible to the host before the kernel ends
+      host[0] = shared;
       host[1] = bv + iv;
       host[3] = bf + jf;
       __threadfence_system();
@@ -220,11 +250,13 @@ constexpr int64_t kScanFuseTiles = 1024;
 __global__ __launch_bounds__(kBlock) void k_scan_apply_sums(
     const uint32_t* __restrict__ cnt, int64_t units, const uint64_t* __restrict__ tilesum,
     int64_t* __restrict__ voff, int64_t* __restrict__ foff, int64_t* __restrict__ totals,
-    int64_t* __restrict__ host, CoordArgs coords) {
+    int64_t* __restrict__ host, CoordArgs coords, const uint32_t* __restrict__ ngroups) {
   __shared__ uint64_t s_w[kWaves];
   __shared__ int64_t s_v[kWaves], s_f[kWaves];
   uint32_t c[kScanItems];
   const int wv = wave_id(), lane = lane_id();
+  int64_t shared = 0;  // (read early, for the last block)
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && ngroups) shared = (int64_t)*ngroups;
   // this tile's offset: the sums of the tiles before it (int64: they
   // outgrow 32 bits over many tiles)
   int64_t pv = 0, pf = 0;
@@ -271,6 +303,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply_sums(
     totals[2] = 0;
     totals[3] = nf;
     if (host) {
+      host[0] = shared;
       host[1] = nv;
       host[3] = nf;
       __threadfence_system();
@@ -847,19 +880,20 @@ hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream
 }
 
 hipError_t launch_scan(const Geom& g, const Workspace& w, hipStream_t st, int64_t* host,
-                       const CoordArgs* coords) {
+                       const CoordArgs* coords, const VolArgs* rows) {
   const int64_t nt = scan_tiles(g.units);
+  const ShareOut share = rows ? share_out(*rows, 0) : ShareOut{};
   hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nt), dim3(kBlock), 0, st, w.cnt, g.units,
-                     w.tilesum);
+                     w.tilesum, share);
   if (nt <= kScanFuseTiles) {
     hipLaunchKernelGGL(k_scan_apply_sums, dim3((unsigned)nt), dim3(kBlock), 0, st, w.cnt,
                        g.units, (const uint64_t*)w.tilesum, w.voff, w.foff, w.totals, host,
-                       coords ? *coords : CoordArgs{});
+                       coords ? *coords : CoordArgs{}, share.ngroups);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanTilesBlock), 0, st,
                      (const uint64_t*)w.tilesum, nt, w.tileoff, w.totals, host,
-                     coords ? *coords : CoordArgs{});
+                     coords ? *coords : CoordArgs{}, share.ngroups);
   hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nt), dim3(kBlock), 0, st, w.cnt, g.units,
                      (const int64_t*)w.tileoff, w.voff, w.foff);
   return hipGetLastError();
@@ -1020,9 +1054,10 @@ hipError_t launch_coords_batch(const VolArgs* vols, int n, hipStream_t st) {
 }
 
 hipError_t launch_fill_maps(const VolArgs* vols, int n, int32_t* cmap, int32_t* emap, int32_t* bmap,
-                            hipStream_t st) {
+                            uint32_t* zero, int nz, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_maps, dim3((unsigned)n), dim3(256), 0, st, vols, cmap, emap, bmap);
+  hipLaunchKernelGGL(k_fill_maps, dim3((unsigned)n), dim3(256), 0, st, vols, cmap, emap, bmap, zero,
+                     nz);
   return hipGetLastError();
 }
 
@@ -1064,17 +1099,17 @@ unsigned persistent_grid(const void* kernel, int64_t ntiles) {
 hipError_t launch_sizes_batch(const VolArgs* vols, int n, const Workspace& w, int64_t units,
                               int64_t* sizes, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sizes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, vols, n,
-                     w.voff, w.foff, w.totals, units, sizes);
+  hipLaunchKernelGGL(k_sizes, dim3((unsigned)n, 1 + 16), dim3(kBlock), 0, st, vols, n, w.voff, w.foff,
+                     w.totals, units, sizes);
   return hipGetLastError();
 }
 
 hipError_t launch_emit_batch(const Plan& p, int variant, const VolArgs* vols,
                              const int32_t* emap, int64_t gbase, int64_t nblocks, uint32_t* ctr,
-                             hipStream_t st) {
+                             const RowsBatch& b, hipStream_t st) {
   if (variant >= kRowsVariant) {
-    const RowsBatch b{vols, emap, gbase, nblocks};
-    return launch_rows_emit(p, variant - kRowsVariant, VolArgs{}, &b, st);
+    const RowsBatch r{vols, emap, gbase, nblocks, b.groups, b.ngroups, b.xblocks};
+    return launch_rows_emit(p, variant - kRowsVariant, VolArgs{}, &r, st);
   }
   return emit_any(p, variant, VolArgs{}, vols, emap, gbase, nblocks, ctr, st);
 }

@@ -210,6 +210,41 @@ __device__ __forceinline__ int64_t word_vertex(const VolArgs& a, int x, uint32_t
   return a.voff[a.ubase + u] + (int64_t)a.wpre[64 * u + (q & 63)];
 }
 
+// ---------------------------------------------------------------------------
+// Shared units.  A wave takes a unit's cells one queue after another, so a
+// unit of a surface that runs along its x plane, up to 2048 cells where most
+// have a few dozen, keeps one wave at work long after the rest of the device
+// is idle (a plane x = const in 256^3 Float32: 32 such units, Marching Cubes
+// call 184 us, tetrahedra 448).  Units of many outputs are therefore cut into
+// parts of neighbouring words with about the same number of vertices
+// (rows_parts, note_parts): the count pass leaves where they start, the scan
+// lists the parts in groups (RowsGroup), and the emit's first blocks take a
+// group each, a part a wave, while the waves of the tiles leave these units
+// out (81 us and 106).  Where many units are full the device is full
+// without this: above rows_group_cap none is shared.
+
+// What a wave of an emit block works on: units [g0, g1) of x plane x, or with
+// a group a part of one unit.
+struct RowsWork {
+  int x, g0, g1;
+  uint32_t cnt;         // lane i: unit g0 + i's counts, 0 if it has none or others take it
+  uint32_t shared;      // bit i: others take unit g0 + i
+  int64_t voff, foff;   // lane i: where the unit's outputs start
+  int w0, wn;           // its words: wn from w0 on
+  uint32_t vpre, fpre;  // the unit's outputs before them
+  __device__ bool has(int lane) const { return (uint32_t)(lane - w0) < (uint32_t)wn; }
+  // (again for a unit behind a shared one, so that the lanes need not keep them)
+  __device__ void unit_offsets(const VolArgs& a, int i, int64_t* v, int64_t* f) const {
+    const int64_t u = a.ubase + (int64_t)x * a.upx + g0 + i;
+    *v = a.voff[u] - a.sz[0];
+    *f = a.foff[u] - a.sz[2];
+  }
+  // shared units between i and the next one of the wave, j?
+  __device__ bool gap(int i, int j) const {
+    return ((shared >> i) & ((1u << (j - i)) - 1u)) != 0;
+  }
+};
+
 static_assert(rows_emit_waves(MC) == kWaves && rows_emit_waves(MT) == kWaves, "their blocks");
 
 // Emit tile t: W x planes (one a wave of the block, so its waves read the
@@ -234,12 +269,6 @@ __device__ __forceinline__ void rows_tile(const VolArgs& a, int64_t t, int* x, i
   *g0 = (int)gi * a.ue;
 }
 
-// Two neighbouring values in one load (aligned as one of them).
-template <typename T>
-struct __attribute__((packed, aligned(sizeof(T)))) Pair {
-  T a, b;
-};
-
 // Emit tile of block b.  Blocks are dealt round-robin to the 8 XCDs; a launch
 // of few blocks gives each XCD one run of tiles (xcd_tile), a larger one runs
 // of 32 in turn, so tiles that share lines meet in one L2 and a field whose
@@ -255,6 +284,124 @@ __device__ __forceinline__ int64_t rows_block_tile(int64_t b, int64_t nb, int64_
   // (turned by one XCD a round: the y range of a plane is not one XCD's)
   const int64_t round = (b >> 3) / C, at = (b >> 3) % C;
   return (round * 8 + (((b & 7) + round) & 7)) * C + at;
+}
+
+// An emit block's work: a group of shared parts (the first blocks; those past
+// the last group have none) or a tile.
+struct RowsBlock {
+  bool none = false;
+  const RowsGroup* grp = nullptr;
+  bool share = false;  // the launch's tiles leave shared units out
+  int64_t tile = 0;    // of the volume
+  int vol = 0;
+};
+__device__ __forceinline__ RowsBlock rows_block(const VolArgs& a) {
+  // (worked out for a tile first: a branch on a kernel argument ahead of it
+  // would put the reads of the others behind the wait for that one)
+  RowsBlock r;
+  r.tile = rows_block_tile((int64_t)blockIdx.x - a.xblocks, a.ntiles);
+  r.share = a.xblocks > 0;
+  if (__builtin_expect((int)blockIdx.x < a.xblocks, 0)) {
+    r.none = blockIdx.x >= a.shared;
+    r.grp = a.groups + blockIdx.x;
+    r.share = false;
+  }
+  return r;
+}
+__device__ __forceinline__ RowsBlock rows_block(const int32_t* __restrict__ map, int64_t gbase,
+                                                const RowsGroup* __restrict__ groups,
+                                                const uint32_t* __restrict__ ngroups,
+                                                int32_t xblocks, int64_t few = 8192) {
+  RowsBlock r;
+  if (__builtin_expect((int)blockIdx.x < xblocks, 0)) {
+    r.none = blockIdx.x >= *ngroups;
+    r.grp = groups + blockIdx.x;
+    if (!r.none) r.vol = __builtin_amdgcn_readfirstlane((int)r.grp->vol);
+  } else {
+    r.tile = gbase + rows_block_tile((int64_t)blockIdx.x - xblocks, (int64_t)gridDim.x - xblocks, few);
+    r.vol = __builtin_amdgcn_readfirstlane(map[r.tile]);
+    r.share = xblocks > 0;
+  }
+  return r;
+}
+template <int METHOD>
+__device__ __forceinline__ RowsWork rows_work(const VolArgs& a, const RowsBlock& b) {
+  const RowsGroup* const grp = b.grp;
+  const bool share = b.share;
+  constexpr int W = rows_emit_waves(METHOD);
+  const int lane = lane_id();
+  RowsWork k{};
+  // (a group's block: any tile, replaced below)
+  rows_tile<W>(a, grp ? 0 : b.tile, &k.x, &k.g0);
+  k.g1 = min(k.g0 + a.ue, a.upx);
+  k.wn = kWave;
+  if (__builtin_expect(grp != nullptr, 0)) {
+    const uint32_t u = grp->unit, parts = grp->parts;
+    const uint32_t part = grp->first + (uint32_t)__builtin_amdgcn_readfirstlane(wave_id());
+    const RowsParts& cut = a.parts[u];
+    const uint32_t pre = cut.pre[part];
+    k.x = (int)(u / (uint32_t)a.upx);
+    k.g0 = (int)(u - (uint32_t)k.x * (uint32_t)a.upx);
+    k.g1 = k.g0 + 1;
+    k.w0 = cut.word[part];
+    k.wn = (part + 1 < parts ? (int)cut.word[part + 1] : kWave) - k.w0;
+    k.vpre = pre & 0xFFFF;
+    k.fpre = pre >> 16;
+  }
+  if (k.x < a.g.nx - 1 && lane < k.g1 - k.g0) {
+    const int64_t u = a.ubase + (int64_t)k.x * a.upx + k.g0 + lane;
+    k.cnt = a.cnt[u];
+    k.voff = a.voff[u] - a.sz[0];
+    k.foff = a.foff[u] - a.sz[2];
+  }
+  const bool others = share && rows_parts(rows_cuts(METHOD), k.cnt & 0xFFFF) > 0;
+  k.shared = (uint32_t)__ballot(others);  // (of kMaxUE units)
+  k.cnt = others ? 0u : k.cnt;
+  return k;
+}
+
+// Two neighbouring values in one load (aligned as one of them).
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) Pair {
+  T a, b;
+};
+
+// What the emits take of volume v of a batch, read as constant memory (it is, from
+// the upload on): scalar loads, and pointers that the compiler knows to be
+// global.  As flat ones, two registers an address, they cost Marching Cubes 98
+// registers instead of 80 and made the tetrahedra kernel spill.
+__device__ __forceinline__ VolArgs batch_volume(const VolArgs* vols, int v) {
+  const auto* s = (const __attribute__((address_space(4))) VolArgs*)vols +
+                  __builtin_amdgcn_readfirstlane(v);
+  VolArgs a{};
+  a.f = s->f;
+  a.g.nx = s->g.nx;
+  a.g.ny = s->g.ny;
+  a.g.nz = s->g.nz;
+  a.iso = s->iso;
+  a.eps = s->eps;
+  a.ome = s->ome;
+  a.cxmask = s->cxmask;
+  a.coords = s->coords;
+  a.cnt = s->cnt;
+  a.voff = s->voff;
+  a.foff = s->foff;
+  a.sz = s->sz;
+  a.verts = s->verts;
+  a.faces = s->faces;
+  a.ubase = s->ubase;
+  a.bits = s->bits;
+  a.wpre = s->wpre;
+  a.parts = s->parts;
+  a.xs = s->xs;
+  a.sw = s->sw;
+  a.cw = s->cw;
+  a.upx = s->upx;
+  a.ue = s->ue;
+  a.cwm = s->cwm;
+  a.cwn = s->cwn;
+  a.eblk0 = s->eblk0;
+  return a;
 }
 
 // 64 records of three values from LDS to the output, each through `value`:

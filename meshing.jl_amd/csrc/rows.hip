@@ -98,6 +98,7 @@ __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
 
 template <typename T, int PW, int E, int WX, bool NT>
 __global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.ngroups = 0;  // for the scan
   bits_tile<T, PW, E, WX, NT>(a, blockIdx.x);
 }
 
@@ -211,6 +212,24 @@ __device__ __forceinline__ uint32_t mt_word_counts(const CellWord& r, bool x0) {
   return v | (f << 16);
 }
 
+// The parts of a shared unit (rows.h): cut where the vertices before a word,
+// of v in all, pass the next multiple of v / parts.
+__device__ __forceinline__ void note_parts(const VolArgs& a, int method, uint32_t u, uint32_t all,
+                                           uint32_t before) {
+  const uint32_t v = all & 0xFFFF, parts = rows_parts(rows_cuts(method), v);
+  if (__builtin_expect(parts == 0, 1)) return;
+  const uint32_t lane = (uint32_t)lane_id();
+  uint32_t first = 0;  // lane p: part p's first word
+  for (uint32_t p = 1; p < parts; ++p) {
+    const uint32_t words = (uint32_t)__popcll(__ballot((before & 0xFFFF) * parts < p * v));
+    first = lane == p ? words : first;
+  }
+  const uint32_t pre =
+      (uint32_t)__builtin_amdgcn_ds_bpermute((int)(min(first, (uint32_t)kWave - 1u) << 2), (int)before);
+  if (lane < parts) a.parts[u].pre[lane] = first < (uint32_t)kWave ? pre : all;
+  if (lane < parts) a.parts[u].word[lane] = (uint8_t)first;
+}
+
 template <int METHOD>
 __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, const uint8_t* extra) {
   const int lane = lane_id();
@@ -228,6 +247,7 @@ __device__ __forceinline__ void rows_count_tile(const VolArgs& a, int64_t t, con
     if constexpr (METHOD == SN) n = sn_word_counts(r, x > 0);
     const uint32_t incl = wave_scan_dpp(n);
     if (lane == kWave - 1) cnt[u] = incl;
+    note_parts(a, METHOD, u, (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1), incl - n);
     if constexpr (METHOD != MC)
       a.wpre[64 * (int64_t)u + lane] = (uint16_t)((incl - n) & 0xFFFF);
   }
@@ -249,6 +269,7 @@ __device__ __forceinline__ void count_table(uint8_t* extra) {
 // visible to the device before it adds itself to `done`).  Small volumes are
 // launches and little else: two launches fewer, 32^3 Float32 sphere call
 // 40.5 -> 36.9 us.
+template <int METHOD>
 __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
   __shared__ bool last;
   __shared__ uint64_t s_w[kWaves];
@@ -271,6 +292,10 @@ __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
     sum += (uint64_t)(c[q] & 0xFFFF) | ((uint64_t)(c[q] >> 16) << 32);
   }
   const uint64_t incl = wave_incl_scan64(sum);
+  __shared__ ShareSums sums;
+  const ShareOut share{a.groups, a.ngroups, a.gcap, (uint32_t)rows_emit_waves(METHOD),
+                       rows_cuts(METHOD), 0};
+  const uint32_t groups = share_count(share, c, &sums);
   if (lane_id() == kWave - 1) s_w[wave_id()] = incl;
   __syncthreads();
   uint64_t before = 0, all = 0;
@@ -290,6 +315,7 @@ __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
     rv += c[q] & 0xFFFF;
     rf += c[q] >> 16;
   }
+  const uint32_t shared = share_list(share, base, c, &sums, groups, true);
   if (threadIdx.x == 0) {
     const int64_t nv = (int64_t)(all & 0xFFFFFFFFu), nf = (int64_t)(all >> 32);
     t.totals[0] = 0;
@@ -297,6 +323,7 @@ __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
     t.totals[2] = 0;
     t.totals[3] = nf;
     *t.done = 0;
+    t.host[0] = (int64_t)shared;
     t.host[1] = nv;
     t.host[3] = nf;
     __threadfence_system();
@@ -311,7 +338,7 @@ __global__ __launch_bounds__(kBlock) void k_rows_count(VolArgs a, ScanTail tail)
       tail.coords.out[i] = coord_at(tail.coords, i);
   count_table<METHOD>(extra);
   rows_count_tile<METHOD>(a, blockIdx.x, extra);
-  if (tail.done) scan_tail(a, tail);
+  if (tail.done) scan_tail<METHOD>(a, tail);
 }
 
 template <int METHOD>
@@ -359,12 +386,14 @@ size_t rows_bytes(const Geom& g, const RowsGeom& r) {
 }
 
 size_t rows_prefix_bytes(const Plan& p, const Geom& g) {
-  return p.method == MC ? 0 : align256((size_t)g.units * 64 * sizeof(uint16_t));
+  return align256((size_t)g.units * ((p.method == MC ? 0 : 64 * sizeof(uint16_t)) +
+                                     sizeof(RowsParts)));
 }
 
-void rows_vol(const RowsGeom& r, void* bits, void* wpre, VolArgs* a) {
+void rows_vol(const RowsGeom& r, void* bits, void* prefixes, VolArgs* a) {
   a->bits = (uint32_t*)bits;
-  a->wpre = (uint16_t*)wpre;
+  a->parts = (RowsParts*)prefixes;
+  a->wpre = (uint16_t*)(a->parts + a->g.units);
   a->xs = r.xs;
   a->sw = r.sw;
   a->cw = r.cw;

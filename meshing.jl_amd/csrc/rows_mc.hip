@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_image() {
 }
 
 template <typename T, typename M, typename Out, int CXM>
-__device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
+__device__ __forceinline__ void rows_mc_tile(const VolArgs& a, const RowsBlock& blk) {
   constexpr int VW = (kCells * 12 + 64) / 64 + 1, FW = (kCells * 5 + 64) / 64 + 1;
   struct Wave {
     union {
@@ -70,18 +70,9 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
   const uint32_t pbytes = (uint32_t)((int64_t)g.nx * g.ny * (int64_t)sizeof(T));
   const uint32_t rbytes = (uint32_t)g.nx * (uint32_t)sizeof(T);
   const int lane = lane_id();
-  int x, g0;
-  rows_tile<kWaves>(a, t, &x, &g0);
-  const int g1 = min(g0 + a.ue, a.upx);
-  // lane i holds unit g0 + i's counts and output offsets
-  uint32_t cnt = 0;
-  int64_t voff = 0, foff = 0;
-  if (x < g.nx - 1 && lane < g1 - g0) {
-    const int64_t u = a.ubase + (int64_t)x * a.upx + g0 + lane;
-    cnt = a.cnt[u];
-    voff = a.voff[u] - a.sz[0];
-    foff = a.foff[u] - a.sz[2];
-  }
+  const RowsWork work = rows_work<MC>(a, blk);
+  const int x = work.x, g0 = work.g0, g1 = work.g1;
+  const uint32_t cnt = work.cnt;
   // a tile whose units are all empty ends here, before its tables
   if (!__syncthreads_or(cnt != 0)) return;
   for (int q = threadIdx.x; q < (int)(sizeof(McImage) / 16); q += kBlock)
@@ -114,10 +105,16 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
   const double* __restrict__ zp = yp + g.ny;
   const double x0 = a.coords[x], x1 = a.coords[x + 1];
   const WordBase wb = word_base(a, g0);
-  int64_t vb = readlane64(voff, 0), fb = readlane64(foff, 0);
-  uint32_t vph = (uint32_t)vb & 63u, fph = (uint32_t)fb & 63u;
-  uint32_t V = vph, F = fph;  // slots of the queue, from the last multiple of 64 records
-  int nc = 0;                 // its cells
+  int64_t vb, fb;     // the queue's first outputs ..
+  uint32_t vph, fph;  // .. beyond a multiple of 64 records
+  uint32_t V, F;      // slots of the queue, from that multiple
+  int nc = 0;         // its cells
+  auto start = [&](int64_t v, int64_t f) {  // at a unit's outputs
+    vb = v;
+    fb = f;
+    V = vph = (uint32_t)vb & 63u;
+    F = fph = (uint32_t)fb & 63u;
+  };
 
   struct Fetch {
     T va, vb;
@@ -204,6 +201,8 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
   };
 
   int gi = g0 + __builtin_ctzll(todo);
+  start(readlane64(work.voff, gi - g0) + (int64_t)work.vpre,
+        readlane64(work.foff, gi - g0) + (int64_t)work.fpre);
   RawWords raw = load_raw(a, x, gi, lane);
 #pragma unroll 1
   while (gi < g1) {
@@ -211,7 +210,8 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
     const uint64_t rest = (todo >> (gi - g0)) & ~1ull;
     const int gn = rest ? gi + __builtin_ctzll(rest) : g1;
     if (gn < g1) raw = load_raw(a, x, gn, lane);  // the next unit's words, meanwhile
-    const uint32_t act = active_cells(r);
+    const bool gap = gn < g1 && work.gap(gi - g0, gn - g0);
+    const uint32_t act = work.has(lane) ? active_cells(r) : 0u;
     const uint32_t incl = wave_scan_dpp(__popc(act));
     const int total = __builtin_amdgcn_readlane((int)incl, kWave - 1);
     for (int lo = 0; lo < total;) {
@@ -237,7 +237,12 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
       F += sum >> 16;
       nc += take;
       lo += take;
-      if (nc == kCells || (lo == total && gn == g1)) flush();
+      if (nc == kCells || (lo == total && (gn == g1 || gap))) flush();
+    }
+    if (gap) {
+      int64_t v, f;
+      work.unit_offsets(a, gn - g0, &v, &f);
+      start(v, f);
     }
     gi = gn;
   }
@@ -245,16 +250,20 @@ __device__ __forceinline__ void rows_mc_tile(const VolArgs& a, int64_t t) {
 
 template <typename T, typename M, typename Out, int CXM>
 __global__ __launch_bounds__(kBlock) void k_rows_mc(VolArgs a) {
-  rows_mc_tile<T, M, Out, CXM>(a, rows_block_tile(blockIdx.x, a.ntiles));
+  const RowsBlock b = rows_block(a);
+  if (!b.none) rows_mc_tile<T, M, Out, CXM>(a, b);
 }
 
-// Batched: a block per tile of the launch; the map names its volume.
+// Batched: a block per group or tile of the launch.
 template <typename T, typename M, typename Out, int CXM>
 __global__ __launch_bounds__(kBlock) void k_rows_mc_b(const VolArgs* __restrict__ vols,
-                                                  const int32_t* __restrict__ emap, int64_t gbase) {
-  const int64_t b = gbase + rows_block_tile(blockIdx.x, gridDim.x);
-  const VolArgs a = vols[__builtin_amdgcn_readfirstlane(emap[b])];
-  rows_mc_tile<T, M, Out, CXM>(a, b - a.eblk0);
+    const int32_t* __restrict__ emap, int64_t gbase, const RowsGroup* __restrict__ groups,
+    const uint32_t* __restrict__ ngroups, int32_t xblocks) {
+  RowsBlock b = rows_block(emap, gbase, groups, ngroups, xblocks);
+  if (b.none) return;
+  const VolArgs a = batch_volume(vols, b.vol);
+  b.tile -= a.eblk0;
+  rows_mc_tile<T, M, Out, CXM>(a, b);
 }
 
 }  // namespace
@@ -270,10 +279,12 @@ hipError_t launch_mc_image(hipStream_t st) {
 template <typename T, typename M, typename Out, int CXM>
 static hipError_t rows_mc_cx(const VolArgs& a, const RowsBatch* b, hipStream_t st) {
   if (b)
-    hipLaunchKernelGGL((k_rows_mc_b<T, M, Out, CXM>), dim3((unsigned)b->nblocks), dim3(kBlock), 0, st, b->vols,
-                       b->map, b->gbase);
+    hipLaunchKernelGGL((k_rows_mc_b<T, M, Out, CXM>), dim3((unsigned)(b->xblocks + b->nblocks)),
+                       dim3(kBlock), 0, st, b->vols, b->map, b->gbase, b->groups,
+                       b->ngroups, b->xblocks);
   else
-    hipLaunchKernelGGL((k_rows_mc<T, M, Out, CXM>), dim3((unsigned)a.ntiles), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_rows_mc<T, M, Out, CXM>), dim3((unsigned)(a.xblocks + a.ntiles)),
+                       dim3(kBlock), 0, st, a);
   return hipGetLastError();
 }
 

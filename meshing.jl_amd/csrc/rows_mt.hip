@@ -159,7 +159,7 @@ __device__ __forceinline__ Planes owned_planes(const Col& a, const Col& b, const
 }
 
 template <typename T, typename M, typename A, typename Out, int CXM>
-__device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
+__device__ __forceinline__ void rows_mt_tile(const VolArgs& a, const RowsBlock& blk) {
   constexpr int VW = (kCells * 13 + 64) / 64 + 1, FW = (kCells * 12 + 64) / 64 + 1;
   struct Owners {
     int32_t first[8][64];  // first vertex of the owner one step back along (bits of) the index,
@@ -192,18 +192,9 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
   const uint32_t pbytes = (uint32_t)((int64_t)g.nx * g.ny * (int64_t)sizeof(T));
   const uint32_t rbytes = (uint32_t)g.nx * (uint32_t)sizeof(T);
   const int lane = lane_id();
-  int x, g0;
-  rows_tile<kWaves>(a, t, &x, &g0);
-  const int g1 = min(g0 + a.ue, a.upx);
-  // lane i holds unit g0 + i's counts and output offsets
-  uint32_t cnt = 0;
-  int64_t voff = 0, foff = 0;
-  if (x < g.nx - 1 && lane < g1 - g0) {
-    const int64_t u = a.ubase + (int64_t)x * a.upx + g0 + lane;
-    cnt = a.cnt[u];
-    voff = a.voff[u] - a.sz[0];
-    foff = a.foff[u] - a.sz[2];
-  }
+  const RowsWork work = rows_work<MT>(a, blk);
+  const int x = work.x, g0 = work.g0, g1 = work.g1;
+  const uint32_t cnt = work.cnt;
   // a tile whose units are all empty ends here, before its tables
   if (!__syncthreads_or(cnt != 0)) return;
   for (int q = threadIdx.x; q < (int)(sizeof(MtImage) / 16); q += kBlock)
@@ -237,10 +228,16 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
   const double* __restrict__ zp = yp + g.ny;
   const double x0 = a.coords[x], x1 = a.coords[x + 1];
   const WordBase wb = word_base(a, g0);
-  int64_t vb = readlane64(voff, 0), fb = readlane64(foff, 0);
-  uint32_t vph = (uint32_t)vb & 63u, fph = (uint32_t)fb & 63u;
-  uint32_t V = vph, F = fph;  // slots of the queue, from the last multiple of 64 records
+  int64_t vb, fb;     // the queue's first outputs ..
+  uint32_t vph, fph;  // .. beyond a multiple of 64 records
+  uint32_t V, F;      // slots of the queue, from that multiple
   int nc = 0, nv = 0, nf = 0;  // its cells, those with vertices, with faces
+  auto start = [&](int64_t v, int64_t f) {  // at a unit's outputs
+    vb = v;
+    fb = f;
+    V = vph = (uint32_t)vb & 63u;
+    F = fph = (uint32_t)fb & 63u;
+  };
 
   struct Fetch {
     T va, vb;
@@ -411,9 +408,12 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
   };
 
   int gi = g0 + __builtin_ctzll(todo), done = 0;  // `done` cells of unit gi are through ..
-  uint32_t udone = 0;                             // .. with this many vertices
+  uint32_t udone = work.vpre;                     // .. with this many vertices
+  start(readlane64(work.voff, gi - g0) + (int64_t)work.vpre,
+        readlane64(work.foff, gi - g0) + (int64_t)work.fpre);
 #pragma unroll 1
   while (gi < g1) {
+    bool gap = false;  // before the next unit
     {
       int y, w;
       word_pos(a, word_base(a, gi), (uint32_t)lane, &y, &w);
@@ -441,7 +441,7 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
           }
       }
       const Col c00 = col_of(k[4]), c10 = col_of(k[7]), c01 = col_of(k[5]), c11 = col_of(k[8]);
-      uint32_t act = active_of(c00, c10, c01, c11, valid);
+      const uint32_t act = work.has(lane) ? active_of(c00, c10, c01, c11, valid) : 0u;
       uint32_t above = 0;
 #pragma unroll
       for (int i = 0; i < 9; ++i) above |= k[i].hi << (2 * i);
@@ -452,9 +452,11 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
       uint32_t w10 = 0, w01 = 0, w11 = 0, pre = 0;
       {
         const uint32_t q = (uint32_t)gi * 64u + (uint32_t)lane, cw = (uint32_t)a.cw;
+        // (read from its lane before the branch: that lane may not take it)
+        const int64_t unit = readlane64(work.voff, gi - g0) + a.sz[0];
         if (act != 0) {
           pre = a.wpre[64 * ((int64_t)x * a.upx + gi) + lane];
-          const int64_t mine = readlane64(voff, gi - g0) + a.sz[0] + (int64_t)pre;
+          const int64_t mine = unit + (int64_t)pre;
           if (x > 0) w10 = (uint32_t)(mine - word_vertex(a, x - 1, q));
           if (y > 0) w01 = (uint32_t)(mine - word_vertex(a, x, q - cw));
           if (x > 0 && y > 0) w11 = (uint32_t)(mine - word_vertex(a, x - 1, q - cw));
@@ -552,27 +554,38 @@ __device__ __forceinline__ void rows_mt_tile(const VolArgs& a, int64_t t) {
       }
       if (done >= total) {  // the next unit with outputs
         const uint64_t rest = (todo >> (gi - g0)) & ~1ull;
-        gi = rest ? gi + __builtin_ctzll(rest) : g1;
+        const int gn = rest ? gi + __builtin_ctzll(rest) : g1;
+        gap = gn < g1 && work.gap(gi - g0, gn - g0);
+        gi = gn;
         done = 0;
         udone = 0;
       }
     }
-    if (nc == kCells || (gi == g1 && nc > 0)) emit();
+    if (nc == kCells || ((gi == g1 || gap) && nc > 0)) emit();
+    if (gap) {
+      int64_t v, f;
+      work.unit_offsets(a, gi - g0, &v, &f);
+      start(v, f);
+    }
   }
 }
 
 template <typename T, typename M, typename A, typename Out, int CXM>
 __global__ __launch_bounds__(kBlock, 4) void k_rows_mt(VolArgs a) {
-  rows_mt_tile<T, M, A, Out, CXM>(a, rows_block_tile(blockIdx.x, a.ntiles));
+  const RowsBlock b = rows_block(a);
+  if (!b.none) rows_mt_tile<T, M, A, Out, CXM>(a, b);
 }
 
-// Batched: a block per tile of the launch; the map names its volume.
+// Batched: a block per group or tile of the launch.
 template <typename T, typename M, typename A, typename Out, int CXM>
 __global__ __launch_bounds__(kBlock, 4) void k_rows_mt_b(const VolArgs* __restrict__ vols,
-                                                  const int32_t* __restrict__ emap, int64_t gbase) {
-  const int64_t b = gbase + rows_block_tile(blockIdx.x, gridDim.x);
-  const VolArgs a = vols[__builtin_amdgcn_readfirstlane(emap[b])];
-  rows_mt_tile<T, M, A, Out, CXM>(a, b - a.eblk0);
+    const int32_t* __restrict__ emap, int64_t gbase, const RowsGroup* __restrict__ groups,
+    const uint32_t* __restrict__ ngroups, int32_t xblocks) {
+  RowsBlock b = rows_block(emap, gbase, groups, ngroups, xblocks);
+  if (b.none) return;
+  const VolArgs a = batch_volume(vols, b.vol);
+  b.tile -= a.eblk0;
+  rows_mt_tile<T, M, A, Out, CXM>(a, b);
 }
 
 }  // namespace
@@ -588,10 +601,12 @@ hipError_t launch_mt_image(hipStream_t st) {
 template <typename T, typename M, typename A, typename Out, int CXM>
 static hipError_t rows_mt_cx(const VolArgs& a, const RowsBatch* b, hipStream_t st) {
   if (b)
-    hipLaunchKernelGGL((k_rows_mt_b<T, M, A, Out, CXM>), dim3((unsigned)b->nblocks), dim3(kBlock), 0, st, b->vols,
-                       b->map, b->gbase);
+    hipLaunchKernelGGL((k_rows_mt_b<T, M, A, Out, CXM>), dim3((unsigned)(b->xblocks + b->nblocks)),
+                       dim3(kBlock), 0, st, b->vols, b->map, b->gbase, b->groups,
+                       b->ngroups, b->xblocks);
   else
-    hipLaunchKernelGGL((k_rows_mt<T, M, A, Out, CXM>), dim3((unsigned)a.ntiles), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_rows_mt<T, M, A, Out, CXM>), dim3((unsigned)(a.xblocks + a.ntiles)),
+                       dim3(kBlock), 0, st, a);
   return hipGetLastError();
 }
 

@@ -43,7 +43,7 @@ struct SnEdges {
 constexpr SnEdges kSnEdges = {{0, 1, 3, 2, 4, 5, 7, 6, 0, 1, 3, 2}, {1, 3, 2, 0, 5, 7, 6, 4, 4, 5, 7, 6}};
 
 template <typename T, typename M, typename Out, int CXM>
-__device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
+__device__ __forceinline__ void rows_sn_tile(const VolArgs& a, const RowsBlock& blk) {
   constexpr int FW = (kCells * 6 + 64) / 64 + 1;
   struct Wave {
     union {
@@ -60,18 +60,9 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
   const uint32_t pbytes = (uint32_t)((int64_t)g.nx * g.ny * (int64_t)sizeof(T));
   const uint32_t rbytes = (uint32_t)g.nx * (uint32_t)sizeof(T);
   const int lane = lane_id();
-  int x, g0;
-  rows_tile<kSnWaves>(a, t, &x, &g0);
-  const int g1 = min(g0 + a.ue, a.upx);
-  // lane i holds unit g0 + i's counts and output offsets
-  uint32_t cnt = 0;
-  int64_t voff = 0, foff = 0;
-  if (x < g.nx - 1 && lane < g1 - g0) {
-    const int64_t u = a.ubase + (int64_t)x * a.upx + g0 + lane;
-    cnt = a.cnt[u];
-    voff = a.voff[u] - a.sz[0];
-    foff = a.foff[u] - a.sz[2];
-  }
+  const RowsWork work = rows_work<SN>(a, blk);
+  const int x = work.x, g0 = work.g0, g1 = work.g1;
+  const uint32_t cnt = work.cnt;
   const uint64_t todo = __ballot(cnt != 0);  // bit i: unit g0 + i has outputs
   if (todo == 0) return;
   Wave& wm = waves[wave_id()];
@@ -85,14 +76,18 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
   const double* __restrict__ yp = a.coords + g.nx;
   const double* __restrict__ zp = yp + g.ny;
   const double x0 = a.coords[x], x1 = a.coords[x + 1];
-  int64_t vb = readlane64(voff, 0), fb = readlane64(foff, 0);
+  int64_t vb, fb;  // the queue's first outputs
 
   const WordBase wb = word_base(a, g0);
   int nc = 0;      // cells in the queue
   uint32_t F = 0;  // its face slots, from the last multiple of 64 records in the output
-  uint32_t fph = (uint32_t)fb & 63u;
-  F = fph;
+  uint32_t fph;
   int nf = 0;  // its cells with faces
+  auto start = [&](int64_t v, int64_t f) {  // at a unit's outputs
+    vb = v;
+    fb = f;
+    F = fph = (uint32_t)fb & 63u;
+  };
 
   struct Fetch {
     Pair<T> s00, s01, s10, s11;  // (y, z) (y+1, z) (y, z+1) (y+1, z+1), samples x and x+1
@@ -206,23 +201,27 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
   };
 
   int gi = g0 + __builtin_ctzll(todo), done = 0;  // `done` cells of unit gi are through
+  start(readlane64(work.voff, gi - g0) + (int64_t)work.vpre,
+        readlane64(work.foff, gi - g0) + (int64_t)work.fpre);
 #pragma unroll 1
   while (gi < g1) {
+    bool gap = false;  // before the next unit
     {
       const CellWord r = load_cells(a, x, gi, lane);
       const BackWords k = load_back(a, x, r);
-      uint32_t act = active_cells(r);
+      const uint32_t act = work.has(lane) ? active_cells(r) : 0u;
       const uint32_t a10 = active_of(k.x0, r.c00, k.x1, r.c01, r.valid);
       const uint32_t a01 = active_of(k.y0, k.y1, r.c00, r.c10, r.valid);
       const uint32_t a11 = active_of(k.xy, k.y0, k.x0, r.c00, r.valid);
       const uint32_t incl = wave_scan_dpp(__popc(act));
       const int total = __builtin_amdgcn_readlane((int)incl, kWave - 1);
-      const int at = (int)incl - (int)__popc(act);
+      // cells of the unit before the word
+      const int at = (int)work.vpre + (int)incl - (int)__popc(act);
       // how far back the first vertices of the words at -x, -y and both are
       // from this word's (only a quad's cells are asked for, and they exist)
       uint32_t w10 = 0, w01 = 0, w11 = 0;
       {
-        const int64_t mine = readlane64(voff, gi - g0) + a.sz[0] + at;
+        const int64_t mine = readlane64(work.voff, gi - g0) + a.sz[0] + at;
         const uint32_t q = (uint32_t)gi * 64u + (uint32_t)lane, cw = (uint32_t)a.cw;
         const bool some = act != 0;
         if (some && x > 0) w10 = (uint32_t)(mine - word_vertex(a, x - 1, q));
@@ -270,28 +269,39 @@ __device__ __forceinline__ void rows_sn_tile(const VolArgs& a, int64_t t) {
       }
       if (done >= total) {  // the next unit with outputs
         const uint64_t rest = (todo >> (gi - g0)) & ~1ull;
-        gi = rest ? gi + __builtin_ctzll(rest) : g1;
+        const int gn = rest ? gi + __builtin_ctzll(rest) : g1;
+        gap = gn < g1 && work.gap(gi - g0, gn - g0);
+        gi = gn;
         done = 0;
       }
     }
-    if (nc == kCells || (gi == g1 && nc > 0)) emit();
+    if (nc == kCells || ((gi == g1 || gap) && nc > 0)) emit();
+    if (gap) {
+      int64_t v, f;
+      work.unit_offsets(a, gi - g0, &v, &f);
+      start(v, f);
+    }
   }
 }
 
 template <typename T, typename M, typename Out, int CXM>
 __global__ __launch_bounds__(kSnBlock) void k_rows_sn(VolArgs a) {
-  rows_sn_tile<T, M, Out, CXM>(a, rows_block_tile(blockIdx.x, a.ntiles));
+  const RowsBlock b = rows_block(a);
+  if (!b.none) rows_sn_tile<T, M, Out, CXM>(a, b);
 }
 
-// Batched: a block per tile of the launch; the map names its volume.  Turns
+// Batched: a block per group or tile of the launch.  Turns
 // over the XCDs from 16384 blocks, as many waves as in the other methods'
 // batches (32 mixed volumes 605 us a batch, 624 with turns from 8192).
 template <typename T, typename M, typename Out, int CXM>
 __global__ __launch_bounds__(kSnBlock) void k_rows_sn_b(const VolArgs* __restrict__ vols,
-                                                  const int32_t* __restrict__ emap, int64_t gbase) {
-  const int64_t b = gbase + rows_block_tile(blockIdx.x, gridDim.x, 16384);
-  const VolArgs a = vols[__builtin_amdgcn_readfirstlane(emap[b])];
-  rows_sn_tile<T, M, Out, CXM>(a, b - a.eblk0);
+    const int32_t* __restrict__ emap, int64_t gbase, const RowsGroup* __restrict__ groups,
+    const uint32_t* __restrict__ ngroups, int32_t xblocks) {
+  RowsBlock b = rows_block(emap, gbase, groups, ngroups, xblocks, 16384);
+  if (b.none) return;
+  const VolArgs a = batch_volume(vols, b.vol);
+  b.tile -= a.eblk0;
+  rows_sn_tile<T, M, Out, CXM>(a, b);
 }
 
 }  // namespace
@@ -302,10 +312,12 @@ __global__ __launch_bounds__(kSnBlock) void k_rows_sn_b(const VolArgs* __restric
 template <typename T, typename M, typename Out, int CXM>
 static hipError_t rows_sn_cx(const VolArgs& a, const RowsBatch* b, hipStream_t st) {
   if (b)
-    hipLaunchKernelGGL((k_rows_sn_b<T, M, Out, CXM>), dim3((unsigned)b->nblocks), dim3(kSnBlock), 0, st, b->vols,
-                       b->map, b->gbase);
+    hipLaunchKernelGGL((k_rows_sn_b<T, M, Out, CXM>), dim3((unsigned)(b->xblocks + b->nblocks)),
+                       dim3(kSnBlock), 0, st, b->vols, b->map, b->gbase, b->groups,
+                       b->ngroups, b->xblocks);
   else
-    hipLaunchKernelGGL((k_rows_sn<T, M, Out, CXM>), dim3((unsigned)a.ntiles), dim3(kSnBlock), 0, st, a);
+    hipLaunchKernelGGL((k_rows_sn<T, M, Out, CXM>), dim3((unsigned)(a.xblocks + a.ntiles)),
+                       dim3(kSnBlock), 0, st, a);
   return hipGetLastError();
 }
 

@@ -106,14 +106,14 @@ class FieldSpec:
 def _workspace_units(nx, ny, nz):
     """Workspace of a volume's count in units of 24 bytes: one per cell row
     for the kernels that count by rows, or the sample bits (a bit per sample,
-    rows of planes padded to 128 bytes) and 156 bytes per 64 words of cells
+    rows of planes padded to 128 bytes) and 236 bytes per 64 words of cells
     for the kernels that go by words, whichever is more."""
     if min(nx, ny, nz) < 2:
         return 0
     words = -(-nz // 32)
     plane = -(-ny * words // 32) * 32
     groups = (nx - 1) * -(-(ny - 1) * -(-(nz - 1) // 32) // 64)
-    return max((nx - 1) * (ny - 1), -(-(4 * nx * plane + 156 * groups) // 24))
+    return max((nx - 1) * (ny - 1), -(-(4 * nx * plane + 236 * groups) // 24))
 
 
 @dataclass
