@@ -525,6 +525,28 @@ bool rows_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t
 // The row kernels serve the default family and family 2.
 bool rows_family(const Plan& p) { return p.family < 0 || p.family == 2; }
 
+// .. but by default not a volume of many short x planes: a unit never spans
+// two of them, so its wave, and each of its passes, has little to do.  Whole
+// calls by lanes along x and by rows, Float32, us:
+//                          Marching Cubes   tetrahedra    surface nets
+//   1000000 x 4 x 4 noise    1010   2165     1409   6198    775   2712
+//   131072 x 8 x 8 noise      595    431      939    988    402    423
+//   100000 x 40 x 3 noise     623    388     1041    985    467    384
+//   100000 x 16 x 16 noise   1719    715     2896   1958   1129    561
+//   21675 x 3 x 129 sparse     82    101      106    189     95     90
+//   12905 x 10 x 65 sparse     81     85       97    147     87     92
+//   10591 x 24 x 33 sparse     84     88      113    141     97     91
+// (sparse: a surface in a third of the planes; such volumes of few or long rows
+// of cells lose up to a quarter of a unit, in tetrahedra half a one, where
+// dense ones gain).  With fewer planes only the shortest ones lose (2000 x 2 x 2
+// Marching Cubes 38 and 44; 2000 x 10 x 4 59 and 60).
+bool rows_default(const Plan& p, const Geom& rows, const RowsGeom& r) {
+  if (p.family == 2 || r.upx > 1) return true;
+  const int64_t cells = (int64_t)(rows.ny - 1) * (rows.nz - 1);
+  if (rows.units < 4096) return rows.units < 1024 || cells >= 16;
+  return cells >= (p.method == MT ? 1024 : 512) || (cells >= 60 && rows.ny >= 10 && rows.nz <= 17);
+}
+
 // By default a single volume goes to them from a number of units on in
 // Marching Tetrahedra, whose waves are the longest: with few units a dense
 // one leaves most of the device idle, where the tiles of the lanes-along-x
@@ -675,7 +697,8 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
   RowsGeom rg{};
   Geom gr = g;
   void* bits = nullptr;  // sample bits | vertex prefixes | counter of shared units | their groups
-  if (rows_family(pl) && rows_geom(pl, &gr, &rg) && rows_single(pl, gr) &&
+  if (rows_family(pl) && rows_geom(pl, &gr, &rg) && rows_default(pl, gr, rg) &&
+      rows_single(pl, gr) &&
       rows_workspace(c, gr.units, ncoords, &w,
                      rows_bytes(gr, rg) + rows_prefix_bytes(pl, gr) + rows_groups_bytes(pl.method),
                      &bits))
@@ -861,7 +884,8 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (geoms[v].units > 0 && !fields[v].data)
       return fail(c, MSH_ERR_ARGUMENT, "volume " + std::to_string(v) + ": null field data");
     rgeoms[v] = geoms[v];
-    b.rows[v] = rows_family(b.plans[v]) && rows_geom(b.plans[v], &rgeoms[v], &rows[v]);
+    b.rows[v] = rows_family(b.plans[v]) && rows_geom(b.plans[v], &rgeoms[v], &rows[v]) &&
+                rows_default(b.plans[v], rgeoms[v], rows[v]);
   }
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, MSH_ERR_DEVICE, "hipSetDevice");
 
@@ -880,10 +904,16 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   }
   Workspace w{};
   void* bits = nullptr;
-  int64_t runits = units;
+  int64_t runits = units, rblocks = 0;
   size_t extra = 0;
   for (int v = 0; v < n; ++v) {
     if (!b.rows[v]) continue;
+    rblocks += rows[v].blocks;
+    if (rblocks >= kMaxBlocks) {  // (the others' launches take as many tiles as there are)
+      b.rows[v] = 0;
+      rblocks -= rows[v].blocks;
+      continue;
+    }
     runits += rgeoms[v].units - geoms[v].units;
     extra += rows_bytes(rgeoms[v], rows[v]) + rows_prefix_bytes(b.plans[v], rgeoms[v]);
   }

@@ -216,7 +216,11 @@ CoordArgs coord_args(const Plan& p, const Geom& g, double* coords);
 struct RowsGeom {
   int64_t xs;
   int32_t sw, cw, upx;
+  int64_t blocks;  // of its largest launch, at most
 };
+// blocks of 256 threads that a launch may have (2^32 threads), less the first
+// ones of an emit
+constexpr int64_t kMaxBlocks = (1ll << 24) - 4096;
 bool rows_geom(const Plan& p, Geom* g, RowsGeom* r);
 // bytes of the sample bits, and VolArgs of a volume with its bits there
 size_t rows_bytes(const Geom& g, const RowsGeom& r);

@@ -375,8 +375,9 @@ bool rows_geom(const Plan& p, Geom* g, RowsGeom* r) {
   r->upx = (int32_t)((words + 63) / 64);
   r->xs = (plane + 31) / 32 * 32;
   const int64_t units = (int64_t)(g->nx - 1) * r->upx;
-  if (units >= (1ll << 31) || (int64_t)((g->nx + 63) / 64) * ((plane + 7) / 8) >= (1ll << 31))
-    return false;  // block numbers are 32-bit
+  r->blocks = std::max((int64_t)(g->nx + 127) / 128 * ((plane + 3) / 4),
+                       (int64_t)(g->nx / 2 + 1) * r->upx);
+  if (r->blocks >= kMaxBlocks) return false;
   g->units = units;
   return true;
 }
