@@ -35,8 +35,8 @@ struct Launch {
   int64_t nblocks = 0;
   double cost = 0;          // estimated work: cells weighted by method
   // emits of the row kernels: the launch's shared units (RowsGroup)
-  RowsGroup* groups = nullptr;
-  uint32_t* ngroups = nullptr;
+  RowsGroups groups{};
+  int list = 2;             // the list it takes (rows_list), and blocks for that
   int32_t xblocks = 0;
 };
 
@@ -86,7 +86,7 @@ struct BatchState {
   std::vector<Launch> bits, counts, emits;  // bits: sample-bit launches of the row kernels
   std::vector<char> rows;          // per volume: goes through the row kernels
   std::vector<int64_t> sizes;      // 4 per volume: first vertex, nverts, first face, nfaces
-  std::vector<uint32_t> ngroups;   // per emit launch: groups of shared units
+  std::vector<uint32_t> ngroups;   // 2 per emit launch: groups of shared units
   int64_t units = 0, ncoords = 0, cblocks = 0, eblocks = 0, bblocks = 0;
   size_t ctr_off = 0;              // work-queue counters in the batch workspace: 8 per
                                    // count launch, then 8 per emit launch
@@ -723,9 +723,7 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
       char* const wpre = (char*)bits + rows_bytes(gr, rg);
       char* const shared = wpre + rows_prefix_bytes(pl, gr);
       rows_vol(rg, bits, wpre, &a);
-      a.ngroups = (uint32_t*)shared;
-      a.groups = (RowsGroup*)(shared + kGroupsAt);
-      a.gcap = rows_group_cap(pl.method);
+      a.groups = rows_groups(pl.method, shared + kGroupsAt, (uint32_t*)shared);
     }
     c->pinned[0] = c->pinned[1] = c->pinned[3] = -1;
     const CoordArgs ca = coord_args(pl, g, w.coords);
@@ -750,8 +748,11 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
     nfc = c->pinned[3];
     if (bits) {
       rows_emit_tiling(&a, nv);
-      a.shared = (uint32_t)c->pinned[0];
-      a.xblocks = rows_xblocks(a.shared, a.gcap);
+      const uint32_t n[3] = {(uint32_t)c->pinned[0], (uint32_t)((uint64_t)c->pinned[0] >> 32), 0};
+      const int list = rows_list(pl.method, n);
+      a.taken = a.groups.list[list & 1];
+      a.shared = n[list];
+      a.xblocks = rows_xblocks(a.shared);
     }
     c->vol = a;
   }
@@ -1037,10 +1038,10 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   const size_t b_cmap = align256(4 * (size_t)(cblocks + 1));
   const size_t b_emap = align256(4 * (size_t)(eblocks + 1));
   const size_t b_bmap = bits ? align256(4 * (size_t)(bblocks + 1)) : 0;
-  const size_t b_sizes = align256(32 * (size_t)(n > 0 ? n : 1) + 4 * b.emits.size());
+  const size_t b_sizes = align256(32 * (size_t)(n > 0 ? n : 1) + 8 * b.emits.size());
   size_t b_groups = 0;
   for (const Launch& L : b.emits)
-    if (L.rows) b_groups += rows_group_cap(L.plan.method) * sizeof(RowsGroup);
+    if (L.rows) b_groups += rows_groups_bytes(L.plan.method) - kGroupsAt;
   const size_t nctr = 8 * (b.counts.size() + b.emits.size());
   const size_t b_ctr = align256(4 * (nctr + 1));
   rc = grow(c, &c->bws, &c->bws_bytes, b_vols + b_cmap + b_emap + b_sizes + b_ctr + b_bmap + b_groups,
@@ -1054,21 +1055,18 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   uint32_t* ctrs = (uint32_t*)((char*)c->bws + b.ctr_off);
   int32_t* bmap = bits ? (int32_t*)((char*)ctrs + b_ctr) : nullptr;
   uint32_t* const ngroups = (uint32_t*)(dsizes + 4 * n);
-  RowsGroup* groups = (RowsGroup*)((char*)ctrs + b_ctr + b_bmap);
+  char* groups = (char*)ctrs + b_ctr + b_bmap;
   for (size_t k = 0; k < b.emits.size(); ++k) {
     Launch& L = b.emits[k];
     if (!L.rows) continue;
-    L.ngroups = ngroups + k;
-    L.groups = groups;
-    groups += rows_group_cap(L.plan.method);
+    L.groups = rows_groups(L.plan.method, groups, ngroups + 2 * k);
+    groups += rows_groups_bytes(L.plan.method) - kGroupsAt;
   }
   for (int v = 0; v < n; ++v) {
     b.vols[v].sz = dsizes + 4 * v;
     b.vols[v].self = v;
     if (!b.rows[v]) continue;
-    b.vols[v].ngroups = b.emits[emit_of[v]].ngroups;
     b.vols[v].groups = b.emits[emit_of[v]].groups;
-    b.vols[v].gcap = rows_group_cap(b.plans[v].method);
   }
   // pinned host side: descriptors | sizes
   if (c->hbatch_bytes < b_vols + b_sizes) {
@@ -1095,7 +1093,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess && n > 0)
       e = hipMemcpyAsync(dvols, c->hbatch, sizeof(VolArgs) * (size_t)n, hipMemcpyHostToDevice,
                          c->stream);
-    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, ngroups, (int)b.emits.size(), c->stream);
+    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, ngroups, (int)(2 * b.emits.size()), c->stream);
     if (e == hipSuccess) e = launch_coords_batch(dvols, n, c->stream);
     if (e == hipSuccess && work_queues(b.counts))
       e = launch_zero_u32(ctrs, (int64_t)(8 * b.counts.size()), c->stream);
@@ -1122,7 +1120,7 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess && units > 0)
       e = launch_sizes_batch(dvols, n, w, units, dsizes, c->stream);
     if (e == hipSuccess && units > 0)
-      e = hipMemcpyAsync(hsizes, dsizes, 32 * (size_t)n + 4 * b.emits.size(), hipMemcpyDeviceToHost,
+      e = hipMemcpyAsync(hsizes, dsizes, 32 * (size_t)n + 8 * b.emits.size(), hipMemcpyDeviceToHost,
                          c->stream);
     return e;
   };
@@ -1141,10 +1139,10 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
   if (e != hipSuccess) return hip_fail(c, e, "batched count/scan");
 
   b.sizes.assign(4 * (size_t)n, 0);
-  b.ngroups.assign(b.emits.size(), 0);
+  b.ngroups.assign(2 * b.emits.size(), 0);
   if (units > 0) {
     memcpy(b.sizes.data(), hsizes, 32 * (size_t)n);
-    memcpy(b.ngroups.data(), hsizes + 4 * n, 4 * b.emits.size());
+    memcpy(b.ngroups.data(), hsizes + 4 * n, 8 * b.emits.size());
   }
   for (int v = 0; v < n; ++v) {
     if (nverts) nverts[v] = b.sizes[4 * v + 1];
@@ -1212,18 +1210,25 @@ int msh_batch_extract(void* ctx, int32_t n, const msh_field* fields, const msh_p
   uint32_t* ectr = (uint32_t*)((char*)c->bws + b.ctr_off) + 8 * b.counts.size();
   // blocks for the shared units: their number in steps, so that a repeated
   // batch with new values in its fields still repeats its launches
-  std::vector<int32_t> xblocks(b.emits.size(), 0);
+  std::vector<int32_t> xblocks(2 * b.emits.size(), 0);  // and the lists
   for (size_t k = 0; k < b.emits.size(); ++k) {
     if (!b.emits[k].rows) continue;
-    const int32_t x = rows_xblocks(b.ngroups[k], rows_group_cap(b.emits[k].plan.method));
-    while (xblocks[k] < x) xblocks[k] = xblocks[k] ? 4 * xblocks[k] : 32;
-    b.emits[k].xblocks = xblocks[k];
+    Launch& L = b.emits[k];
+    const uint32_t* const n = &b.ngroups[2 * k];
+    L.list = rows_list(L.plan.method, n);
+    const int32_t x = L.list < 2 ? rows_xblocks(n[L.list]) : 0;
+    L.xblocks = 0;
+    while (L.xblocks < x) L.xblocks = L.xblocks ? 4 * L.xblocks : 32;
+    xblocks[2 * k] = L.xblocks;
+    xblocks[2 * k + 1] = L.list;
   }
   auto shared_blocks = [](const Launch& L) {
     RowsBatch r{};
-    r.groups = L.groups;
-    r.ngroups = L.ngroups;
-    r.xblocks = L.xblocks;
+    if (L.xblocks > 0) {
+      r.groups = L.groups.list[L.list];
+      r.ngroups = L.groups.n + L.list;
+      r.xblocks = L.xblocks;
+    }
     return r;
   };
   // the output pointers travel in the descriptors (copied from hbatch by

@@ -287,35 +287,38 @@ __device__ __forceinline__ double coord_at(const CoordArgs& c, int i) {
 // The shared units of a volume of the row kernels among kScanTile units, of
 // which this thread of the block holds kScanItems, c of units first on: the
 // block counts their groups before a barrier that it has anyway (share_count),
-// and lists them after it (share_list) behind those that *o.ngroups counts, or
+// and lists them after it (share_list) behind those that o.to.n counts, or
 // with `alone` as the only ones.  One entry of the counter a tile: one a unit
 // from the count, 9 ns each, cost 256^3 Float32 value noise, whose units are
 // all full, 76 us.
 struct ShareOut {
-  RowsGroup* groups;
-  uint32_t* ngroups;
-  uint32_t cap, waves;  // waves of an emit block: parts of a group
+  RowsGroups to;
+  uint32_t cap[2], waves;  // waves of an emit block: parts of a group
   RowsCuts cuts;
   uint32_t vol;
 };
 __host__ __device__ inline ShareOut share_out(const VolArgs& a, int vol) {
-  return {a.groups, a.ngroups, a.gcap, (uint32_t)rows_emit_waves(a.method), rows_cuts(a.method),
+  return {a.groups, {rows_group_cap(a.method, 0), rows_group_cap(a.method, 1)}, (uint32_t)rows_emit_waves(a.method), rows_cuts(a.method),
           (uint32_t)vol};
 }
 struct ShareSums {
-  uint32_t w[kWaves], base;
+  uint32_t w[kWaves], base[2];
 };
 __device__ __forceinline__ uint32_t share_count(const ShareOut& o, const uint32_t (&c)[kScanItems],
                                                 ShareSums* s) {
   uint32_t mine = 0;
 #pragma unroll
-  for (int q = 0; q < kScanItems; ++q) mine += rows_parts(o.cuts, c[q] & 0xFFFF);
-  mine /= o.waves;  // (a power of two, which the parts are multiples of)
+  for (int q = 0; q < kScanItems; ++q) {
+    // (groups of the first list | of the second << 16; the parts are multiples of `waves`)
+    const uint32_t p = rows_parts(o.cuts, c[q] & 0xFFFF);
+    mine += p | (p > 0 ? 4u << 16 : 0u);
+  }
+  mine /= o.waves;
   const uint32_t incl = wave_scan_dpp(mine);
   if (lane_id() == kWave - 1) s->w[wave_id()] = incl;
   return incl - mine;
 }
-// (before: share_count's; returns the tile's groups)
+// (before: share_count's; returns the tile's groups, likewise)
 __device__ __forceinline__ uint32_t share_list(const ShareOut& o, int64_t first,
                                                const uint32_t (&c)[kScanItems], ShareSums* s,
                                                uint32_t before, bool alone) {
@@ -326,11 +329,12 @@ __device__ __forceinline__ uint32_t share_list(const ShareOut& o, int64_t first,
     all += s->w[w];
   }
   if (__builtin_expect(all == 0, 1)) return 0;
+  uint32_t at0 = at & 0xFFFF, at1 = at >> 16;
   if (!alone) {
-    if (threadIdx.x == 0) s->base = atomicAdd(o.ngroups, all);
+    if (threadIdx.x < 2) s->base[threadIdx.x] = atomicAdd(o.to.n + threadIdx.x, threadIdx.x ? all >> 16 : all & 0xFFFF);
     __syncthreads();
-    if (s->base >= o.cap) return all;
-    at += s->base;
+    at0 += s->base[0];
+    at1 += s->base[1];
   }
 #pragma unroll 1
   for (int q = 0; q < kScanItems; ++q) {
@@ -338,8 +342,11 @@ __device__ __forceinline__ uint32_t share_list(const ShareOut& o, int64_t first,
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) v = i == q ? c[i] & 0xFFFF : v;
     const uint32_t p = rows_parts(o.cuts, v);
-    for (uint32_t k = 0; k < p; k += o.waves, ++at)
-      if (at < o.cap) o.groups[at] = {o.vol, (uint32_t)first + (uint32_t)q, k, p};
+    const uint32_t u = (uint32_t)first + (uint32_t)q, quarter = p / 4;
+    for (uint32_t k = 0; k < p; k += o.waves, ++at0)
+      if (at0 < o.cap[0]) o.to.list[0][at0] = {o.vol, u, k, 1, (uint16_t)p};
+    for (uint32_t k = 0; k < p; k += o.waves * quarter, ++at1)
+      if (at1 < o.cap[1]) o.to.list[1][at1] = {o.vol, u, k, (uint16_t)quarter, (uint16_t)p};
   }
   return all;
 }

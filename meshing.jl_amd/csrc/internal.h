@@ -21,8 +21,9 @@ constexpr int rows_emit_waves(int method) { return method == SN ? 2 : 4; }
 struct RowsGroup {
   uint32_t vol;     // volume, in a batch
   uint32_t unit;
-  uint32_t first;   // its first part ..
-  uint32_t parts;   // .. of this many
+  uint32_t first;   // wave w: the unit's parts from first + w * step on, ..
+  uint16_t step;    // .. this many ..
+  uint16_t parts;   // .. of so many
 };
 constexpr int kMaxParts = 16;
 // Where the parts of a unit start.
@@ -30,10 +31,21 @@ struct RowsParts {
   uint32_t pre[kMaxParts];  // the unit's vertices | faces << 16 before it
   uint8_t word[kMaxParts];  // its first word of the unit
 };
-// Groups of an emit launch, at most: two rounds of the device's waves (with one,
-// 4096 parts, surface nets of 128^3 Float32 value noise take 141 us a call
-// instead of 100, tetrahedra of a 512^3 box 536 instead of 335).
-constexpr uint32_t rows_group_cap(int method) { return 8192 / rows_emit_waves(method); }
+// A launch's groups are listed twice: one part a wave, and a quarter of the unit
+// a wave, for launches whose first list outgrows its room.
+struct RowsGroups {
+  RowsGroup* list[2];  // room for rows_group_cap
+  uint32_t* n;         // [2]: their numbers; above that: not used
+};
+// Their room.  The first list: two rounds of the device's waves (one, 4096 parts:
+// surface nets of 128^3 Float32 value noise 141 us a call instead of 100,
+// tetrahedra of a 512^3 box 536 instead of 335).  The second, Float32 calls, us,
+// with none / 16384 / 32768 quarters: 16 x 1024 x 1024 tetrahedra of a gentle
+// surface across x 749 / 218 / 218, of value noise 963 / 968 / 732; 256 x 256 x
+// 100 value noise surface nets 151 / 128 / 128, 16 x 1024 x 1024 318 / 324 / 446.
+constexpr uint32_t rows_group_cap(int method, int list) {
+  return (list == 0 ? 8192 : method == MT ? 32768 : 16384) / rows_emit_waves(method);
+}
 // Vertices from which a unit has 4, 8 and 16 parts (about 128 cells each).
 struct RowsCuts {
   uint32_t four, eight, sixteen;
@@ -136,9 +148,8 @@ struct VolArgs {
   int32_t xblocks;         // blocks of groups before the tiles of a single emit ..
   uint32_t shared;         // .. and their groups
   RowsParts* parts;        // per unit, of the shared ones
-  RowsGroup* groups;       // room for gcap
-  uint32_t* ngroups;       // their number, while the scan counts them; above gcap no unit is shared
-  uint32_t gcap;
+  RowsGroups groups;       // as the scan lists them
+  const RowsGroup* taken;  // the list that a single emit takes
   int64_t bntiles, bblk0;  // sample-bit tiles in a batched launch, its first block there
   uint32_t cwm, cwn;       // 2^32 / cw and 2^16 / cw, rounded down and up (word_pos)
   int32_t nti, ntj;        // emit tiles along x and y
@@ -235,15 +246,20 @@ struct ScanTail {
   int64_t *voff, *foff, *totals, *host;
   CoordArgs coords;
 };
-// bytes of the group list of a launch, its counter first
+// bytes of a launch's group lists, their counters first
 constexpr size_t kGroupsAt = 256;
 constexpr size_t rows_groups_bytes(int method) {
-  return kGroupsAt + rows_group_cap(method) * sizeof(RowsGroup);
+  return kGroupsAt + (rows_group_cap(method, 0) + rows_group_cap(method, 1)) * sizeof(RowsGroup);
 }
-// blocks for n groups: none when there are too many
-inline int32_t rows_xblocks(uint32_t n, uint32_t gcap) {
-  return n > gcap ? 0 : (int32_t)((n + 7) / 8 * 8);
+// The lists of a launch, their counters at n.
+inline RowsGroups rows_groups(int method, void* lists, uint32_t* n) {
+  return {{(RowsGroup*)lists, (RowsGroup*)lists + rows_group_cap(method, 0)}, n};
 }
+// The list that a launch takes by the counters' values (0 or 1; 2: none).
+inline int rows_list(int method, const uint32_t* n) {
+  return n[0] <= rows_group_cap(method, 0) ? 0 : n[1] <= rows_group_cap(method, 1) ? 1 : 2;
+}
+inline int32_t rows_xblocks(uint32_t n) { return (int32_t)((n + 7) / 8 * 8); }
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, const ScanTail& tail, hipStream_t st);
 // A batched launch: tiles gbase .. gbase + nblocks of the batch, whose volumes
 // the map names.
@@ -276,7 +292,8 @@ hipError_t launch_coords(const Plan& p, const Geom& g, double* coords, hipStream
 hipError_t launch_count(const Plan& p, const VolArgs& a, hipStream_t st,
                         const ScanTail& tail = ScanTail{});
 // host: pinned host words that also receive the vertex and face totals
-// (at [1] and [3]) and the number of groups of shared units (at [0]), or null;
+// (at [1] and [3]) and the numbers of groups of shared units (at [0],
+// the second in its high half), or null;
 // coords: coordinate tables the scan also fills (in its one-block tile scan,
 // or block 0 of the fused apply) instead of a launch of their own, or null;
 // rows: a volume of the row kernels, whose shared units are listed, or null

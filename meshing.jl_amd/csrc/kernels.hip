@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_reduce(const uint32_t* __restri
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
   const uint64_t incl = wave_incl_scan64(scan_load(cnt, units, base, c));
   __shared__ ShareSums sums;
-  const uint32_t before = share.groups ? share_count(share, c, &sums) : 0u;
+  const uint32_t before = share.to.n ? share_count(share, c, &sums) : 0u;
   if (lane_id() == kWave - 1) s_w[wave_id()] = incl;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_reduce(const uint32_t* __restri
     for (int q = 0; q < kWaves; ++q) agg += s_w[q];
     tilesum[blockIdx.x] = agg;
   }
-  if (share.groups) (void)share_list(share, base, c, &sums, before, false);
+  if (share.to.n) (void)share_list(share, base, c, &sums, before, false);
 }
 
 constexpr int kScanTilesBlock = 1024;
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kScanTilesBlock) void k_scan_tiles(
       coords.out[i] = coord_at(coords, i);
   __shared__ int64_t s_v[kScanTilesBlock / kWave], s_f[kScanTilesBlock / kWave];
   const int t = threadIdx.x, lane = lane_id(), wv = t / kWave;
-  const int64_t shared = ngroups ? (int64_t)*ngroups : 0;
+  const int64_t shared = ngroups ? (int64_t)ngroups[0] | ((int64_t)ngroups[1] << 32) : 0;
   const int64_t per = (ntiles + kScanTilesBlock - 1) / kScanTilesBlock;
   const int64_t lo = t * per, hi = lo + per < ntiles ? lo + per : ntiles;
   int64_t sv = 0, sf = 0;  // int64: the sums over many tiles outgrow 32 bits
@@ -256,7 +256,8 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply_sums(
   uint32_t c[kScanItems];
   const int wv = wave_id(), lane = lane_id();
   int64_t shared = 0;  // (read early, for the last block)
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && ngroups) shared = (int64_t)*ngroups;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && ngroups)
+    shared = (int64_t)ngroups[0] | ((int64_t)ngroups[1] << 32);
   // this tile's offset: the sums of the tiles before it (int64: they
   // outgrow 32 bits over many tiles)
   int64_t pv = 0, pf = 0;
@@ -888,12 +889,12 @@ hipError_t launch_scan(const Geom& g, const Workspace& w, hipStream_t st, int64_
   if (nt <= kScanFuseTiles) {
     hipLaunchKernelGGL(k_scan_apply_sums, dim3((unsigned)nt), dim3(kBlock), 0, st, w.cnt,
                        g.units, (const uint64_t*)w.tilesum, w.voff, w.foff, w.totals, host,
-                       coords ? *coords : CoordArgs{}, share.ngroups);
+                       coords ? *coords : CoordArgs{}, share.to.n);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanTilesBlock), 0, st,
                      (const uint64_t*)w.tilesum, nt, w.tileoff, w.totals, host,
-                     coords ? *coords : CoordArgs{}, share.ngroups);
+                     coords ? *coords : CoordArgs{}, share.to.n);
   hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nt), dim3(kBlock), 0, st, w.cnt, g.units,
                      (const int64_t*)w.tileoff, w.voff, w.foff);
   return hipGetLastError();

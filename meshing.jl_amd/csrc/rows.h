@@ -220,8 +220,8 @@ __device__ __forceinline__ int64_t word_vertex(const VolArgs& a, int x, uint32_t
 // (rows_parts, note_parts): the count pass leaves where they start, the scan
 // lists the parts in groups (RowsGroup), and the emit's first blocks take a
 // group each, a part a wave, while the waves of the tiles leave these units
-// out (81 us and 106).  Where many units are full the device is full
-// without this: above rows_group_cap none is shared.
+// out (81 us and 106).  Where many units are full a wave takes a quarter of one,
+// and where that is too many (rows_group_cap) the device is full without this.
 
 // What a wave of an emit block works on: units [g0, g1) of x plane x, or with
 // a group a part of one unit.
@@ -303,7 +303,7 @@ __device__ __forceinline__ RowsBlock rows_block(const VolArgs& a) {
   r.share = a.xblocks > 0;
   if (__builtin_expect((int)blockIdx.x < a.xblocks, 0)) {
     r.none = blockIdx.x >= a.shared;
-    r.grp = a.groups + blockIdx.x;
+    r.grp = a.taken + blockIdx.x;
     r.share = false;
   }
   return r;
@@ -336,15 +336,15 @@ __device__ __forceinline__ RowsWork rows_work(const VolArgs& a, const RowsBlock&
   k.g1 = min(k.g0 + a.ue, a.upx);
   k.wn = kWave;
   if (__builtin_expect(grp != nullptr, 0)) {
-    const uint32_t u = grp->unit, parts = grp->parts;
-    const uint32_t part = grp->first + (uint32_t)__builtin_amdgcn_readfirstlane(wave_id());
+    const uint32_t u = grp->unit, step = grp->step;
+    const uint32_t part = grp->first + step * (uint32_t)__builtin_amdgcn_readfirstlane(wave_id());
     const RowsParts& cut = a.parts[u];
     const uint32_t pre = cut.pre[part];
     k.x = (int)(u / (uint32_t)a.upx);
     k.g0 = (int)(u - (uint32_t)k.x * (uint32_t)a.upx);
     k.g1 = k.g0 + 1;
     k.w0 = cut.word[part];
-    k.wn = (part + 1 < parts ? (int)cut.word[part + 1] : kWave) - k.w0;
+    k.wn = (part + step < grp->parts ? (int)cut.word[part + step] : kWave) - k.w0;
     k.vpre = pre & 0xFFFF;
     k.fpre = pre >> 16;
   }

@@ -98,7 +98,7 @@ __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
 
 template <typename T, int PW, int E, int WX, bool NT>
 __global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.ngroups = 0;  // for the scan
+  if (blockIdx.x == 0 && threadIdx.x < 2) a.groups.n[threadIdx.x] = 0;  // for the scan
   bits_tile<T, PW, E, WX, NT>(a, blockIdx.x);
 }
 
@@ -293,7 +293,7 @@ __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
   }
   const uint64_t incl = wave_incl_scan64(sum);
   __shared__ ShareSums sums;
-  const ShareOut share{a.groups, a.ngroups, a.gcap, (uint32_t)rows_emit_waves(METHOD),
+  const ShareOut share{a.groups, {rows_group_cap(METHOD, 0), rows_group_cap(METHOD, 1)}, (uint32_t)rows_emit_waves(METHOD),
                        rows_cuts(METHOD), 0};
   const uint32_t groups = share_count(share, c, &sums);
   if (lane_id() == kWave - 1) s_w[wave_id()] = incl;
@@ -323,7 +323,7 @@ __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
     t.totals[2] = 0;
     t.totals[3] = nf;
     *t.done = 0;
-    t.host[0] = (int64_t)shared;
+    t.host[0] = (int64_t)(shared & 0xFFFF) | ((int64_t)(shared >> 16) << 32);
     t.host[1] = nv;
     t.host[3] = nf;
     __threadfence_system();

@@ -17,10 +17,11 @@ def method_of(pkg, name):
 
 @pytest.fixture
 def rows(pkg):
-    # (small tetrahedra volumes go to the row kernels only when these are asked for)
+    # (some of these volumes go to the row kernels only when they are asked for)
     def reset(family):
-        for t in ("float32", "float64"):
-            pkg.set_kernel_family(method_of(pkg, "mt"), t, family)
+        for name in ("mc", "mt", "sn"):
+            for t in ("float32", "float64"):
+                pkg.set_kernel_family(method_of(pkg, name), t, family)
     reset(2)
     yield
     reset(-1)
@@ -52,9 +53,16 @@ def test_planes_at_the_counts(pkg, oracle, rows, name, dtype, nz):
 
 
 @pytest.mark.parametrize("name", ["mc", "mt", "sn"])
-@pytest.mark.parametrize("nx", [34, 64, 80])  # 64: 8064 parts, 80: more than are shared
+@pytest.mark.parametrize("nx", [34, 64, 80])  # 64: 8064 parts, 80: too many but by quarters
 def test_many_full_units(pkg, oracle, rows, name, nx):
     f = np.random.default_rng(nx).standard_normal((nx, 129, 129)).astype(np.float32)
+    assert check(pkg, oracle, f, name) > 100000
+
+
+@pytest.mark.parametrize("name", ["mc", "mt", "sn"])
+@pytest.mark.parametrize("nx", [2049, 2050, 4097, 4098, 8193, 8194])  # 2048, 4096, 8192 full units and one more
+def test_most_shared_units(pkg, oracle, rows, name, nx):
+    f = np.random.default_rng(nx).standard_normal((nx, 10, 33)).astype(np.float32)
     assert check(pkg, oracle, f, name) > 100000
 
 
@@ -74,7 +82,8 @@ def test_batches(pkg, oracle, name):
     host = [plane((40, 70, 65), np.float32, 0.2, 0.01), noise((30, 40, 50), 1, np.float32),
             plane((20, 130, 33), np.float64, -0.4, 0.0), np.ones((9, 9, 9), np.float32),
             plane((33, 65, 129), np.float32, 0.7, 0.02, 3),
-            np.random.default_rng(0).standard_normal((12, 66, 66)).astype(np.float32)]
+            np.random.default_rng(0).standard_normal((12, 66, 66)).astype(np.float32),
+            np.random.default_rng(1).standard_normal((70, 129, 129)).astype(np.float64)]
     res = pkg.isosurface_batch([dev_field(f) for f in host], method_of(pkg, name))
     for f, (V, F) in zip(host, res):
         Vo, Fo = oracle.isosurface(f, name, iso=0)
