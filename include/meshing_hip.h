@@ -134,10 +134,10 @@ int msh_batch_graph_launches(void* ctx, int64_t* count_phase, int64_t* emit_phas
  * type throughout and Float64 axes; otherwise lanes along x with full-depth
  * bricks), 1 lanes along z and 0 a generic kernel; each family falls back to
  * the next one down for volumes it cannot take.
- * msh_autotune counts the given field, times the emit of every family that
- * takes it (the best of 3 to 50 launches each, about 2 ms, on the
- * context's stream, into a scratch buffer) and records the fastest for the
- * field's (method, element type, size class) in the context, where later
+ * msh_autotune times the whole call, count and emit, of every family that
+ * takes the given field (from device memory; the best of 3 to 50 calls each,
+ * about 2 ms, on the context's stream, into a scratch buffer) and records the
+ * fastest for the field's (method, element type, size class) in the context, where later
  * msh_count and msh_batch_count calls on volumes of that class use it (size
  * classes by cell count: below 2^20, below 2^23, larger; a batch of mixed
  * sizes then runs each volume with its class's choice);
@@ -147,9 +147,10 @@ int msh_batch_graph_launches(void* ctx, int64_t* count_phase, int64_t* emit_phas
  * loop). */
 int msh_autotune(void* ctx, const msh_field* field, const msh_params* params, int32_t* family);
 /* msh_autotune for a batch: the batch's volumes are grouped by (method,
- * element type, size class), and each group's batched emit (all its volumes
- * in one msh_batch_extract, device outputs in a scratch buffer) is timed
- * with every family that takes all of them (a warm-up, then the best of 3);
+ * element type, size class), and each group's batched call (all its volumes
+ * in one msh_batch_count and msh_batch_extract, device outputs in a scratch
+ * buffer) is timed with every family that takes all of them (the best of 3
+ * after two warm-ups);
  * the fastest is recorded for the group; then, since the groups' launches
  * run side by side, one pass over the groups (most volumes first) times the
  * whole batch with each other family that takes the group and keeps a

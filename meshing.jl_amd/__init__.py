@@ -338,7 +338,7 @@ def isosurface_batch(fields, methods=None, axes=None, device=0):
 
 
 def autotune(sdf, method=None, *args, X=(-1, 1), Y=(-1, 1), Z=(-1, 1), device=0):
-    """Time every emit kernel family on this field and method and keep the
+    """Time the whole call with every kernel family on this field and method and keep the
     fastest for its (method, element type, size class) in the device's
     context (size classes by cell count: below 2^20, below 2^23, larger);
     later calls of isosurface, isosurface_batch and the server on that
@@ -361,7 +361,7 @@ def autotune(sdf, method=None, *args, X=(-1, 1), Y=(-1, 1), Z=(-1, 1), device=0)
 
 def autotune_batch(fields, methods=None, axes=None):
     """:func:`autotune` for a batch of device fields: each (method, element
-    type, size class) group of the batch is timed as one batched emit with
+    type, size class) group of the batch is timed as one batch with
     every kernel family, and the fastest is kept for that group; later
     batches (and single calls) on the device use it.  Returns the family
     chosen for each volume."""

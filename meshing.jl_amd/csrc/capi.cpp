@@ -14,6 +14,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <mutex>
 #include <new>
 #include <string>
@@ -511,6 +512,15 @@ int setup_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t
   return MSH_OK;
 }
 
+// Whether a volume set to family fam runs it, and not a lower one (family 3
+// means full-depth bricks where there are no half-depth ones; it is family 2
+// only to a volume that the row kernels do not take).
+bool takes_family(int fam, const Plan& p, VolArgs a) {
+  if (a.bits) return fam == 2;
+  const int runs = variant_family(emit_variant(p, &a));
+  return fam == 3 ? runs >= 2 : runs == fam;
+}
+
 // Workspace with the sample bits of the row kernels; false, with no error
 // left, where they are not to take that much (msh_set_limit) or the device
 // has no room: the other kernels, which need less, take the call then.
@@ -520,6 +530,10 @@ bool rows_workspace(Ctx* c, int64_t units, int64_t ncoords, Workspace* w, size_t
   *bits = nullptr;
   (void)hipGetLastError();
   return false;
+}
+
+double elapsed_us(std::chrono::steady_clock::time_point since) {
+  return std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - since).count();
 }
 
 // The row kernels serve the default family and family 2.
@@ -1324,45 +1338,46 @@ int msh_autotune(void* ctx, const msh_field* f, const msh_params* p, int32_t* fa
   const size_t vbytes = align256((size_t)nv * 3 * osz), fbytes = (size_t)nf * 3 * 8;
   rc = grow(c, &c->ostage, &c->ostage_bytes, vbytes + fbytes + 256, "autotune output buffer");
   if (rc) return rc;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  hipError_t e = hipEventCreate(&e0);
-  if (e == hipSuccess) e = hipEventCreate(&e1);
+  // (a host field has been uploaded by the count above)
+  msh_field df = *f;
+  if (f->memory == MSH_HOST) {
+    df.memory = MSH_DEVICE;
+    df.data = c->fstage;
+  }
+  hipError_t e = hipSuccess;
   int best = -1;
-  float best_ms = 0.f;
+  double best_us = 0;
   const int before = c->family[base.method][base.T][cls];
-  for (int fam = 3; fam >= 0 && e == hipSuccess; --fam) {
-    // the families count in units of their own
+  for (int fam = 3; fam >= 0 && e == hipSuccess && rc == MSH_OK; --fam) {
     c->family[base.method][base.T][cls] = fam;
-    rc = msh_count(ctx, f, p, &nv, &nf);
-    if (rc) break;
-    const Plan q = c->plan;
-    VolArgs a = c->vol;
-    a.verts = c->ostage;
-    a.faces = (int64_t*)((char*)c->ostage + vbytes);
-    VolArgs probe = a;
-    if (!a.bits && variant_family(emit_variant(q, &probe)) != fam) continue;  // not for this volume
-    e = launch_emit(q, a, c->stream);  // warm-up
-    // the best of at least 3 launches, and of as many as fill about 2 ms
-    // (short launches vary more)
-    float ms = 0.f;
+    // the whole call, as the families count in ways of their own: after a
+    // warm-up the best of at least 3 calls, and of as many as fill about 2 ms
+    // (short ones vary more)
+    double us = 0;
     int reps = 3;
-    for (int rep = 0; rep < reps && e == hipSuccess; ++rep) {
-      e = hipEventRecord(e0, c->stream);
-      if (e == hipSuccess) e = launch_emit(q, a, c->stream);
-      if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
-      if (e == hipSuccess) e = hipEventSynchronize(e1);
-      float t = 0.f;
-      if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
-      if (e == hipSuccess && (rep == 0 || t < ms)) ms = t;
-      if (rep == 0 && t > 0.f) reps = t >= 2.f / 3 ? 3 : (int)(2.f / t) < 50 ? (int)(2.f / t) : 50;
+    bool takes = true;
+    for (int rep = -1; rep < reps && e == hipSuccess; ++rep) {
+      const auto t0 = std::chrono::steady_clock::now();
+      rc = msh_count(ctx, &df, p, &nv, &nf);
+      if (rc) break;
+      VolArgs a = c->vol;
+      a.verts = c->ostage;
+      a.faces = (int64_t*)((char*)c->ostage + vbytes);
+      if (rep < 0) {
+        takes = takes_family(fam, c->plan, a);
+        if (!takes) break;  // not for this volume
+      }
+      e = launch_emit(c->plan, a, c->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+      const double t = elapsed_us(t0);
+      if (rep == 0 || (rep > 0 && t < us)) us = t;
+      if (rep == 0) reps = std::clamp((int)(2000.0 / std::max(t, 1.0)), 3, 50);
     }
-    if (e == hipSuccess && (best < 0 || ms < best_ms)) {
+    if (rc == MSH_OK && e == hipSuccess && takes && (best < 0 || us < best_us)) {
       best = fam;
-      best_ms = ms;
+      best_us = us;
     }
   }
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
   if (rc || e != hipSuccess) c->family[base.method][base.T][cls] = before;
   if (rc) return rc;
   if (e != hipSuccess) return hip_fail(c, e, "autotune");
@@ -1395,10 +1410,23 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
     members[g].push_back(v);
     group[v] = (int)g;
   }
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  hipError_t e = hipEventCreate(&e0);
-  if (e == hipSuccess) e = hipEventCreate(&e1);
-  int rc = e == hipSuccess ? MSH_OK : hip_fail(c, e, "autotune events");
+  int rc = MSH_OK;
+  // A batch's count and emit together: the first two calls (the second
+  // captures the phases' graphs) are warm-ups, then the best of 3.
+  auto time_batch = [&](int m, const msh_field* fs, const msh_params* ps, void* const* vp,
+                        int64_t* const* fp, double* us) -> int {
+    for (int rep = -2; rep < 3; ++rep) {
+      const auto t0 = std::chrono::steady_clock::now();
+      int r = msh_batch_count(ctx, m, fs, ps, nullptr, nullptr);
+      if (r == MSH_OK) r = msh_batch_extract(ctx, m, fs, ps, vp, fp, MSH_DEVICE);
+      if (r) return r;
+      const hipError_t he = hipStreamSynchronize(c->stream);
+      if (he != hipSuccess) return hip_fail(c, he, "autotune");
+      const double t = elapsed_us(t0);
+      if (rep == 0 || (rep > 0 && t < *us)) *us = t;
+    }
+    return MSH_OK;
+  };
   std::vector<int> best((size_t)gkey.size(), -1);
   for (size_t g = 0; g < gkey.size() && rc == MSH_OK; ++g) {
     const int method = gkey[g] / (3 * kSizeClasses), T = (gkey[g] / kSizeClasses) % 3,
@@ -1410,7 +1438,7 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
       fs[i] = fields[members[g][i]];
       ps[i] = params[members[g][i]];
     }
-    float best_ms = 0.f;
+    double best_us = 0;
     for (int fam = 3; fam >= 0 && rc == MSH_OK; --fam) {
       c->family[method][T][cls] = fam;
       std::vector<int64_t> nv(m), nf(m);
@@ -1420,9 +1448,7 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
       // same launch as a lower family's)
       bool takes = true;
       for (size_t i = 0; i < m && takes; ++i) {
-        Plan q = c->batch.plans[i];
-        VolArgs probe = c->batch.vols[i];
-        takes = probe.bits ? fam == 2 : variant_family(emit_variant(q, &probe)) == fam;
+        takes = takes_family(fam, c->batch.plans[i], c->batch.vols[i]);
       }
       if (!takes) continue;
       size_t total = 256;
@@ -1440,23 +1466,11 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
         fp[i] = (int64_t*)((char*)c->ostage + off);
         off += align256((size_t)nf[i] * 24);
       }
-      float ms = 0.f;
-      for (int rep = 0; rep < 4 && rc == MSH_OK; ++rep) {  // a warm-up, then the best of 3
-        e = hipEventRecord(e0, c->stream);
-        if (e == hipSuccess)
-          rc = msh_batch_extract(ctx, (int32_t)m, fs.data(), ps.data(), vp.data(), fp.data(),
-                                 MSH_DEVICE);
-        if (rc) break;
-        if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(e1);
-        float t = 0.f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
-        if (e != hipSuccess) rc = hip_fail(c, e, "autotune");
-        if (rep == 1 || (rep > 1 && t < ms)) ms = t;
-      }
-      if (rc == MSH_OK && (best[g] < 0 || ms < best_ms)) {
+      double us = 0;
+      rc = time_batch((int)m, fs.data(), ps.data(), vp.data(), fp.data(), &us);
+      if (rc == MSH_OK && (best[g] < 0 || us < best_us)) {
         best[g] = fam;
-        best_ms = ms;
+        best_us = us;
       }
     }
     c->family[method][T][cls] = best[g];
@@ -1464,20 +1478,18 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
   // Then the whole batch: its groups' launches run side by side (Spread),
   // so a group's fastest shape alone need not be fastest beside the others.
   // One pass over the groups, most volumes first, keeps a change of one
-  // group's family when it takes the whole batch's emit 1% below the best so
+  // group's family when it takes the whole batch 1% below the best so
   // far (skipped when the device has no room for all the outputs at once).
   // took: every volume of group g takes family fam.
   bool no_room = false;
-  auto time_all = [&](int g, int fam, float* ms, bool* took) -> int {
+  auto time_all = [&](int g, int fam, double* us, bool* took) -> int {
     std::vector<int64_t> nv((size_t)n), nf((size_t)n);
     int r = msh_batch_count(ctx, n, fields, params, nv.data(), nf.data());
     if (r) return r;
     *took = true;
     if (g >= 0)
-      for (int v : members[(size_t)g]) {
-        VolArgs probe = c->batch.vols[v];
-        *took = *took && (probe.bits ? fam == 2 : variant_family(emit_variant(c->batch.plans[v], &probe)) == fam);
-      }
+      for (int v : members[(size_t)g])
+        *took = *took && takes_family(fam, c->batch.plans[v], c->batch.vols[v]);
     if (!*took) return MSH_OK;
     size_t total = 256;
     for (int v = 0; v < n; ++v)
@@ -1500,22 +1512,10 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
       fp[v] = (int64_t*)((char*)c->ostage + off);
       off += align256((size_t)nf[v] * 24);
     }
-    for (int rep = 0; rep < 4; ++rep) {  // a warm-up, then the best of 3
-      hipError_t he = hipEventRecord(e0, c->stream);
-      if (he != hipSuccess) return hip_fail(c, he, "autotune");
-      r = msh_batch_extract(ctx, n, fields, params, vp.data(), fp.data(), MSH_DEVICE);
-      if (r) return r;
-      he = hipEventRecord(e1, c->stream);
-      if (he == hipSuccess) he = hipEventSynchronize(e1);
-      float t = 0.f;
-      if (he == hipSuccess) he = hipEventElapsedTime(&t, e0, e1);
-      if (he != hipSuccess) return hip_fail(c, he, "autotune");
-      if (rep == 1 || (rep > 1 && t < *ms)) *ms = t;
-    }
-    return MSH_OK;
+    return time_batch(n, fields, params, vp.data(), fp.data(), us);
   };
   if (rc == MSH_OK && gkey.size() > 1) {
-    float cur = 0.f;
+    double cur = 0;
     bool took = true;
     rc = time_all(-1, 0, &cur, &took);
     // (with no room for the whole batch there is nothing to compare against)
@@ -1529,20 +1529,18 @@ int msh_autotune_batch(void* ctx, int32_t n, const msh_field* fields, const msh_
       for (int fam = 3; fam >= 0 && rc == MSH_OK; --fam) {
         if (fam == best[g]) continue;
         c->family[method][T][cls] = fam;
-        float ms = 0.f;
-        rc = time_all((int)g, fam, &ms, &took);
+        double us = 0;
+        rc = time_all((int)g, fam, &us, &took);
         if (no_room) break;
-        if (rc == MSH_OK && took && ms < 0.99f * cur) {
+        if (rc == MSH_OK && took && us < 0.99 * cur) {
           best[g] = fam;
-          cur = ms;
+          cur = us;
         }
       }
       c->family[method][T][cls] = best[g];
       if (rc || no_room) break;
     }
   }
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
   c->batch.have = false;  // the timing batches are not the caller's
   c->have = false;
   if (rc) return rc;

@@ -1,0 +1,66 @@
+"""The autotuner's choice against the whole call: a family that its emit alone
+would not recommend (its count takes longer), or that only lanes along x with
+full-depth bricks serve (tetrahedra), and a host field."""
+import time
+
+import numpy as np
+import pytest
+
+from helpers import assert_same_mesh, dev_field, noise
+
+pytestmark = pytest.mark.gpu
+
+
+def method_of(pkg, name):
+    return {"mc": pkg.MarchingCubes, "mt": pkg.MarchingTetrahedra,
+            "sn": pkg.NaiveSurfaceNets}[name](iso=0)
+
+
+def call_time(pkg, f, m):
+    import torch
+    best = None
+    for _ in range(20):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        pkg.isosurface(f, m)
+        torch.cuda.synchronize()
+        t = time.perf_counter() - t
+        best = t if best is None or t < best else best
+    return best
+
+
+@pytest.fixture
+def reset(pkg):
+    yield
+    for name in ("mc", "mt", "sn"):
+        pkg.set_kernel_family(method_of(pkg, name), "float32", -1)
+
+
+def across_x(shape):
+    x, y, z = (np.linspace(-1, 1, n) for n in shape)
+    return (x[:, None, None] - 0.15 * np.sin(5 * y)[None, :, None] * np.cos(4 * z)[None, None, :]).astype(np.float32)
+
+
+@pytest.mark.parametrize("name,shape", [("mt", (24, 24, 24)), ("mt", (160, 160, 160)), ("mc", (16, 2048, 2048)),
+                                        ("mc", (100000, 4, 8)), ("sn", (64, 512, 512))])
+def test_choice_is_among_the_fastest(pkg, reset, name, shape):
+    f, m = dev_field(across_x(shape)), method_of(pkg, name)
+    times = {}
+    for family in (3, 2, 1, 0):
+        pkg.set_kernel_family(m, "float32", family)
+        times[family] = call_time(pkg, f, m)
+    pkg.set_kernel_family(m, "float32", -1)
+    chosen = pkg.autotune(f, m)
+    assert times[chosen] < 1.25 * min(times.values()), (chosen, times)
+
+
+@pytest.mark.parametrize("name", ["mc", "mt", "sn"])
+def test_host_field(pkg, oracle, reset, name):
+    f, m = np.asfortranarray(noise((40, 30, 50), 3, np.float32)), method_of(pkg, name)
+    assert pkg.autotune(f, m) in (0, 1, 2, 3)
+    Vo, Fo = oracle.isosurface(f, name, iso=0)
+    for g in (f, dev_field(f)):
+        V, F = pkg.isosurface(g, m)
+        if not isinstance(V, np.ndarray):
+            V, F = V.cpu().numpy(), F.cpu().numpy()
+        assert_same_mesh(V, F, Vo, Fo)
