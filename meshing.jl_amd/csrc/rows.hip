@@ -96,6 +96,49 @@ __device__ __forceinline__ void bits_tile(const VolArgs& a, int64_t t) {
   }
 }
 
+// A field of few columns along x leaves most of a tile's lanes on columns that
+// others have: its columns are dealt to the lanes along x and y alike, as they
+// lie in memory, and a lane makes kNarrowWords words of its column (2, 8, 16 and
+// 32 x 2048 x 2048 Float32 124, 128, 147 and 188 us by the tiles above, 10, 24,
+// 48 and 125 so; 48 x 1024 x 1024 takes 39 by those), as long as that makes
+// blocks enough to fill the device.
+constexpr int kNarrow = 32, kNarrowWords = 4;
+__host__ __device__ inline int64_t narrow_tiles(const VolArgs& a) {  // 0: not by these
+  const int64_t n = ((int64_t)a.g.nx * a.g.ny + kBlock - 1) / kBlock *
+                    ((a.sw + kNarrowWords - 1) / kNarrowWords);
+  return a.g.nx <= kNarrow && n >= 256 ? n : 0;
+}
+template <typename T, bool NT>
+__device__ __forceinline__ void narrow_tile(const VolArgs& a, int64_t t) {
+  const Geom g = a.g;
+  const T thr = (T)a.thr;
+  const uint32_t cols = (uint32_t)g.nx * (uint32_t)g.ny, nb = (cols + kBlock - 1) / kBlock;
+  const uint32_t tw = (uint32_t)t / nb, c = ((uint32_t)t - tw * nb) * kBlock + threadIdx.x;
+  if (c >= cols) return;
+  const uint32_t y = c / (uint32_t)g.nx, x = c - y * (uint32_t)g.nx;
+  const uint64_t pbytes = (uint64_t)cols * sizeof(T);
+  uint32_t* const out = a.bits + (int64_t)x * a.xs + (int64_t)y * a.sw;
+#pragma unroll 1
+  for (int k = 0; k < kNarrowWords; ++k) {
+    const int w = (int)tw * kNarrowWords + k;
+    if (w >= a.sw) return;
+    const int n = min(32, g.nz - 32 * w);  // samples of this word
+    const char* col = (const char*)a.f + (uint64_t)(32 * w) * pbytes + (uint64_t)c * sizeof(T);
+    Vec<T, 1> v[32];
+#pragma unroll
+    for (int z = 0; z < 32; ++z) v[z] = load_vec<T, 1, NT>(col + (uint64_t)min(z, n - 1) * pbytes);
+    uint32_t word = 0;
+#pragma unroll
+    for (int z = 0; z < 32; ++z) word |= v[z].v[0] < thr ? 1u << z : 0u;
+    out[w] = n < 32 ? word & ((1u << n) - 1u) : word;
+  }
+}
+template <typename T, bool NT>
+__global__ __launch_bounds__(kBlock) void k_bits_narrow(VolArgs a) {
+  if (blockIdx.x == 0 && threadIdx.x < 2) a.groups.n[threadIdx.x] = 0;  // for the scan
+  narrow_tile<T, NT>(a, blockIdx.x);
+}
+
 template <typename T, int PW, int E, int WX, bool NT>
 __global__ __launch_bounds__(kBlock) void k_bits(VolArgs a) {
   if (blockIdx.x == 0 && threadIdx.x < 2) a.groups.n[threadIdx.x] = 0;  // for the scan
@@ -108,7 +151,10 @@ __global__ __launch_bounds__(kBlock) void k_bits_b(const VolArgs* __restrict__ v
                                                    const int32_t* __restrict__ bmap, int64_t gbase) {
   const int64_t b = gbase + blockIdx.x;
   const VolArgs a = vols[__builtin_amdgcn_readfirstlane(bmap[b])];
-  bits_tile<T, PW, E, 1, false>(a, b - a.bblk0);
+  if (narrow_tiles(a) > 0)
+    narrow_tile<T, false>(a, b - a.bblk0);
+  else
+    bits_tile<T, PW, E, 1, false>(a, b - a.bblk0);
 }
 
 // ---------------------------------------------------------------------------
@@ -403,8 +449,10 @@ void rows_vol(const RowsGeom& r, void* bits, void* prefixes, VolArgs* a) {
   a->cwn = (65536u + (uint32_t)r.cw - 1u) / (uint32_t)r.cw;
   a->cntiles = (a->g.units + kCountTile - 1) / kCountTile;
   // (a batch's tiles are those of a small volume: its volumes fill the device)
-  a->bntiles = (int64_t)((a->g.nx + 2 * kWave - 1) / (2 * kWave)) *
-               (((int64_t)a->g.ny * a->sw + kBatchPW - 1) / kBatchPW);
+  a->bntiles = narrow_tiles(*a);
+  if (a->bntiles == 0)
+    a->bntiles = (int64_t)((a->g.nx + 2 * kWave - 1) / (2 * kWave)) *
+                 (((int64_t)a->g.ny * a->sw + kBatchPW - 1) / kBatchPW);
 }
 
 // Units a wave emits one after another: one where a unit alone has cells
@@ -445,8 +493,14 @@ static void launch_bits_e(const VolArgs& a, hipStream_t st) {
 // ms (1.51).
 template <typename T>
 static void launch_bits_t(const VolArgs& a, hipStream_t st) {
+  const bool large = (int64_t)a.g.nx * a.g.ny * a.g.nz * (int64_t)sizeof(T) > (512ll << 20);
+  if (narrow_tiles(a) > 0) {
+    hipLaunchKernelGGL((large ? k_bits_narrow<T, true> : k_bits_narrow<T, false>),
+                       dim3((unsigned)narrow_tiles(a)), dim3(kBlock), 0, st, a);
+    return;
+  }
   const int64_t nq = (int64_t)a.g.ny * a.sw, x128 = (a.g.nx + 127) / 128, x256 = (a.g.nx + 255) / 256;
-  if ((int64_t)a.g.nx * a.g.ny * a.g.nz * (int64_t)sizeof(T) > (512ll << 20))
+  if (large)
     2 * x256 == x128 ? launch_bits_e<T, 32, 1, 4, true>(a, st)
                      : launch_bits_e<T, 32, 2, 1, true>(a, st);
   else if (x128 * ((nq + 31) / 32) >= 2048)
