@@ -166,7 +166,8 @@ int msh_set_kernel_family(void* ctx, int32_t method, int32_t dtype, int32_t fami
 /* Limits of a context.  Results do not depend on them.
  * MSH_LIMIT_SAMPLE_BITS: the most bytes of workspace that a call's row
  * kernels may take for their sample bits and what goes with them (a bit per
- * sample, and for tetrahedra and surface nets 2 bytes per 32 cells);
+ * sample, 80 bytes per unit of up to 64 x 32 cells and, for tetrahedra and
+ * surface nets, 2 bytes per 32 cells);
  * negative, the default: no limit.  A call over it takes the other kernels,
  * as one does for whose bits the device has no room.
  * MSH_LIMIT_WELD_INDEX32: the most vertices that msh_weld welds with 32-bit

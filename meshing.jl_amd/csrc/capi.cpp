@@ -43,8 +43,11 @@ struct Launch {
 
 // Estimated work of a volume in a batched launch, for spreading the launches
 // over streams: its tile-cells (a partly filled tile costs about what a full
-// one does), and for an emit weighted by method (MC 1, surface nets 2,
-// tetrahedra 3: the 256^3 gyroid emits take 0.056, 0.12 and 0.17 ms);
+// one does; the row kernels' units), and for an emit weighted by method (MC 1,
+// surface nets 2, tetrahedra 3: the 256^3 Float32 gyroid emits take 0.056,
+// 0.12 and 0.17 ms with lanes along x; by rows 0.034, 0.035 and 0.088, and
+// those of 384 x 320 x 448 Float32 noise 0.27, 0.28 and 0.69, so surface nets
+// weigh too much there, which the order of three launches does not feel);
 // counting costs the same per cell for every method.
 double cell_cost(const VolArgs& v, const Plan& p, bool emit) {
   const double w = p.method == MT ? 3.0 : p.method == SN ? 2.0 : 1.0;

@@ -112,6 +112,7 @@ template <typename T, bool NT>
 __device__ __forceinline__ void narrow_tile(const VolArgs& a, int64_t t) {
   const Geom g = a.g;
   const T thr = (T)a.thr;
+  // (below 2^31: kMaxBlocks holds ny under 2^26)
   const uint32_t cols = (uint32_t)g.nx * (uint32_t)g.ny, nb = (cols + kBlock - 1) / kBlock;
   const uint32_t tw = (uint32_t)t / nb, c = ((uint32_t)t - tw * nb) * kBlock + threadIdx.x;
   if (c >= cols) return;

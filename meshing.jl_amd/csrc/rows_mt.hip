@@ -20,11 +20,12 @@
 //
 // Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 158 -> 90 us, 512^3
 // Float32 value noise 2.05 -> 1.55 ms.
-// Bound by vector issue (55% of the cycles on the noise) and the
-// latency of each step at 2.8 waves a SIMD (128 registers, 40 KB of LDS a
-// block).  A queue of 64 cells with all 19 edge numbers in LDS, which saves
-// three look-ups a face vertex, was slower (100 us, 1.70 ms): a unit is then
-// read about twice as often.
+// Bound by vector issue (54% of the SIMDs' cycles on the noise, 38% on the
+// gyroid) and the latency of each step at 2.8 and 1.6 waves a SIMD on average
+// (128 registers and 40 KB of LDS a block would let it hold 4).  A queue of 64
+// cells with all 19 edge numbers in LDS, which saves three look-ups a face
+// vertex, was slower (100 us, 1.70 ms): a unit is then read about twice as
+// often.
 #include <type_traits>
 
 #include "rows.h"

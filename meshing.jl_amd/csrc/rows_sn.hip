@@ -14,11 +14,13 @@
 // the emit, which so needs no registers for it.
 //
 // Emit, before (halo5.hip) -> now: 256^3 Float32 gyroid 114 -> 34 us,
-// 384 x 320 x 448 Float64 value noise 774 -> 430 us.  Bound by vector issue
-// (58% of the cycles there, most of it the divisions and interpolations of
-// the edges) and by the latency of each step's look-ups at 3 to 4 waves a
-// SIMD; holding the samples of a step in registers while its unit is listed
-// (122 registers) was slower, and so were caps on the registers, which spill.
+// 384 x 320 x 448 Float64 value noise 774 -> 419 us.  Bound by vector issue
+// (53% of the SIMDs' cycles there, 51% on the gyroid, most of it the divisions
+// and interpolations of the edges) and by the latency of each step's look-ups
+// at 2.7 and 2.3 waves a SIMD on average (94 registers, Float64 114, would
+// let it hold 5 or 4); holding the samples of a step in registers while its
+// unit is listed (122 registers) was slower, and so were caps on the
+// registers, which spill.
 #include <type_traits>
 
 #include "rows.h"
