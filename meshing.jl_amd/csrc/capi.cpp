@@ -765,11 +765,8 @@ int msh_count(void* ctx, const msh_field* f, const msh_params* p, int64_t* nvert
     nfc = c->pinned[3];
     if (bits) {
       rows_emit_tiling(&a, nv);
-      const uint32_t n[3] = {(uint32_t)c->pinned[0], (uint32_t)((uint64_t)c->pinned[0] >> 32), 0};
-      const int list = rows_list(pl.method, n);
-      a.taken = a.groups.list[list & 1];
-      a.shared = n[list];
-      a.xblocks = rows_xblocks(a.shared);
+      const uint32_t n[2] = {(uint32_t)c->pinned[0], (uint32_t)((uint64_t)c->pinned[0] >> 32)};
+      rows_take_groups(n, &a);
     }
     c->vol = a;
   }

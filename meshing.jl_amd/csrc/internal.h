@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 
 #include "../../include/meshing_hip.h"
@@ -146,7 +147,8 @@ struct VolArgs {
   int32_t ue;              // units a wave emits one after another
   int32_t self;            // this volume's number in a batch
   int32_t xblocks;         // blocks of groups before the tiles of a single emit ..
-  uint32_t shared;         // .. and their groups
+  uint32_t shared;         // .. their groups
+  uint32_t gcols;          // .. and the groups of an x plane whose units are all shared
   RowsParts* parts;        // per unit, of the shared ones
   RowsGroups groups;       // as the scan lists them
   const RowsGroup* taken;  // the list that a single emit takes
@@ -260,6 +262,20 @@ inline int rows_list(int method, const uint32_t* n) {
   return n[0] <= rows_group_cap(method, 0) ? 0 : n[1] <= rows_group_cap(method, 1) ? 1 : 2;
 }
 inline int32_t rows_xblocks(uint32_t n) { return (int32_t)((n + 7) / 8 * 8); }
+// A single emit's groups: gcols (at most their number) from the units of an x
+// plane and the groups of a unit, which the second list's number tells: it has
+// 4 parts of each.  1: taken as they are listed (group_of_block).
+inline void rows_take_groups(const uint32_t* n, VolArgs* a) {
+  const uint32_t none[3] = {n[0], n[1], 0};
+  const int list = rows_list(a->method, n);
+  a->taken = a->groups.list[list & 1];
+  a->shared = none[list];
+  const uint64_t units = std::max<uint64_t>(n[1] * (uint64_t)rows_emit_waves(a->method) / 4, 1);
+  const uint64_t each = std::max<uint64_t>((a->shared + units / 2) / units, 1);
+  const uint64_t cols = std::max<uint64_t>(std::min<uint64_t>(each * (uint64_t)a->upx, a->shared), 1);
+  a->gcols = cols % 8 == 0 ? 1u : (uint32_t)cols;
+  a->xblocks = rows_xblocks((a->shared + a->gcols - 1) / a->gcols * a->gcols);
+}
 hipError_t launch_rows_count(const Plan& p, const VolArgs& a, const ScanTail& tail, hipStream_t st);
 // A batched launch: tiles gbase .. gbase + nblocks of the batch, whose volumes
 // the map names.
