@@ -56,12 +56,13 @@ double cell_cost(const VolArgs& v, const Plan& p, bool emit) {
   return emit ? (double)v.ntiles * zc * w : (double)v.cntiles * zc;
 }
 
-// Launch order for spreading: most work first (each goes to the stream with
-// the least work so far, so the short launches fill in at the end).
+// Whether any of the launches takes its tiles from a work queue.
 bool work_queues(const std::vector<Launch>& ls) {
   return std::any_of(ls.begin(), ls.end(), [](const Launch& l) { return !l.rows; });
 }
 
+// Launch order for spreading: most work first (each goes to the stream with
+// the least work so far, so the short launches fill in at the end).
 std::vector<size_t> by_cost(const std::vector<Launch>& ls) {
   std::vector<size_t> o(ls.size());
   for (size_t i = 0; i < o.size(); ++i) o[i] = i;
@@ -1107,7 +1108,8 @@ int msh_batch_count(void* ctx, int32_t n, const msh_field* fields, const msh_par
     if (e == hipSuccess && n > 0)
       e = hipMemcpyAsync(dvols, c->hbatch, sizeof(VolArgs) * (size_t)n, hipMemcpyHostToDevice,
                          c->stream);
-    if (e == hipSuccess) e = launch_fill_maps(dvols, n, cmap, emap, bmap, ngroups, (int)(2 * b.emits.size()), c->stream);
+    if (e == hipSuccess)
+      e = launch_fill_maps(dvols, n, cmap, emap, bmap, ngroups, (int)(2 * b.emits.size()), c->stream);
     if (e == hipSuccess) e = launch_coords_batch(dvols, n, c->stream);
     if (e == hipSuccess && work_queues(b.counts))
       e = launch_zero_u32(ctrs, (int64_t)(8 * b.counts.size()), c->stream);

@@ -298,8 +298,8 @@ struct ShareOut {
   uint32_t vol;
 };
 __host__ __device__ inline ShareOut share_out(const VolArgs& a, int vol) {
-  return {a.groups, {rows_group_cap(a.method, 0), rows_group_cap(a.method, 1)}, (uint32_t)rows_emit_waves(a.method), rows_cuts(a.method),
-          (uint32_t)vol};
+  return {a.groups, {rows_group_cap(a.method, 0), rows_group_cap(a.method, 1)},
+          (uint32_t)rows_emit_waves(a.method), rows_cuts(a.method), (uint32_t)vol};
 }
 struct ShareSums {
   uint32_t w[kWaves], base[2];
@@ -331,7 +331,8 @@ __device__ __forceinline__ uint32_t share_list(const ShareOut& o, int64_t first,
   if (__builtin_expect(all == 0, 1)) return 0;
   uint32_t at0 = at & 0xFFFF, at1 = at >> 16;
   if (!alone) {
-    if (threadIdx.x < 2) s->base[threadIdx.x] = atomicAdd(o.to.n + threadIdx.x, threadIdx.x ? all >> 16 : all & 0xFFFF);
+    if (threadIdx.x < 2)
+      s->base[threadIdx.x] = atomicAdd(o.to.n + threadIdx.x, threadIdx.x ? all >> 16 : all & 0xFFFF);
     __syncthreads();
     at0 += s->base[0];
     at1 += s->base[1];

@@ -340,8 +340,8 @@ __device__ __forceinline__ void scan_tail(const VolArgs& a, const ScanTail& t) {
   }
   const uint64_t incl = wave_incl_scan64(sum);
   __shared__ ShareSums sums;
-  const ShareOut share{a.groups, {rows_group_cap(METHOD, 0), rows_group_cap(METHOD, 1)}, (uint32_t)rows_emit_waves(METHOD),
-                       rows_cuts(METHOD), 0};
+  const ShareOut share{a.groups, {rows_group_cap(METHOD, 0), rows_group_cap(METHOD, 1)},
+                       (uint32_t)rows_emit_waves(METHOD), rows_cuts(METHOD), 0};
   const uint32_t groups = share_count(share, c, &sums);
   if (lane_id() == kWave - 1) s_w[wave_id()] = incl;
   __syncthreads();
